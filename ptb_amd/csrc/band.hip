@@ -1,0 +1,1055 @@
+// FP64 tridiagonalisation in two stages, K = Q1 B Q1^T (dense to a band of kBW
+// subdiagonals) and B = Q2 T Q2^T (bulge chasing), batched over submatrices.
+//
+// The one-stage reduction (tridiag.hip) reads the trailing matrix once per
+// column: sum 4 m^3 / 3 bytes, which HBM bounds.  Here the trailing matrix is
+// read and rewritten once per kBW columns by matrix-core products, and the band
+// (17 m doubles) is reduced inside one CU.
+//
+// Stage 1, per panel of kBW columns k0 .. k0 + 15 (rows from r0 = k0 + 16 on):
+//   k_band_qr    Householder QR of the panel below the band in registers;
+//                V into the matrix and the panel buffers, R into the band,
+//                the WY factor T;
+//   k_band_symm  X = A22 V from the lower triangle;
+//   k_band_w     W = X T - V (T^T (V^T X) T) / 2;
+//   then A22 -= [W V] [V W]^T (lower triangle) by the batched GEMM.
+// The reflector of column c has its unit at row c + kBW.
+//
+// Stage 2 (k_chase): sweep s removes column s outside the tridiagonal with a
+// reflector over rows s+1 .. s+16 and chases the bulge down in windows of 16
+// rows, window k of sweep s being rows s + 1 + 16 k + (0 .. 15).  Reflector
+// (s, k) acts on that window.
+//
+// Application of Q2: the reflectors of 16 consecutive sweeps at one window k
+// form a block I - V T V^T of 31 rows.  Q2 is the product over the sweep
+// groups G ascending, and inside a group over k descending (blocks of a group
+// overlap only their neighbours, and this order keeps every overlapping pair).
+#include <algorithm>
+#include <type_traits>
+
+#include "sm_internal.hpp"
+
+namespace {
+
+typedef double d4_t __attribute__((ext_vector_type(4)));
+typedef double d2_t __attribute__((ext_vector_type(2)));
+
+constexpr int kBW = kBandWidth;  // 16
+constexpr int kABL = kBW + 1;    // doubles per column of the band buffer
+
+// One submatrix of the band route (largest first).
+struct BandSub {
+    int64_t off;   // matrix block in the arena
+    int64_t pw;    // panel buffers: [W V W] (ld x 48), V and X by rows (ld x 16 each), T (256)
+    int64_t ab;    // band: column c at ab + 17 c, element d below the diagonal at + d
+    int64_t blk;   // first block of its Q2 reflectors
+    int m, ld, mapoff, ng;  // ng sweep groups
+};
+
+// blocks of Q2 per submatrix: group G has ng - G of them (windows that hold at
+// least two rows), group after group
+__host__ __device__ inline int q2_groups(int m) { return m >= 3 ? (m - 3) / kBW + 1 : 0; }
+__device__ inline int64_t q2_block(int ng, int G, int k) {
+    return (int64_t)G * ng - (int64_t)G * (G - 1) / 2 + k;
+}
+
+// ---- cross-lane sums --------------------------------------------------------
+template <int CTRL>
+__device__ __forceinline__ double dpp_add(double v) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
+    return v + __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+// sum over the 16 lanes of a row, in every lane: quad_perm 1032, 2301, then
+// the mirrors within 8 and within 16
+__device__ __forceinline__ double row_sum(double v) {
+    v = dpp_add<0xB1>(v);
+    v = dpp_add<0x4E>(v);
+    v = dpp_add<0x141>(v);
+    return dpp_add<0x140>(v);
+}
+// sum over the four 16-lane rows, in every lane
+__device__ __forceinline__ double rows_sum(double v) {
+    {
+        const long long b = __double_as_longlong(v);
+        const auto l = __builtin_amdgcn_permlane16_swap((unsigned)b, (unsigned)b, false, false);
+        const auto h = __builtin_amdgcn_permlane16_swap((unsigned)(b >> 32), (unsigned)(b >> 32), false, false);
+        v = __longlong_as_double(((long long)h[0] << 32) | l[0]) +
+            __longlong_as_double(((long long)h[1] << 32) | l[1]);
+    }
+    const long long b = __double_as_longlong(v);
+    const auto l = __builtin_amdgcn_permlane32_swap((unsigned)b, (unsigned)b, false, false);
+    const auto h = __builtin_amdgcn_permlane32_swap((unsigned)(b >> 32), (unsigned)(b >> 32), false, false);
+    return __longlong_as_double(((long long)h[0] << 32) | l[0]) +
+           __longlong_as_double(((long long)h[1] << 32) | l[1]);
+}
+__device__ __forceinline__ double read_lane(double v, int lane) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_readlane((int)b, lane);
+    const int hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+// Sum over the wavefront of 16 values per lane; value q ends in the lanes with
+// (lane >> 2) & 15 == q.
+__device__ __forceinline__ double sum16(const double (&p)[16], int lane) {
+    double h8[8], h4[4], h2[2];
+    const bool b5 = lane & 32, b4 = lane & 16, b3 = lane & 8, b2 = lane & 4;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) h8[j] = (b5 ? p[j + 8] : p[j]) + __shfl_xor(b5 ? p[j] : p[j + 8], 32);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) h4[j] = (b4 ? h8[j + 4] : h8[j]) + __shfl_xor(b4 ? h8[j] : h8[j + 4], 16);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) h2[j] = (b3 ? h4[j + 2] : h4[j]) + __shfl_xor(b3 ? h4[j] : h4[j + 2], 8);
+    const double v = (b2 ? h2[1] : h2[0]) + __shfl_xor(b2 ? h2[0] : h2[1], 4);
+    return dpp_add<0x4E>(dpp_add<0xB1>(v));
+}
+
+// The reflector of x (alpha at the pivot, sigma the squares of the rest):
+// H = I - tau u u^T, u = 1 at the pivot and x * scale elsewhere, H x = beta.
+struct Reflector {
+    double beta, tau, scale;
+};
+__device__ __forceinline__ Reflector reflector(double alpha, double sigma) {
+    if (sigma == 0.0) return {alpha, 0.0, 0.0};
+    const double beta = -copysign(sqrt(alpha * alpha + sigma), alpha);
+    return {beta, (beta - alpha) / beta, 1.0 / (alpha - beta)};
+}
+
+// ---- stage 1 ------------------------------------------------------------------
+
+// QR of one 16-column panel, rows r0 .. m - 1 in registers (thread t holds rows
+// t + NT q): per column one pass of 16 dot products x^T A(:, l) over the rows
+// below the pivot (l = j: sigma; l > j: the update; l < j: V^T v for T), one
+// barrier, one update.  A workgroup's time is the serial chain of its 16 columns
+// (about 1 us each), so the panel stays in registers and the workgroups of
+// other submatrices fill the CU.  The row-to-thread map and the order of every sum
+// depend on the panel's own height only.
+template <int NT, int R>
+__global__ __launch_bounds__(NT, R == 4 ? 2 : 4) void k_band_qr(const BandSub *__restrict__ subs,
+                                                 double *__restrict__ Aa, double *__restrict__ PW,
+                                                 double *__restrict__ ABa,
+                                                 double *__restrict__ tau_all, int first, int panel) {
+    constexpr int NW = NT / PTB_WAVE;
+    const BandSub d = subs[first + blockIdx.x];
+    const int k0 = panel * kBW, r0 = k0 + kBW;
+    const int n = d.m - r0;
+    if (n < 2) return;
+    const int nref = min(kBW, n - 1);
+    __shared__ double red[2][NW][kBW], prow[2][kBW], zt[kBW][kBW], ts[kBW];
+    const int lane = threadIdx.x % PTB_WAVE, wave = threadIdx.x / PTB_WAVE;
+    double *a = Aa + d.off + (int64_t)k0 * d.ld + r0;
+    double x[R][kBW];
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+        const int i = threadIdx.x + NT * q;
+        const unsigned ic = (unsigned)min(i, n - 1);
+#pragma unroll
+        for (int l = 0; l < kBW; ++l) x[q][l] = a[(unsigned)(l * d.ld) + ic];
+    }
+#pragma unroll
+    for (int q = 0; q < R; ++q)
+#pragma unroll
+        for (int l = 0; l < kBW; ++l) x[q][l] = (int)threadIdx.x + NT * q < n ? x[q][l] : 0.0;
+    auto column = [&](auto J) {
+        constexpr int j = decltype(J)::value;
+        if (j >= nref) return;
+        const int bf = j & 1;
+        double p[kBW];
+#pragma unroll
+        for (int l = 0; l < kBW; ++l) p[l] = 0.0;
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+            const double xi = (int)threadIdx.x + NT * q > j ? x[q][j] : 0.0;
+#pragma unroll
+            for (int l = 0; l < kBW; ++l) p[l] += xi * x[q][l];
+        }
+        const double s = sum16(p, lane);
+        if ((lane & 3) == 0) red[bf][wave][lane >> 2] = s;
+        if ((int)threadIdx.x == j)
+#pragma unroll
+            for (int l = 0; l < kBW; ++l) prow[bf][l] = x[0][l];
+        __syncthreads();
+        // every wavefront forms the scalars, lane l (mod 16) those of column l
+        const int l = lane & 15;
+        double dot = 0.0;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) dot += red[bf][w][l];
+        const double pl = prow[bf][l];
+        const Reflector h = reflector(read_lane(pl, j), read_lane(dot, j));
+        const double zl = pl + h.scale * dot;  // A(:, l)^T v
+        const double wl = l > j ? h.tau * zl : 0.0;
+        if (threadIdx.x < kBW) zt[j][l] = zl;
+        if (threadIdx.x == 0) ts[j] = h.tau;
+        double ws_[kBW];
+#pragma unroll
+        for (int c = j + 1; c < kBW; ++c) ws_[c] = read_lane(wl, c);
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+            const int i = threadIdx.x + NT * q;
+            const double vi = i > j ? x[q][j] * h.scale : i == j ? 1.0 : 0.0;
+#pragma unroll
+            for (int c = j + 1; c < kBW; ++c) x[q][c] -= ws_[c] * vi;
+            x[q][j] = i > j ? vi : i == j ? h.beta : x[q][j];
+        }
+    };
+    column(std::integral_constant<int, 0>{}), column(std::integral_constant<int, 1>{});
+    column(std::integral_constant<int, 2>{}), column(std::integral_constant<int, 3>{});
+    column(std::integral_constant<int, 4>{}), column(std::integral_constant<int, 5>{});
+    column(std::integral_constant<int, 6>{}), column(std::integral_constant<int, 7>{});
+    column(std::integral_constant<int, 8>{}), column(std::integral_constant<int, 9>{});
+    column(std::integral_constant<int, 10>{}), column(std::integral_constant<int, 11>{});
+    column(std::integral_constant<int, 12>{}), column(std::integral_constant<int, 13>{});
+    column(std::integral_constant<int, 14>{}), column(std::integral_constant<int, 15>{});
+    __syncthreads();
+    double *pw = PW + d.pw;
+    double *vr = pw + (int64_t)48 * d.ld;
+    double *T = vr + (int64_t)32 * d.ld;
+    // R into the band, T (wavefront 0; lane i holds row i)
+    if (threadIdx.x < kBW) {
+        const int i = threadIdx.x;
+        double *ab = ABa + d.ab;
+        if (i < n)
+#pragma unroll
+            for (int l = 0; l < kBW; ++l)
+                if (l >= i) ab[(int64_t)(k0 + l) * kABL + kBW + i - l] = x[0][l];
+        double t[kBW];
+#pragma unroll
+        for (int j = 0; j < kBW; ++j) {
+            double s = 0.0;
+            if (j < nref) {
+#pragma unroll
+                for (int c = 0; c < j; ++c) s += t[c] * zt[j][c];
+                const double tj = ts[j];
+                t[j] = i == j ? tj : i < j ? -tj * s : 0.0;
+                if (i == j) tau_all[d.mapoff + k0 + j] = tj;
+            } else {
+                t[j] = 0.0;
+            }
+            T[j * kBW + i] = t[j];
+        }
+    }
+    // V: unit lower trapezoidal, zero columns past the last reflector
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+        const int i = threadIdx.x + NT * q;
+#pragma unroll
+        for (int l = 0; l < kBW; ++l) {
+            const double v = l >= nref ? 0.0 : i > l ? x[q][l] : i == l ? 1.0 : 0.0;
+            x[q][l] = v;
+            if (i < n) {
+                if (l < nref) a[(unsigned)(l * d.ld) + (unsigned)i] = v;
+                pw[(unsigned)((kBW + l) * d.ld) + (unsigned)(r0 + i)] = v;
+            }
+        }
+        // by rows, zero up to the next multiple of 16 rows
+        if (i < ((n + 15) & ~15)) {
+            d2_t *row = reinterpret_cast<d2_t *>(vr + (int64_t)(r0 + i) * kBW);
+#pragma unroll
+            for (int l = 0; l < kBW / 2; ++l) {
+                const bool in = i < n;
+                row[l] = d2_t{in ? x[q][2 * l] : 0.0, in ? x[q][2 * l + 1] : 0.0};
+            }
+        }
+    }
+}
+
+// X = A22 V (rows r0 .., V by rows): one wavefront per 16 rows, straight from
+// memory to v_mfma_f64_16x16x4 operands (no LDS, no barrier): the rows' part
+// left of the diagonal tile, the diagonal tile, and the part below it
+// transposed.  Every element of the lower triangle is read twice, once as row
+// and once as column; bound by that traffic.  A workgroup's four wavefronts
+// take 64 consecutive rows; a submatrix's workgroups run on one XCD.
+__global__ __launch_bounds__(256) void k_band_symm(const BandSub *__restrict__ subs, int nsub,
+                                                   const double *__restrict__ Aa,
+                                                   double *__restrict__ PW, int panel, int nblk) {
+    const unsigned lin = blockIdx.x, slot = lin >> 3;
+    const int si = (int)((slot / (unsigned)nblk) * 8 + (lin & 7));
+    if (si >= nsub) return;
+    const BandSub d = subs[si];
+    const int r0 = panel * kBW + kBW;
+    const int n = d.m - r0;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PTB_WAVE);
+    const int R0 = (int)(slot % (unsigned)nblk) * 64 + wave * 16;
+    if (n < 2 || R0 >= n) return;
+    const int lane = threadIdx.x % PTB_WAVE, lr = lane & 15, g = lane >> 4;
+    const unsigned ld = (unsigned)d.ld;
+    const double *a = Aa + d.off + (int64_t)r0 * d.ld + r0;
+    double *vr = PW + d.pw + (int64_t)48 * d.ld;
+    double *xr = vr + (int64_t)16 * d.ld;
+    const double *v = vr + (int64_t)r0 * kBW;
+    d4_t acc = d4_t{0.0, 0.0, 0.0, 0.0}, acc2 = acc;
+    // rows: A(R0 + i, k), k < R0 (slices of 4 columns); rows past the end
+    // clamped (their results are not used)
+    {
+        const double *ar = a + (unsigned)min(R0 + lr, n - 1) + (unsigned)g * ld;
+        const double *vk = v + (unsigned)g * kBW + lr;
+        for (int k = 0; k < R0; k += 16) {
+            double av[4], bv[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                av[u] = ar[(unsigned)(4 * u) * ld];
+                bv[u] = vk[4 * u * kBW];
+            }
+            ar += 16u * ld;
+            vk += 16 * kBW;
+            acc = __builtin_amdgcn_mfma_f64_16x16x4f64(av[0], bv[0], acc, 0, 0, 0);
+            acc2 = __builtin_amdgcn_mfma_f64_16x16x4f64(av[1], bv[1], acc2, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f64_16x16x4f64(av[2], bv[2], acc, 0, 0, 0);
+            acc2 = __builtin_amdgcn_mfma_f64_16x16x4f64(av[3], bv[3], acc2, 0, 0, 0);
+        }
+    }
+    // the diagonal tile, from its lower triangle
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const int i = R0 + lr, k = R0 + 4 * u + g;
+        const int hi = min(max(i, k), n - 1), lo = min(min(i, k), n - 1);
+        const double x = a[(unsigned)lo * ld + (unsigned)hi];
+        const double av = (i < n && k < n) ? x : 0.0;
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(av, v[(unsigned)k * kBW + lr], acc, 0, 0, 0);
+    }
+    // columns: A(k, R0 + i), k >= R0 + 16, 16 rows at a time, lane group g
+    // holding rows 4 g .. 4 g + 3 (slice u: k = 4 g + u in both operands)
+    if (R0 + 16 < n) {
+        const double *ac = a + (unsigned)(R0 + lr) * ld;
+        for (int k = R0 + 16; k < n; k += 16) {
+            const d2_t *p = reinterpret_cast<const d2_t *>(ac + k + 4 * g);
+            const d2_t p0 = p[0], p1 = p[1];
+            const double *vk = v + (unsigned)(k + 4 * g) * kBW + lr;
+            double av[4] = {p0[0], p0[1], p1[0], p1[1]}, bv[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) bv[u] = vk[u * kBW];
+            if (k + 16 > n)
+#pragma unroll
+                for (int u = 0; u < 4; ++u) av[u] = k + 4 * g + u < n ? av[u] : 0.0;
+            acc = __builtin_amdgcn_mfma_f64_16x16x4f64(av[0], bv[0], acc, 0, 0, 0);
+            acc2 = __builtin_amdgcn_mfma_f64_16x16x4f64(av[1], bv[1], acc2, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f64_16x16x4f64(av[2], bv[2], acc, 0, 0, 0);
+            acc2 = __builtin_amdgcn_mfma_f64_16x16x4f64(av[3], bv[3], acc2, 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+        xr[(unsigned)(r0 + R0 + 4 * r + g) * kBW + lr] = acc[r] + acc2[r];
+}
+
+// W = X T - V S, S = T^T (V^T X) T / 2, by columns into the panel buffer
+// (columns 0 .. 15 and 32 .. 47).  One workgroup per submatrix: V^T X on the
+// matrix cores (wavefronts on alternate 16-row tiles), the 16 x 16 products in
+// LDS, then W^T tile by tile.
+__global__ __launch_bounds__(256) void k_band_w(const BandSub *__restrict__ subs,
+                                                double *__restrict__ PW, int panel) {
+    const BandSub d = subs[blockIdx.x];
+    const int r0 = panel * kBW + kBW;
+    const int n = d.m - r0;
+    if (n < 2) return;
+    double *pw = PW + d.pw;
+    const double *vr = pw + (int64_t)48 * d.ld + (int64_t)r0 * kBW;
+    const double *xr = vr + (int64_t)16 * d.ld;
+    const double *T = pw + (int64_t)80 * d.ld;
+    __shared__ double gs[4][16][17], ts[16][17], ms[16][17], ss[16][17];
+    const int lane = threadIdx.x % PTB_WAVE, wave = threadIdx.x / PTB_WAVE;
+    const int lr = lane & 15, g = lane >> 4;
+    d4_t acc = d4_t{0.0, 0.0, 0.0, 0.0};
+    for (int k = 16 * wave; k < n; k += 64) {
+        double av[4], bv[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            av[u] = vr[(unsigned)(k + 4 * u + g) * kBW + lr];
+            bv[u] = xr[(unsigned)(k + 4 * u + g) * kBW + lr];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(av[u], bv[u], acc, 0, 0, 0);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) gs[wave][4 * r + g][lr] = acc[r];
+    const int ti = threadIdx.x & 15, tj = threadIdx.x >> 4;
+    ts[ti][tj] = T[tj * kBW + ti];
+    __syncthreads();
+    {
+        const double s = ((gs[0][ti][tj] + gs[1][ti][tj]) + gs[2][ti][tj]) + gs[3][ti][tj];
+        ss[ti][tj] = s;
+    }
+    __syncthreads();
+    {
+        double s = 0.0;  // M = G T
+#pragma unroll
+        for (int c = 0; c < 16; ++c) s += ss[ti][c] * ts[c][tj];
+        ms[ti][tj] = s;
+    }
+    __syncthreads();
+    {
+        double s = 0.0;  // S = T^T M / 2
+#pragma unroll
+        for (int c = 0; c < 16; ++c) s += ts[c][ti] * ms[c][tj];
+        ss[ti][tj] = 0.5 * s;
+    }
+    __syncthreads();
+    // W^T(col, row) = sum_c T(c, col) X(row, c) - S(c, col) V(row, c)
+    double ta[4], sa[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        ta[u] = ts[4 * u + g][lr];
+        sa[u] = -ss[4 * u + g][lr];
+    }
+    for (int k = 16 * wave; k < n; k += 64) {
+        double xb[4], vb[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            xb[u] = xr[(unsigned)(k + lr) * kBW + 4 * u + g];
+            vb[u] = vr[(unsigned)(k + lr) * kBW + 4 * u + g];
+        }
+        d4_t w = d4_t{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            w = __builtin_amdgcn_mfma_f64_16x16x4f64(ta[u], xb[u], w, 0, 0, 0);
+            w = __builtin_amdgcn_mfma_f64_16x16x4f64(sa[u], vb[u], w, 0, 0, 0);
+        }
+        if (k + lr < n)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                double *o = pw + (unsigned)((4 * r + g) * d.ld) + (unsigned)(r0 + k + lr);
+                o[0] = w[r];
+                o[(unsigned)(32 * d.ld)] = w[r];
+            }
+    }
+}
+
+// The band's diagonal blocks (lower) and the rows below them that no panel
+// reduced; then zeros in the reflector columns above the panel's own rows, as far
+// as the block readers see (from 16 rows below the column's block of `qblk`
+// reflectors).  grid: (submatrix, 16-column block)
+__global__ __launch_bounds__(256) void k_band_extract(const BandSub *__restrict__ subs,
+                                                      double *__restrict__ Aa,
+                                                      double *__restrict__ ABa, int qblk) {
+    const BandSub d = subs[blockIdx.x];
+    const int k0 = blockIdx.y * kBW;
+    if (k0 >= d.m) return;
+    const bool qr = d.m - (k0 + kBW) >= 2;  // the panel was factored: R is in the band
+    double *a = Aa + d.off;
+    double *ab = ABa + d.ab;
+    for (int l = threadIdx.x; l < kBW * kABL; l += 256) {
+        const int c = k0 + l / kABL, dd = l % kABL, r = c + dd;
+        if (c >= d.m) continue;
+        if (r < k0 + kBW || !qr) ab[(int64_t)c * kABL + dd] = r < d.m ? a[(int64_t)c * d.ld + r] : 0.0;
+    }
+    __syncthreads();
+    if (!qr) return;
+    const int b0 = k0 & ~(qblk - 1);
+    const int rows = k0 - b0;  // rows b0 + 16 .. k0 + 15
+    for (int l = threadIdx.x; l < kBW * rows; l += 256) {
+        const int c = k0 + l / rows, r = b0 + kBW + l % rows;
+        if (c < d.m - kBW - 1) a[(int64_t)c * d.ld + r] = 0.0;
+    }
+}
+
+// ---- stage 2 ------------------------------------------------------------------
+
+// Message area of a chase, per window k: the reflector that acts on it (vm, by
+// slot; tm), its diagonal block's first column and the element below it (cm,
+// bm), and its off-diagonal block's first row (rm).
+struct ChaseLds {
+    double *vm, *tm, *cm, *bm, *rm, *wsc;
+};
+
+// One step of the chase: window k of sweep s.  A wavefront holds the window's
+// diagonal block D and the block B below it (rows of window k + 1), 16 x 16, in
+// cyclic slots: row or column r sits in slot r mod 16, so moving from sweep s - 1
+// to sweep s replaces one slot and shifts nothing.  Lane l holds row slot l % 16
+// and column slots 4 (l / 16) + c.  f = (s + 1) mod 16 is the slot of every
+// window's first row.
+__device__ __forceinline__ void chase_step(double (&D)[4], double (&B)[4], int k, int s, int m, int ng,
+                                           const ChaseLds &L, double *__restrict__ raw,
+                                           double *__restrict__ rtau, double *__restrict__ dv,
+                                           double *__restrict__ ev, int lane) {
+    const int i = lane & 15, g = lane >> 4;
+    const int fo = s & 15, f = (s + 1) & 15;
+    if (s > 0) {
+        // the slot of the row that left takes the row that enters: D's from B's
+        // first row, B's column from the next window's first column
+        const double cmv = L.cm[(k + 1) * 16 + i], bmv = L.bm[k + 1], rmv = L.rm[k * 16 + i];
+        const bool rf = i == fo;
+        const double dcol = rf ? cmv : rmv, bcol = rf ? bmv : cmv;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const bool cc = 4 * g + c == fo;
+            D[c] = cc ? dcol : rf ? B[c] : D[c];
+            B[c] = cc ? bcol : rf ? 0.0 : B[c];
+        }
+    }
+    if (k == 0) {
+        // the sweep's first reflector: column s below its diagonal
+        const double dia = L.cm[fo];
+        const double x = i == fo ? L.bm[0] : L.cm[i];
+        const Reflector h = reflector(read_lane(x, f), row_sum(i == f ? 0.0 : x * x));
+        const double u = i == f ? 1.0 : x * h.scale;
+        if (g == 0) {
+            L.vm[i] = u;
+            if (s < m - 2) raw[q2_block(ng, s >> 4, 0) * 256 + (s & 15) * 16 + ((i - f) & 15)] = u;
+        }
+        if (lane == 0) {
+            L.tm[0] = h.tau;
+            dv[s] = dia;
+            ev[s] = s < m - 1 ? h.beta : 0.0;
+            if (s < m - 2) rtau[q2_block(ng, s >> 4, 0) * 16 + (s & 15)] = h.tau;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
+    const double vr = L.vm[k * 16 + i], tau = L.tm[k];
+    double vc[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) vc[c] = L.vm[k * 16 + 4 * g + c];
+    double p = D[0] * vc[0], y = B[0] * vc[0];
+#pragma unroll
+    for (int c = 1; c < 4; ++c) {
+        p += D[c] * vc[c];
+        y += B[c] * vc[c];
+    }
+    p = tau * rows_sum(p);
+    y = tau * rows_sum(y);
+    const double w = p - (0.5 * tau * row_sum(p * vr)) * vr;
+    if (g == 0) L.wsc[i] = w;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    // B <- B H, then the reflector of its first column
+#pragma unroll
+    for (int c = 0; c < 4; ++c) B[c] -= y * vc[c];
+    const int gf = f >> 2, cf = f & 3;
+    const double b0 = cf & 1 ? B[1] : B[0], b1 = cf & 1 ? B[3] : B[2];
+    const double x = rows_sum(g == gf ? (cf & 2 ? b1 : b0) : 0.0);
+    const Reflector h = reflector(read_lane(x, f), row_sum(i == f ? 0.0 : x * x));
+    const double u = i == f ? 1.0 : x * h.scale;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        const double z = h.tau * row_sum(u * B[c]);
+        const double t = B[c] - u * z;
+        B[c] = 4 * g + c == f ? (i == f ? h.beta : 0.0) : t;
+    }
+    // D <- H D H
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        const double wc = L.wsc[4 * g + c];
+        D[c] -= vr * wc;
+        D[c] -= w * vc[c];
+    }
+    if (g == 0) {
+        L.vm[(k + 1) * 16 + i] = u;
+        if (s < m - 2 && s + 1 + 16 * (k + 1) <= m - 2)
+            raw[q2_block(ng, s >> 4, k + 1) * 256 + (s & 15) * 16 + ((i - f) & 15)] = u;
+    }
+    if (lane == 0) {
+        L.tm[k + 1] = h.tau;
+        L.bm[k] = h.beta;
+        if (s < m - 2 && s + 1 + 16 * (k + 1) <= m - 2)
+            rtau[q2_block(ng, s >> 4, k + 1) * 16 + (s & 15)] = h.tau;
+    }
+    if (g == gf) {
+        const double d0 = cf & 1 ? D[1] : D[0], d1 = cf & 1 ? D[3] : D[2];
+        L.cm[k * 16 + i] = cf & 2 ? d1 : d0;
+    }
+    if (i == f)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) L.rm[k * 16 + 4 * g + c] = B[c];
+}
+
+// Bulge chasing of one submatrix per workgroup of NW wavefronts.  Step (s, k)
+// needs (s, k - 1) and (s - 1, k + 1), so at time t = 2 s + k all windows of one
+// parity step at once; a barrier ends each time step.  Wavefront w owns the
+// windows 2 w and 2 w + 1 (mod 2 NW), so the work stays even as the band
+// shortens.  MEM false: the windows live in registers (P per wavefront, 16 VGPRs
+// each), up to 16 NW P rows; MEM true: in device memory (state), for larger m.
+template <int NW, int P, bool MEM>
+__global__ __launch_bounds__(NW * 64) void k_chase(const BandSub *__restrict__ subs, int first,
+                                                   const double *__restrict__ ABa,
+                                                   double *__restrict__ raw_all,
+                                                   double *__restrict__ rtau_all,
+                                                   double *__restrict__ d_all,
+                                                   double *__restrict__ e_all,
+                                                   double *__restrict__ state) {
+    extern __shared__ double sm[];
+    const BandSub b = subs[first + blockIdx.x];
+    const int m = b.m;
+    const int K = max((m - 1 + kBW - 1) / kBW, 1);  // windows
+    const int lane = threadIdx.x % PTB_WAVE;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PTB_WAVE);
+    ChaseLds L;
+    L.vm = sm;
+    L.cm = L.vm + 16 * (K + 2);
+    L.rm = L.cm + 16 * (K + 2);
+    L.wsc = L.rm + 16 * (K + 2) + 16 * wave;
+    L.tm = L.rm + 16 * (K + 2) + 16 * NW;
+    L.bm = L.tm + (K + 2);
+    const double *ab = ABa + b.ab;
+    for (int l = threadIdx.x; l < 16 * (K + 2); l += NW * 64) {
+        L.vm[l] = 0.0;
+        L.rm[l] = 0.0;
+        L.cm[l] = l < 16 && l < m ? ab[l] : 0.0;
+    }
+    for (int l = threadIdx.x; l < K + 2; l += NW * 64) {
+        L.tm[l] = 0.0;
+        L.bm[l] = l == 0 && m > kBW ? ab[kBW] : 0.0;
+    }
+    double *raw = raw_all + b.blk * 256, *rtau = rtau_all + b.blk * 16;
+    double *dv = d_all + b.mapoff, *ev = e_all + b.mapoff;
+    double *st = MEM ? state + b.pw : nullptr;  // (the panel buffers are free by now)
+    const int i = lane & 15, g = lane >> 4;
+    auto load_window = [&](int k, double (&D)[4], double (&B)[4]) {
+        const int r = 1 + 16 * k + ((i - 1) & 15);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const int cl = 1 + 16 * k + ((4 * g + c - 1) & 15);
+            const int lo = min(r, cl), hi = max(r, cl);
+            D[c] = hi < m ? ab[(int64_t)lo * kABL + hi - lo] : 0.0;
+            B[c] = r + 16 < m && r <= cl ? ab[(int64_t)cl * kABL + r + 16 - cl] : 0.0;
+        }
+    };
+    auto active = [&](int k, int s) { return s >= 0 && s < m && (k == 0 || s + 1 + 16 * k < m); };
+    const int T2 = m - 1;  // every step (s, k) has s + k / 2 <= m - 1
+    if constexpr (!MEM) {
+        double D[P][4], B[P][4];
+#pragma unroll
+        for (int q = 0; q < P; ++q) {
+            const int k = 2 * wave + 2 * NW * (q / 2) + (q & 1);
+            load_window(k, D[q], B[q]);
+        }
+        __syncthreads();
+        for (int t = 0; t <= T2; ++t) {
+#pragma unroll
+            for (int par = 0; par < 2; ++par) {
+#pragma unroll
+                for (int q = par; q < P; q += 2) {
+                    const int k = 2 * wave + 2 * NW * (q / 2) + par, s = t - wave - NW * (q / 2);
+                    if (active(k, s)) chase_step(D[q], B[q], k, s, m, b.ng, L, raw, rtau, dv, ev, lane);
+                }
+                __syncthreads();
+            }
+        }
+    } else {
+        for (int k = wave; k < K; k += NW) {
+            double D[4], B[4];
+            load_window(k, D, B);
+            d4_t *p = reinterpret_cast<d4_t *>(st) + ((int64_t)k * 64 + lane) * 2;
+            p[0] = d4_t{D[0], D[1], D[2], D[3]};
+            p[1] = d4_t{B[0], B[1], B[2], B[3]};
+        }
+        __syncthreads();
+        for (int t = 0; t <= T2; ++t)
+            for (int par = 0; par < 2; ++par) {
+                for (int j = 0; 2 * wave + par + 2 * NW * j < K; ++j) {
+                    const int k = 2 * wave + par + 2 * NW * j, s = t - wave - NW * j;
+                    if (!active(k, s)) continue;
+                    d4_t *p = reinterpret_cast<d4_t *>(st) + ((int64_t)k * 64 + lane) * 2;
+                    const d4_t p0 = p[0], p1 = p[1];
+                    double D[4] = {p0[0], p0[1], p0[2], p0[3]}, B[4] = {p1[0], p1[1], p1[2], p1[3]};
+                    chase_step(D, B, k, s, m, b.ng, L, raw, rtau, dv, ev, lane);
+                    p[0] = d4_t{D[0], D[1], D[2], D[3]};
+                    p[1] = d4_t{B[0], B[1], B[2], B[3]};
+                }
+                __syncthreads();
+            }
+    }
+}
+
+// ---- application of Q2 ---------------------------------------------------------
+
+// Factor of every block of 16 reflectors: with V the block's 31 x 16
+// parallelogram (reflector j at rows j .. j + 15) and T its WY factor,
+// -(V T) is stored as vt[refl * 32 + row].  Reflectors that the chase never
+// made (past the last sweep or window) are cleared.  One wavefront per block,
+// kPrepBlk blocks each.  grid: (submatrix, ceil(blocks / (4 kPrepBlk)))
+constexpr int kPrepBlk = 4;
+__global__ __launch_bounds__(256, 4) void k_q2_prep(const BandSub *__restrict__ subs,
+                                                 double *__restrict__ raw_all,
+                                                 const double *__restrict__ rtau_all,
+                                                 double *__restrict__ vt_all) {
+    const BandSub d = subs[blockIdx.x];
+    const int lane = threadIdx.x % PTB_WAVE, wave = threadIdx.x / PTB_WAVE;
+    const int lr = lane & 15, g = lane >> 4;
+    __shared__ double gsh[4][16][18], vsh[4][16][17], ths[4][16][17];
+    double (*gs)[18] = gsh[wave], (*vs)[17] = vsh[wave];
+    const int nblk = d.ng * (d.ng + 1) / 2;
+    for (int u = 0; u < kPrepBlk; ++u) {
+        const int bi = (blockIdx.y * 4 + wave) * kPrepBlk + u;
+        if (bi >= nblk) return;
+        // group G of block bi: the last with base(G) <= bi
+        int G = 0;
+        {
+            const double t = 2.0 * d.ng + 1.0;
+            G = (int)((t - sqrt(fmax(t * t - 8.0 * bi, 0.0))) * 0.5);
+            while (G > 0 && q2_block(d.ng, G, 0) > bi) --G;
+            while (G + 1 < d.ng && q2_block(d.ng, G + 1, 0) <= bi) ++G;
+        }
+        const int k = bi - (int)q2_block(d.ng, G, 0);
+        const int64_t blk = d.blk + bi;
+        double *raw = raw_all + blk * 256;
+        double *vt = vt_all + blk * 512;
+        // reflector 16 G + j exists for j < nv
+        const int nv = min(16, min(d.m - 2 - 16 * G, d.m - 2 - 16 * (G + k)));
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int j = 4 * q + g;
+            double v = raw[j * 16 + lr];
+            if (j >= nv) {
+                v = 0.0;
+                raw[j * 16 + lr] = 0.0;
+            }
+            vs[j][lr] = v;
+        }
+        double tj = lr < nv ? rtau_all[blk * 16 + lr] : 0.0;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        // Gram matrix: V(row, refl) = vs[refl][row - refl]
+        d4_t acc = d4_t{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int ks = 0; ks < 8; ++ks) {
+            const int rel = 4 * ks + g - lr;
+            const double x = vs[lr][rel & 15];
+            const double v = (rel >= 0 && rel < 16) ? x : 0.0;
+            acc = __builtin_amdgcn_mfma_f64_16x16x4f64(v, v, acc, 0, 0, 0);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) gs[4 * r + g][lr] = acc[r];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        // T(i, j) = -tau_j sum_{i <= c < j} T(i, c) G(c, j), T(j, j) = tau_j:
+        // lane i + 16 g holds row i, columns 4 g .. 4 g + 3 (G is symmetric:
+        // row j of it supplies column j)
+        double t[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 1
+        for (int jg = 0; jg < 4; ++jg)
+#pragma unroll
+            for (int jq = 0; jq < 4; ++jq) {
+                const int j = 4 * jg + jq;
+                const double tauj = read_lane(tj, j);
+                double s = 0.0;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) s += t[q] * gs[j][4 * g + q];  // t is zero past column j
+                s = rows_sum(s);
+                const double v = lr == j ? tauj : lr < j ? -tauj * s : 0.0;
+                t[jq] = g == jg ? v : t[jq];
+            }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) ths[wave][lr][4 * g + q] = t[q];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        // (V T)^T(refl, row) = sum_c T(c, refl) V(row, c)
+        d4_t o0 = d4_t{0.0, 0.0, 0.0, 0.0}, o1 = o0;
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) {
+            const int c = 4 * ks + g;
+            const double tc = -ths[wave][c][lr];
+            const int e0 = lr - c, e1 = 16 + lr - c;
+            const double x0 = vs[c][e0 & 15], x1 = vs[c][e1 & 15];
+            o0 = __builtin_amdgcn_mfma_f64_16x16x4f64(tc, e0 >= 0 ? x0 : 0.0, o0, 0, 0, 0);
+            o1 = __builtin_amdgcn_mfma_f64_16x16x4f64(tc, e1 < 16 ? x1 : 0.0, o1, 0, 0, 0);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            vt[(4 * r + g) * 32 + lr] = o0[r];
+            vt[(4 * r + g) * 32 + 16 + lr] = o1[r];
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
+}
+
+// A chunk of columns of one submatrix's right-hand sides.
+struct Q2Job {
+    int64_t y;    // first element (row 0 of the first column)
+    int64_t blk;  // the submatrix's first block
+    int m, ld, ng, nc;
+};
+
+// Y <- Q2 Y (TRANS false: groups descending, windows ascending) or Q2^T Y (the
+// reverse) for up to 16 CT columns per wavefront.  The 32 rows a block touches sit
+// in registers as two 16 x 16 tiles per 16 columns, in the layout in which
+// v_mfma_f64_16x16x4 takes its B operand and leaves its result (register r of
+// lane l: row 4 r + l / 16, column l % 16), so nothing moves between the two
+// products of a block; the next block shares one tile.  Bound by the matrix
+// cores (16 MFMA per block and 16 columns); the factors come from L1 and L2,
+// shared by the columns of a submatrix.
+template <bool TRANS, int CT>
+__global__ __launch_bounds__(256) void k_q2_apply(const Q2Job *__restrict__ jobs, int njobs,
+                                                  const double *__restrict__ raw_all,
+                                                  const double *__restrict__ vt_all,
+                                                  double *__restrict__ Ya) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PTB_WAVE);
+    const int ji = blockIdx.x * 4 + wave;
+    if (ji >= njobs) return;
+    const Q2Job jb = jobs[ji];
+    const int lane = threadIdx.x % PTB_WAVE, lr = lane & 15, g = lane >> 4;
+    const int m = jb.m;
+    double *y[CT];
+    bool cok[CT];
+#pragma unroll
+    for (int c = 0; c < CT; ++c) {
+        cok[c] = 16 * c + lr < jb.nc;
+        y[c] = Ya + jb.y + (int64_t)min(16 * c + lr, jb.nc - 1) * jb.ld;
+    }
+    // tile t: rows 16 t + 1 .. 16 t + 16
+    auto load = [&](int t, d4_t (&x)[CT]) {
+#pragma unroll
+        for (int c = 0; c < CT; ++c)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int row = 16 * t + 1 + 4 * r + g;
+                const double v = y[c][min(row, m - 1)];
+                x[c][r] = row < m ? v : 0.0;
+            }
+    };
+    auto store = [&](int t, const d4_t (&x)[CT]) {
+#pragma unroll
+        for (int c = 0; c < CT; ++c)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int row = 16 * t + 1 + 4 * r + g;
+                if (row < m && cok[c]) y[c][row] = x[c][r];
+            }
+    };
+    // operands of block b: f1 (refl x rows, 8 slices) and f2 (rows x refl, two
+    // tiles of 4 slices); TRANS takes (V T)^T first and V second
+    auto fetch = [&](int64_t b, double (&f1)[8], double (&f2)[8]) {
+        const double *raw = raw_all + (jb.blk + b) * 256, *vt = vt_all + (jb.blk + b) * 512;
+#pragma unroll
+        for (int ks = 0; ks < 8; ++ks) {
+            if (!TRANS) {
+                f1[ks] = raw[(lr * 15 + 4 * ks + g) & 255];  // V(4 ks + g, lr)
+                f2[ks] = vt[(4 * (ks & 3) + g) * 32 + 16 * (ks >> 2) + lr];
+            } else {
+                f1[ks] = vt[lr * 32 + 4 * ks + g];
+                f2[ks] = raw[((4 * (ks & 3) + g) * 15 + 16 * (ks >> 2) + lr) & 255];
+            }
+        }
+    };
+    auto mask = [&](double (&f1)[8], double (&f2)[8]) {
+#pragma unroll
+        for (int ks = 0; ks < 8; ++ks) {
+            if (!TRANS) {
+                const int rel = 4 * ks + g - lr;
+                if (rel < 0 || rel > 15) f1[ks] = 0.0;
+            } else {
+                const int rel = 16 * (ks >> 2) + lr - (4 * (ks & 3) + g);
+                if (rel < 0 || rel > 15) f2[ks] = 0.0;
+            }
+        }
+    };
+    const int ng = jb.ng;
+    double f1[8], f2[8], n1[8], n2[8];
+    fetch(TRANS ? q2_block(ng, 0, ng - 1) : q2_block(ng, ng - 1, 0), f1, f2);
+    for (int gi = 0; gi < ng; ++gi) {
+        const int G = TRANS ? gi : ng - 1 - gi;
+        const int nb = ng - G;
+        d4_t xa[CT], xb[CT], xn[CT];
+        load(TRANS ? G + nb : G, xa);
+        load(TRANS ? G + nb - 1 : G + 1, xb);
+        for (int ki = 0; ki < nb; ++ki) {
+            const int k = TRANS ? nb - 1 - ki : ki;
+            const bool last = ki + 1 == nb;
+            // the next block's operands and the next tile
+            const int G2 = last ? (TRANS ? min(G + 1, ng - 1) : max(G - 1, 0)) : G;
+            const int k2 = last ? (TRANS ? ng - G2 - 1 : 0) : (TRANS ? k - 1 : k + 1);
+            fetch(q2_block(ng, G2, k2), n1, n2);
+            const int tn = TRANS ? G + k - 1 : G + k + 2;
+            if (!last) load(tn, xn);
+            mask(f1, f2);
+#pragma unroll
+            for (int c = 0; c < CT; ++c) {
+                d4_t &lo = TRANS ? xb[c] : xa[c], &hi = TRANS ? xa[c] : xb[c];
+                d4_t w = d4_t{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+                for (int r = 0; r < 4; ++r) w = __builtin_amdgcn_mfma_f64_16x16x4f64(f1[r], lo[r], w, 0, 0, 0);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) w = __builtin_amdgcn_mfma_f64_16x16x4f64(f1[4 + r], hi[r], w, 0, 0, 0);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) lo = __builtin_amdgcn_mfma_f64_16x16x4f64(f2[r], w[r], lo, 0, 0, 0);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) hi = __builtin_amdgcn_mfma_f64_16x16x4f64(f2[4 + r], w[r], hi, 0, 0, 0);
+            }
+            store(TRANS ? G + k + 1 : G + k, xa);
+#pragma unroll
+            for (int c = 0; c < CT; ++c) {
+                xa[c] = xb[c];
+                xb[c] = xn[c];
+            }
+#pragma unroll
+            for (int ks = 0; ks < 8; ++ks) {
+                f1[ks] = n1[ks];
+                f2[ks] = n2[ks];
+            }
+            if (last) store(TRANS ? G + k : G + k + 1, xa);
+        }
+    }
+}
+
+}  // namespace
+
+namespace ptb {
+
+int64_t band_blocks(int m) {
+    const int64_t ng = q2_groups(m);
+    return ng * (ng + 1) / 2;
+}
+
+int sytrd_band(ptbgpu_ctx *ctx, const std::vector<SubDesc> &desc, double *A, double *d, double *e,
+               double *tau, QFactor &qf) {
+    const int nsm = (int)desc.size();
+    qf.q2blk.assign(nsm, -1);
+    qf.q2raw = qf.q2vt = nullptr;
+    std::vector<int> order;
+    for (int s = 0; s < nsm; ++s)
+        if (desc[s].flags & kSubBand) order.push_back(s);
+    const int nb = (int)order.size();
+    if (nb == 0) return PTBGPU_OK;
+    std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return desc[a].m > desc[b].m; });
+    std::vector<BandSub> subs(nb);
+    int64_t pw = 0, ab = 0, blk = 0;
+    for (int i = 0; i < nb; ++i) {
+        const SubDesc &x = desc[order[i]];
+        subs[i] = {x.off, pw, ab, blk, x.m, x.ld, x.mapoff, q2_groups(x.m)};
+        qf.q2blk[order[i]] = blk;
+        pw += (int64_t)x.ld * 80 + 256;
+        ab += ((int64_t)x.m * kABL + 15) & ~15;
+        blk += band_blocks(x.m);
+    }
+    auto *PW = static_cast<double *>(ws(ctx, "band_pw", sizeof(double) * pw));
+    auto *AB = static_cast<double *>(ws(ctx, "band_ab", sizeof(double) * ab));
+    auto *raw = static_cast<double *>(ws(ctx, "band_q2raw", sizeof(double) * 256 * std::max<int64_t>(blk, 1)));
+    auto *rtau = static_cast<double *>(ws(ctx, "band_q2tau", sizeof(double) * 16 * std::max<int64_t>(blk, 1)));
+    auto *vt = static_cast<double *>(ws(ctx, "band_q2vt", sizeof(double) * 512 * std::max<int64_t>(blk, 1)));
+    if (!PW || !AB || !raw || !rtau || !vt) return PTBGPU_E_NOMEM;
+    auto *ds = static_cast<BandSub *>(upload_table(ctx, "band_subs", subs.data(), sizeof(BandSub) * nb));
+    if (!ds) return PTBGPU_E_NOMEM;
+    qf.q2raw = raw;
+    qf.q2vt = vt;
+    hipStream_t st = ctx->stream;
+    const int max_m = subs[0].m;
+    // submatrices (largest first) of at least `rows` rows
+    auto count = [&](int rows) {
+        return (int)(std::partition_point(subs.begin(), subs.end(), [&](const BandSub &x) { return x.m >= rows; }) -
+                     subs.begin());
+    };
+    // panels: at least two rows below the band
+    const int npanel = max_m >= kBW + 2 ? (max_m - kBW - 2) / kBW + 1 : 0;
+    std::vector<GemmDesc> g;
+    std::vector<int> start(npanel + 1, 0);
+    for (int p = 0; p < npanel; ++p) {
+        start[p] = (int)g.size();
+        const int r0 = (p + 1) * kBW, na = count(r0 + 2);
+        for (int i = 0; i < na; ++i) {
+            const BandSub &x = subs[i];
+            double *w = PW + x.pw + r0, *C = A + x.off + (int64_t)r0 * x.ld + r0;
+            g.push_back({w, w + (int64_t)kBW * x.ld, C, x.m - r0, x.m - r0, 2 * kBW, x.ld, x.ld, x.ld,
+                         -1.0, 1.0, 1, 0});
+        }
+    }
+    start[npanel] = (int)g.size();
+    GemmDesc *dg = nullptr;
+    TileList tl;
+    if (npanel > 0) {
+        dg = static_cast<GemmDesc *>(upload_table(ctx, "band_g", g.data(), sizeof(GemmDesc) * g.size()));
+        if (!dg) return PTBGPU_E_NOMEM;
+        for (int p = 0; p < npanel; ++p) tl.add(g.data() + start[p], start[p + 1] - start[p]);
+        PTB_TRY(tl.upload(ctx, "band_w"));
+    }
+    {
+        ProfScope prof_(ctx, "band_reduce");
+        for (int p = 0; p < npanel; ++p) {
+            const int r0 = (p + 1) * kBW, na = start[p + 1] - start[p];
+            const int n = max_m - r0;  // the tallest panel
+            {
+                ProfScope kprof_(ctx, "band_qr");
+                const int big = count(r0 + 1025);  // panels of more than 1024 rows
+                if (big > 0)
+                    hipLaunchKernelGGL((k_band_qr<512, 4>), dim3(big), dim3(512), 0, st, ds, A, PW, AB, tau, 0, p);
+                const int nl = big < na ? subs[big].m - r0 : 0;
+                if (nl > 512)
+                    hipLaunchKernelGGL((k_band_qr<256, 4>), dim3(na - big), dim3(256), 0, st, ds, A, PW, AB, tau, big, p);
+                else if (nl > 256)
+                    hipLaunchKernelGGL((k_band_qr<256, 2>), dim3(na - big), dim3(256), 0, st, ds, A, PW, AB, tau, big, p);
+                else if (nl > 0)
+                    hipLaunchKernelGGL((k_band_qr<256, 1>), dim3(na - big), dim3(256), 0, st, ds, A, PW, AB, tau, big, p);
+                PTB_CHECK_LAUNCH(ctx);
+            }
+            {
+                ProfScope kprof_(ctx, "band_symm");
+                const int nblk = (n + 63) / 64;
+                hipLaunchKernelGGL(k_band_symm, dim3((unsigned)((na + 7) / 8 * 8 * nblk)), dim3(256), 0, st,
+                                   ds, na, A, PW, p, nblk);
+                PTB_CHECK_LAUNCH(ctx);
+            }
+            {
+                ProfScope kprof_(ctx, "band_w");
+                hipLaunchKernelGGL(k_band_w, dim3(na), dim3(256), 0, st, ds, PW, p);
+                PTB_CHECK_LAUNCH(ctx);
+            }
+            PTB_TRY(tl.launch(ctx, p, false, true, dg + start[p], "sytrd"));
+        }
+        hipLaunchKernelGGL(k_band_extract, dim3(nb, (max_m + kBW - 1) / kBW), dim3(256), 0, st, ds, A, AB,
+                           kQBlk);
+        PTB_CHECK_LAUNCH(ctx);
+    }
+    {
+        ProfScope prof_(ctx, "band_chase");
+        // size classes by the rows a workgroup's registers hold
+        int done = 0;
+        auto lds = [&](int m, int nw) {
+            const int K = std::max((m - 1 + kBW - 1) / kBW, 1);
+            return sizeof(double) * (size_t)(50 * (K + 2) + 16 * nw);
+        };
+#define PTB_CHASE(NW, P, MEM, LOW)                                                                    \
+    do {                                                                                              \
+        const int to = count(LOW);                                                                    \
+        if (to > done) {                                                                              \
+            hipLaunchKernelGGL((k_chase<NW, P, MEM>), dim3(to - done), dim3(NW * 64),                 \
+                               lds(subs[done].m, NW), st, ds, done, AB, raw, rtau, d, e, PW);         \
+            PTB_CHECK_LAUNCH(ctx);                                                                    \
+            done = to;                                                                                \
+        }                                                                                             \
+    } while (0)
+        PTB_CHASE(16, 2, true, 1026);
+        PTB_CHASE(16, 4, false, 514);
+        PTB_CHASE(8, 4, false, 258);
+        PTB_CHASE(4, 4, false, 130);
+        PTB_CHASE(4, 2, false, 66);
+        PTB_CHASE(2, 2, false, 0);
+#undef PTB_CHASE
+    }
+    if (blk > 0) {
+        ProfScope prof_(ctx, "q2_prep");
+        const int nblk = (int)band_blocks(max_m);
+        hipLaunchKernelGGL(k_q2_prep, dim3(nb, (nblk + 4 * kPrepBlk - 1) / (4 * kPrepBlk)), dim3(256), 0, st,
+                           ds, raw, rtau, vt);
+        PTB_CHECK_LAUNCH(ctx);
+    }
+    return PTBGPU_OK;
+}
+
+int apply_q2(ptbgpu_ctx *ctx, const std::vector<SubDesc> &desc, const QFactor &qf, double *Y,
+             const std::vector<int64_t> &yoff, const std::vector<int> &ncols, bool trans,
+             const char *tag) {
+    if (!qf.q2raw) return PTBGPU_OK;
+    ProfScope prof_(ctx, "apply_q2");
+    // two 16-column tiles per wavefront, except for a last piece of at most 16
+    std::vector<Q2Job> wide, narrow;
+    for (int s = 0; s < (int)desc.size(); ++s) {
+        const SubDesc &x = desc[s];
+        if (qf.q2blk[s] < 0 || x.m < 3) continue;
+        for (int c = 0; c < ncols[s]; c += 32) {
+            const int nc = std::min(32, ncols[s] - c);
+            (nc > 16 ? wide : narrow)
+                .push_back({yoff[s] + (int64_t)c * x.ld, qf.q2blk[s], x.m, x.ld, q2_groups(x.m), nc});
+        }
+    }
+    auto run = [&](std::vector<Q2Job> &jobs, const char *nm, bool two) -> int {
+        if (jobs.empty()) return PTBGPU_OK;
+        std::stable_sort(jobs.begin(), jobs.end(), [](const Q2Job &a, const Q2Job &b) { return a.m > b.m; });
+        auto *dj = static_cast<Q2Job *>(
+            upload_table(ctx, (std::string(nm) + tag).c_str(), jobs.data(), sizeof(Q2Job) * jobs.size()));
+        if (!dj) return PTBGPU_E_NOMEM;
+        const dim3 grid((unsigned)((jobs.size() + 3) / 4));
+        auto kern = two ? (trans ? k_q2_apply<true, 2> : k_q2_apply<false, 2>)
+                        : (trans ? k_q2_apply<true, 1> : k_q2_apply<false, 1>);
+        hipLaunchKernelGGL(kern, grid, dim3(256), 0, ctx->stream, dj, (int)jobs.size(), qf.q2raw, qf.q2vt, Y);
+        PTB_CHECK_LAUNCH(ctx);
+        return PTBGPU_OK;
+    };
+    PTB_TRY(run(wide, "q2_jw_", true));
+    return run(narrow, "q2_jn_", false);
+}
+
+}  // namespace ptb

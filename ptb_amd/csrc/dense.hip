@@ -22,11 +22,6 @@
 namespace {
 
 constexpr int kT = 256;
-// reflectors per block of the WY application of Q.  Every reader of the
-// reflector arena (T factors, Q application) reads column c only from row
-// (c rounded down to a block) + 1 on, so only those rows above the unit need
-// to hold zeros.
-constexpr int kQBlk = 128;
 
 typedef double d4_t __attribute__((ext_vector_type(4)));
 
@@ -615,7 +610,7 @@ __global__ __launch_bounds__(kT) void k_larft_all(const SubDesc *__restrict__ de
                                                   const int64_t *__restrict__ toff,
                                                   double *__restrict__ Ta) {
     const SubDesc d = desc[blockIdx.x];
-    const int nr = d.m - 2;
+    const int nr = d.m - 1 - q_shift(d);
     const int nblk = nr > 0 ? (nr + 31) / 32 : 0;
     const int b = blockIdx.y;
     if (b >= nblk) return;
@@ -632,7 +627,7 @@ __global__ __launch_bounds__(kT) void k_larft_all(const SubDesc *__restrict__ de
     // block's rows, 64 at a time through LDS (lane l supplies V(k0 + l/16,
     // i0 + l%16) and V(k0 + l/16, j0 + l%16); result value r of lane l is
     // G(i0 + 4r + l/16, j0 + l%16)).  Column c is zero above its unit at row
-    // b0 + c + 1, so every element runs over rows b0 + 1 .. m - 1.  The next
+    // b0 + c + shift, so every element runs over rows b0 + shift .. m - 1.  The next
     // 64 rows are loaded into registers while the current ones run.
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int i0 = (wave & 1) * 16, j0 = (wave >> 1) * 16;
@@ -657,12 +652,13 @@ __global__ __launch_bounds__(kT) void k_larft_all(const SubDesc *__restrict__ de
             Vs[rr][cc] = (r0 + rr < d.m && cc < kb) ? x[u] : 0.0;
         }
     };
-    if (b0 + 1 < d.m) {
-        load(b0 + 1);
-        stage(b0 + 1);
+    const int rb = b0 + q_shift(d);
+    if (rb < d.m) {
+        load(rb);
+        stage(rb);
     }
     __syncthreads();
-    for (int r0 = b0 + 1; r0 < d.m; r0 += 64) {
+    for (int r0 = rb; r0 < d.m; r0 += 64) {
         const bool more = r0 + 64 < d.m;
         if (more) load(r0 + 64);
 #pragma unroll
@@ -710,7 +706,7 @@ __global__ __launch_bounds__(kT) void k_larft_merge(const SubDesc *__restrict__ 
                                                     const int64_t *__restrict__ toff64,
                                                     double *__restrict__ T64a) {
     const SubDesc d = desc[blockIdx.x];
-    const int nr = d.m - 2;
+    const int nr = d.m - 1 - q_shift(d);
     const int nblk = nr > 0 ? (nr + 31) / 32 : 0;
     const int p = blockIdx.y, b = 2 * p;
     if (b >= nblk) return;
@@ -757,7 +753,7 @@ __global__ __launch_bounds__(kT) void k_larft_merge(const SubDesc *__restrict__ 
                 V2s[rr][cc] = (in && cc < kb2) ? x2[u] : 0.0;
             }
         };
-        const int rb = (b + 1) * 32 + 1;
+        const int rb = (b + 1) * 32 + q_shift(d);
         if (rb < d.m) {
             load(rb);
             stage(rb);
@@ -822,7 +818,7 @@ __global__ __launch_bounds__(kT) void k_t128_assemble(const SubDesc *__restrict_
                                                       const int64_t *__restrict__ toff128,
                                                       double *__restrict__ T128a) {
     const SubDesc d = desc[blockIdx.x];
-    const int nr = d.m - 2;
+    const int nr = d.m - 1 - q_shift(d);
     const int n64 = nr > 0 ? (nr + 63) / 64 : 0;
     const int p = blockIdx.y;
     if (2 * p >= n64) return;
@@ -1457,7 +1453,7 @@ int larft_all(ptbgpu_ctx *ctx, const std::vector<SubDesc> &desc, const SubDesc *
     int64_t tot = 0;
     int maxblk = 0;
     for (int s = 0; s < nsm; ++s) {
-        const int nr = desc[s].m - 2;
+        const int nr = desc[s].m - 1 - q_shift(desc[s]);
         const int nblk = nr > 0 ? (nr + 31) / 32 : 0;
         qf.toff[s] = tot;
         tot += (int64_t)nblk * 1024;
@@ -1471,7 +1467,7 @@ int larft_all(ptbgpu_ctx *ctx, const std::vector<SubDesc> &desc, const SubDesc *
     qf.toff64.assign(nsm, 0);
     int64_t tot64 = 0;
     for (int s = 0; s < nsm; ++s) {
-        const int nr = desc[s].m - 2;
+        const int nr = desc[s].m - 1 - q_shift(desc[s]);
         const int npair = nr > 0 ? (nr + 63) / 64 : 0;
         qf.toff64[s] = tot64;
         tot64 += (int64_t)npair * 4096;
@@ -1494,7 +1490,7 @@ int larft_all(ptbgpu_ctx *ctx, const std::vector<SubDesc> &desc, const SubDesc *
     qf.toff128.assign(nsm, 0);
     int64_t tot128 = 0, npairs = 0;
     for (int s = 0; s < nsm; ++s) {
-        const int nr = desc[s].m - 2;
+        const int nr = desc[s].m - 1 - q_shift(desc[s]);
         const int n64 = nr > 0 ? (nr + 63) / 64 : 0;
         qf.toff128[s] = tot128;
         tot128 += (int64_t)((n64 + 1) / 2) * 16384;
@@ -1513,10 +1509,10 @@ int larft_all(ptbgpu_ctx *ctx, const std::vector<SubDesc> &desc, const SubDesc *
     int64_t sc = 0;
     for (int s = 0; s < nsm; ++s) {
         const SubDesc &d = desc[s];
-        const int nr = d.m - 2;
+        const int nr = d.m - 1 - q_shift(d);
         const int n64 = nr > 0 ? (nr + 63) / 64 : 0;
         for (int p = 0; 2 * p + 1 < n64; ++p) {
-            const int b0 = 128 * p, kb2 = std::min(64, nr - (b0 + 64)), r0 = b0 + 65;
+            const int b0 = 128 * p, kb2 = std::min(64, nr - (b0 + 64)), r0 = b0 + 64 + q_shift(d);
             const double *V1 = V + d.off + (int64_t)b0 * d.ld + r0;
             const double *V2 = V + d.off + (int64_t)(b0 + 64) * d.ld + r0;
             const double *T1 = qf.T64 + qf.toff64[s] + (int64_t)(2 * p) * 4096, *T2 = T1 + 4096;
@@ -1560,7 +1556,9 @@ int apply_q(ptbgpu_ctx *ctx, const std::vector<SubDesc> &desc, const QFactor &qf
     ProfScope prof_(ctx, "apply_q");
     ProfScope tprof_(ctx, (std::string("apply_q_") + tag).c_str());
     const int nsm = (int)desc.size();
-    if (qf.maxblk128 == 0) return PTBGPU_OK;
+    // Q = Q1 Q2 on the band route
+    if (!trans) PTB_TRY(apply_q2(ctx, desc, qf, Y, yoff, ncols, false, tag));
+    if (qf.maxblk128 == 0) return trans ? apply_q2(ctx, desc, qf, Y, yoff, ncols, true, tag) : PTBGPU_OK;
     constexpr int kQB = kQBlk;
     std::vector<int64_t> woff(nsm);
     int64_t wtot = 0;
@@ -1582,14 +1580,14 @@ int apply_q(ptbgpu_ctx *ctx, const std::vector<SubDesc> &desc, const QFactor &qf
         for (int s = 0; s < nsm; ++s) {
             const SubDesc &d = desc[s];
             const int nc = ncols[s];
-            const int nr = d.m - 2;
+            const int nr = d.m - 1 - q_shift(d);
             const int nblk = nr > 0 ? (nr + kQB - 1) / kQB : 0;
             if (nc <= 0 || q >= nblk) continue;
             const int p = trans ? q : nblk - 1 - q;
             const int b0 = p * kQB, kb = std::min(kQB, nr - b0);
-            const int rowsv = d.m - b0 - 1;
-            const double *V = qf.V + d.off + (int64_t)b0 * d.ld + b0 + 1;
-            double *Yb = Y + yoff[s] + b0 + 1;
+            const int sh = q_shift(d), rowsv = d.m - b0 - sh;
+            const double *V = qf.V + d.off + (int64_t)b0 * d.ld + b0 + sh;
+            double *Yb = Y + yoff[s] + b0 + sh;
             const double *T = qf.T128 + qf.toff128[s] + (int64_t)p * kQB * kQB;
             double *w1 = W1 + woff[s], *w2 = W2 + woff[s];
             g1.push_back({V, Yb, w1, kb, nc, rowsv, d.ld, d.ld, kQB, 1.0, 0.0});
@@ -1599,7 +1597,7 @@ int apply_q(ptbgpu_ctx *ctx, const std::vector<SubDesc> &desc, const QFactor &qf
     }
     start[qf.maxblk128] = (int)g1.size();
     const std::string t(tag);
-    if (g1.empty()) return PTBGPU_OK;
+    if (g1.empty()) return trans ? apply_q2(ctx, desc, qf, Y, yoff, ncols, true, tag) : PTBGPU_OK;
     const size_t gb = sizeof(GemmDesc) * g1.size();
     GemmDesc *dg1 = static_cast<GemmDesc *>(upload_table(ctx, ("q_g1_" + t).c_str(), g1.data(), gb));
     GemmDesc *dg2 = static_cast<GemmDesc *>(upload_table(ctx, ("q_g2_" + t).c_str(), g2.data(), gb));
@@ -1621,7 +1619,7 @@ int apply_q(ptbgpu_ctx *ctx, const std::vector<SubDesc> &desc, const QFactor &qf
         PTB_TRY(t2.launch(ctx, q, trans, false, dg2 + start[q], "q"));
         PTB_TRY(t3.launch(ctx, q, false, false, dg3 + start[q], "q"));
     }
-    return PTBGPU_OK;
+    return trans ? apply_q2(ctx, desc, qf, Y, yoff, ncols, true, tag) : PTBGPU_OK;
 }
 
 }  // namespace ptb

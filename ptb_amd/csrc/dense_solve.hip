@@ -68,7 +68,7 @@ std::vector<SubDesc> one_desc(int64_t n) {
     d.mapoff = 0;
     d.gbeg = 0;
     d.gend = (int)n;
-    d.flags = 0;
+    d.flags = band_flag(d.m);
     return {d};
 }
 

@@ -377,7 +377,8 @@ int refine_occupied(ptbgpu_ctx *ctx, const std::vector<SubDesc> &desc, const Sub
 const char *const kChunkBufs[] = {"sm_A",      "sm_B",       "sm_Z",  "sm_W",   "sm_X",
                                   "sm_Li",     "sm_K32",     "sm_V",  "sm_R",   "sm_xa",
                                   "sm_f",      "sytrd_pw",   "sytrd_pw32", "q_T", "q_T64",
-                                  "q_T128",    "q_t128_gm"};
+                                  "q_T128",    "q_t128_gm", "band_pw",   "band_ab",
+                                  "band_q2raw", "band_q2tau", "band_q2vt"};
 
 // Device bytes the per-submatrix arenas of one chunk may take: the free
 // device memory plus what this context holds in the chunk-sized buffers
@@ -592,6 +593,7 @@ int sm_density_batch_device(ptbgpu_ctx *ctx, const std::vector<MolIn> &mols, int
             d.gbeg = gptr[s];
             d.gend = gptr[s + 1];
             d.flags = mixed && d.m < ctx->mixed_min_m ? kSubExact : 0;
+            if (!mixed || d.flags) d.flags |= band_flag(d.m);
             d.mol = i;
             arena += (int64_t)d.ld * d.m;
             rows += d.m;
@@ -636,7 +638,10 @@ int sm_density_batch_device(ptbgpu_ctx *ctx, const std::vector<MolIn> &mols, int
             // panel buffer (ld x 96) and the 32/64/128-reflector T factors
             const size_t c = per_elem * (size_t)desc[s].ld * desc[s].m +
                              2 * sizeof(double) * (size_t)desc[s].ld * 2 * (desc[s].gend - desc[s].gbeg) +
-                             sizeof(double) * (size_t)desc[s].ld * (96 + 32 + 64 + 128);
+                             sizeof(double) * (size_t)desc[s].ld * (96 + 32 + 64 + 128) +
+                             (desc[s].flags & kSubBand
+                                  ? sizeof(double) * (256 + 16 + 512) * (size_t)ptb::band_blocks(desc[s].m)
+                                  : 0);
             if (used > 0 && used + c > budget) {
                 cb.push_back(s);
                 used = 0;
@@ -1099,6 +1104,24 @@ int check_sm_args(ptbgpu_ctx *ctx, int64_t ndim, int64_t nelref, const void *H, 
 
 namespace ptb {
 
+// One-stage FP64 tridiagonalisation of the submatrices that are not on the band
+// route, A = V afterwards.
+static int sytrd_rest(ptbgpu_ctx *ctx, const std::vector<SubDesc> &desc, const SubDesc *ddesc, double *A,
+                      double *d, double *e, double *tau) {
+    std::vector<SubDesc> rest;
+    int max_m = 0;
+    for (const auto &x : desc)
+        if (!(x.flags & kSubBand)) {
+            rest.push_back(x);
+            max_m = std::max(max_m, x.m);
+        }
+    if (rest.empty()) return PTBGPU_OK;
+    SubDesc *dr = const_cast<SubDesc *>(ddesc);
+    if (rest.size() < desc.size()) PTB_TRY(upload(ctx, "sm_desc_rest", rest, &dr));
+    PTB_TRY(sytrd_batch(ctx, rest, dr, A, d, e, tau));
+    return zero_upper_batch(ctx, dr, (int)rest.size(), max_m, A);
+}
+
 // Tridiagonal eigendecomposition of a batch of dense symmetric matrices (full
 // storage in A, both triangles): Householder tridiagonalisation A = Q T Q^T and
 // divide and conquer T = Z diag(d) Z^T.  On return Z holds the eigenvectors of
@@ -1146,13 +1169,13 @@ int eig_tri_batch(ptbgpu_ctx *ctx, const std::vector<SubDesc> &desc, const SubDe
         if (!ex.empty()) {
             const int n = (int)ex.size();
             PTB_TRY(copy_lower_batch(ctx, dex, n, ex_m, A, V));
-            PTB_TRY(sytrd_batch(ctx, ex, dex, V, dvec, evec, tau));
-            PTB_TRY(zero_upper_batch(ctx, dex, n, ex_m, V));
+            PTB_TRY(sytrd_rest(ctx, ex, dex, V, dvec, evec, tau));
+            PTB_TRY(sytrd_band(ctx, desc, V, dvec, evec, tau, qf));
         }
         PTB_TRY(larft_all(ctx, desc, ddesc, V, tau, qf));
     } else {
-        PTB_TRY(sytrd_batch(ctx, desc, ddesc, A, dvec, evec, tau));
-        PTB_TRY(zero_upper_batch(ctx, ddesc, nsm, max_m, A));              // A = V
+        PTB_TRY(sytrd_rest(ctx, desc, ddesc, A, dvec, evec, tau));
+        PTB_TRY(sytrd_band(ctx, desc, A, dvec, evec, tau, qf));
         PTB_TRY(larft_all(ctx, desc, ddesc, A, tau, qf));
     }
     // divide and conquer

@@ -19,9 +19,25 @@ struct SubDesc {
     int pad;
 };
 constexpr int kSubExact = 2;
+// bit 2: tridiagonalised through a band (band.hip); its reflector c has its
+// unit at row c + kBandWidth instead of c + 1
+constexpr int kSubBand = 4;
+constexpr int kBandWidth = 16;
+// the largest matrix of the band route: a panel's rows fit the registers of a
+// workgroup
+constexpr int kBandMaxM = 2048;
+inline int band_flag(int m) { return m <= kBandMaxM ? kSubBand : 0; }
 // the largest dense matrix or submatrix the eigensolver takes (n^2 < 2^31:
 // 32-bit element offsets inside a matrix)
 constexpr int kDenseMax = 32768;
+
+// row of reflector c's unit below c
+__host__ __device__ inline int q_shift(const SubDesc &d) { return d.flags & kSubBand ? kBandWidth : 1; }
+// reflectors per block of the WY application of Q.  Every reader of the
+// reflector arena (T factors, Q application) reads column c only from row
+// (c rounded down to a block) + q_shift on, so only those rows above the unit
+// need to hold zeros.
+constexpr int kQBlk = 128;
 
 // One molecule of a batch on the device: its packed matrices and where its
 // pattern bitmap, its submatrices' row unions and its submatrices begin.
@@ -99,6 +115,11 @@ struct QFactor {
     double *T128 = nullptr;       // 128 x 128 factors of pairs of those (what apply_q uses)
     std::vector<int64_t> toff128;
     int maxblk128 = 0;
+    // band route: reflectors of the chase (16 x 16 per block) and -(V T) of
+    // every block (32 x 16); first block per submatrix (-1: not on that route)
+    const double *q2raw = nullptr;
+    const double *q2vt = nullptr;
+    std::vector<int64_t> q2blk;
 };
 
 // Right-hand sides of a batched triangular solve that are not the submatrices'
@@ -206,6 +227,19 @@ int promote_reflectors(ptbgpu_ctx *ctx, const SubDesc *ddesc, int nsm, int max_m
 int apply_q(ptbgpu_ctx *ctx, const std::vector<SubDesc> &desc, const QFactor &qf, double *Y,
             const std::vector<int64_t> &yoff, const std::vector<int> &ncols, bool trans,
             const char *tag);
+
+// band.hip
+// blocks of chase reflectors of one submatrix of m rows
+int64_t band_blocks(int m);
+// FP64 tridiagonalisation of the submatrices flagged kSubBand (lower triangle
+// of A): d and e, the reflectors and tau of the band reduction in A, and the
+// chase's in qf
+int sytrd_band(ptbgpu_ctx *ctx, const std::vector<SubDesc> &desc, double *A, double *d, double *e,
+               double *tau, QFactor &qf);
+// Y <- Q2 Y or Q2^T Y for those submatrices
+int apply_q2(ptbgpu_ctx *ctx, const std::vector<SubDesc> &desc, const QFactor &qf, double *Y,
+             const std::vector<int64_t> &yoff, const std::vector<int> &ncols, bool trans,
+             const char *tag);
 
 // tridiag.hip
 int sytrd_batch(ptbgpu_ctx *ctx, const std::vector<SubDesc> &desc, const SubDesc *ddesc,
