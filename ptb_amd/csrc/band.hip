@@ -26,6 +26,7 @@
 // overlap only their neighbours, and this order keeps every overlapping pair).
 #include <algorithm>
 #include <type_traits>
+#include <utility>
 
 #include "sm_internal.hpp"
 
@@ -651,16 +652,16 @@ __global__ __launch_bounds__(NW * 64) void k_chase(const BandSub *__restrict__ s
 
 // ---- application of Q2 ---------------------------------------------------------
 
-// Factor of every block of 16 reflectors: with V the block's 31 x 16
-// parallelogram (reflector j at rows j .. j + 15) and T its WY factor,
-// -(V T) is stored as vt[refl * 32 + row].  Reflectors that the chase never
-// made (past the last sweep or window) are cleared.  One wavefront per block,
-// kPrepBlk blocks each.  grid: (submatrix, ceil(blocks / (4 kPrepBlk)))
+// Factors of every block of 16 reflectors: V, the block's 31 x 16 parallelogram
+// (reflector j at rows j .. j + 15), and -(V T), T its WY factor, both 32 x 16 by
+// rows (V at fac, -(V T) at fac + 512).  Reflectors that the chase never made
+// (past the last sweep or window) are zero.  One wavefront per block, kPrepBlk
+// blocks each.  grid: (submatrix, ceil(blocks / (4 kPrepBlk)))
 constexpr int kPrepBlk = 4;
 __global__ __launch_bounds__(256, 4) void k_q2_prep(const BandSub *__restrict__ subs,
-                                                 double *__restrict__ raw_all,
+                                                 const double *__restrict__ raw_all,
                                                  const double *__restrict__ rtau_all,
-                                                 double *__restrict__ vt_all) {
+                                                 double *__restrict__ fac_all) {
     const BandSub d = subs[blockIdx.x];
     const int lane = threadIdx.x % PTB_WAVE, wave = threadIdx.x / PTB_WAVE;
     const int lr = lane & 15, g = lane >> 4;
@@ -680,19 +681,15 @@ __global__ __launch_bounds__(256, 4) void k_q2_prep(const BandSub *__restrict__ 
         }
         const int k = bi - (int)q2_block(d.ng, G, 0);
         const int64_t blk = d.blk + bi;
-        double *raw = raw_all + blk * 256;
-        double *vt = vt_all + blk * 512;
+        const double *raw = raw_all + blk * 256;
+        double *fac = fac_all + blk * 1024;
         // reflector 16 G + j exists for j < nv
         const int nv = min(16, min(d.m - 2 - 16 * G, d.m - 2 - 16 * (G + k)));
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             const int j = 4 * q + g;
-            double v = raw[j * 16 + lr];
-            if (j >= nv) {
-                v = 0.0;
-                raw[j * 16 + lr] = 0.0;
-            }
-            vs[j][lr] = v;
+            const double v = raw[j * 16 + lr];
+            vs[j][lr] = j < nv ? v : 0.0;
         }
         double tj = lr < nv ? rtau_all[blk * 16 + lr] : 0.0;
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -704,6 +701,7 @@ __global__ __launch_bounds__(256, 4) void k_q2_prep(const BandSub *__restrict__ 
             const double x = vs[lr][rel & 15];
             const double v = (rel >= 0 && rel < 16) ? x : 0.0;
             acc = __builtin_amdgcn_mfma_f64_16x16x4f64(v, v, acc, 0, 0, 0);
+            fac[(4 * ks + g) * 16 + lr] = v;
         }
 #pragma unroll
         for (int r = 0; r < 4; ++r) gs[4 * r + g][lr] = acc[r];
@@ -728,7 +726,7 @@ __global__ __launch_bounds__(256, 4) void k_q2_prep(const BandSub *__restrict__ 
 #pragma unroll
         for (int q = 0; q < 4; ++q) ths[wave][lr][4 * g + q] = t[q];
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        // (V T)^T(refl, row) = sum_c T(c, refl) V(row, c)
+        // V T(row, refl) = sum_c V(row, c) T(c, refl)
         d4_t o0 = d4_t{0.0, 0.0, 0.0, 0.0}, o1 = o0;
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
@@ -736,17 +734,19 @@ __global__ __launch_bounds__(256, 4) void k_q2_prep(const BandSub *__restrict__ 
             const double tc = -ths[wave][c][lr];
             const int e0 = lr - c, e1 = 16 + lr - c;
             const double x0 = vs[c][e0 & 15], x1 = vs[c][e1 & 15];
-            o0 = __builtin_amdgcn_mfma_f64_16x16x4f64(tc, e0 >= 0 ? x0 : 0.0, o0, 0, 0, 0);
-            o1 = __builtin_amdgcn_mfma_f64_16x16x4f64(tc, e1 < 16 ? x1 : 0.0, o1, 0, 0, 0);
+            o0 = __builtin_amdgcn_mfma_f64_16x16x4f64(e0 >= 0 ? x0 : 0.0, tc, o0, 0, 0, 0);
+            o1 = __builtin_amdgcn_mfma_f64_16x16x4f64(e1 < 16 ? x1 : 0.0, tc, o1, 0, 0, 0);
         }
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            vt[(4 * r + g) * 32 + lr] = o0[r];
-            vt[(4 * r + g) * 32 + 16 + lr] = o1[r];
+            fac[512 + (4 * r + g) * 16 + lr] = o0[r];
+            fac[768 + (4 * r + g) * 16 + lr] = o1[r];
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     }
 }
+
+constexpr int kQ2Groups = 4;  // sweep groups per pass of k_q2_apply (even)
 
 // A chunk of columns of one submatrix's right-hand sides.
 struct Q2Job {
@@ -758,121 +758,167 @@ struct Q2Job {
 // Y <- Q2 Y (TRANS false: groups descending, windows ascending) or Q2^T Y (the
 // reverse) for up to 16 CT columns per wavefront.  The 32 rows a block touches sit
 // in registers as two 16 x 16 tiles per 16 columns, in the layout in which
-// v_mfma_f64_16x16x4 takes its B operand and leaves its result (register r of
-// lane l: row 4 r + l / 16, column l % 16), so nothing moves between the two
-// products of a block; the next block shares one tile.  Bound by the matrix
-// cores (16 MFMA per block and 16 columns); the factors come from L1 and L2,
-// shared by the columns of a submatrix.
+// v_mfma_f64_16x16x4 takes its B operand and leaves its result, so nothing moves
+// between the two products of a block; the next block shares one tile.  The
+// matrix instruction's row 4 r + g (register r, lane group g) stands for row
+// 4 g + r of the tile, so a lane's four values are four consecutive rows (two
+// 16-byte accesses), and for reflector 4 g + r between the products, so the
+// second factor is read 32 bytes per lane.
+//
+// Q groups run in one pass over the rows, group after group one window behind
+// the previous one: a window's step applies Q blocks to Q + 1 tiles, and each tile is
+// read and written once per Q groups.  On the 512-water box (1.5e6 blocks, 126
+// columns on average) one group per pass moved 43 GB of right-hand sides beside
+// 12 GB of factors and took 24.5 ms for both applications; four take 15.7.
+// Factors are fetched two blocks ahead, tiles three windows ahead.
 template <bool TRANS, int CT>
-__global__ __launch_bounds__(256) void k_q2_apply(const Q2Job *__restrict__ jobs, int njobs,
-                                                  const double *__restrict__ raw_all,
-                                                  const double *__restrict__ vt_all,
-                                                  double *__restrict__ Ya) {
+__global__ __launch_bounds__(256, 2) void k_q2_apply(const Q2Job *__restrict__ jobs, int njobs,
+                                                     const double *__restrict__ fac_all,
+                                                     double *__restrict__ Ya) {
+    typedef double d2u_t __attribute__((ext_vector_type(2), aligned(8)));
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PTB_WAVE);
     const int ji = blockIdx.x * 4 + wave;
     if (ji >= njobs) return;
     const Q2Job jb = jobs[ji];
     const int lane = threadIdx.x % PTB_WAVE, lr = lane & 15, g = lane >> 4;
-    const int m = jb.m;
+    const int m = jb.m, ng = jb.ng;
     double *y[CT];
     bool cok[CT];
 #pragma unroll
     for (int c = 0; c < CT; ++c) {
         cok[c] = 16 * c + lr < jb.nc;
-        y[c] = Ya + jb.y + (int64_t)min(16 * c + lr, jb.nc - 1) * jb.ld;
+        y[c] = Ya + jb.y + (int64_t)min(16 * c + lr, jb.nc - 1) * jb.ld + 1 + 4 * g;
     }
-    // tile t: rows 16 t + 1 .. 16 t + 16
+    // tile t: rows 16 t + 1 .. 16 t + 16, the last one cut at m (t < 0: none)
     auto load = [&](int t, d4_t (&x)[CT]) {
+        if (t < 0) {
 #pragma unroll
-        for (int c = 0; c < CT; ++c)
+            for (int c = 0; c < CT; ++c) x[c] = d4_t{0.0, 0.0, 0.0, 0.0};
+        } else if (16 * t + 17 <= m) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int row = 16 * t + 1 + 4 * r + g;
-                const double v = y[c][min(row, m - 1)];
-                x[c][r] = row < m ? v : 0.0;
+            for (int c = 0; c < CT; ++c) {
+                const d2u_t *p = reinterpret_cast<const d2u_t *>(y[c] + 16 * t);
+                const d2u_t u = p[0], v = p[1];
+                x[c] = d4_t{u[0], u[1], v[0], v[1]};
             }
+        } else {
+#pragma unroll
+            for (int c = 0; c < CT; ++c)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int row = 16 * t + 1 + 4 * g + r;
+                    const double v = y[c][min(row, m - 1) - 1 - 4 * g];
+                    x[c][r] = row < m ? v : 0.0;
+                }
+        }
     };
     auto store = [&](int t, const d4_t (&x)[CT]) {
+        if (t < 0) return;
+        if (16 * t + 17 <= m) {
 #pragma unroll
-        for (int c = 0; c < CT; ++c)
+            for (int c = 0; c < CT; ++c)
+                if (cok[c]) {
+                    d2u_t *p = reinterpret_cast<d2u_t *>(y[c] + 16 * t);
+                    p[0] = d2u_t{x[c][0], x[c][1]};
+                    p[1] = d2u_t{x[c][2], x[c][3]};
+                }
+        } else {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int row = 16 * t + 1 + 4 * r + g;
-                if (row < m && cok[c]) y[c][row] = x[c][r];
-            }
-    };
-    // operands of block b: f1 (refl x rows, 8 slices) and f2 (rows x refl, two
-    // tiles of 4 slices); TRANS takes (V T)^T first and V second
-    auto fetch = [&](int64_t b, double (&f1)[8], double (&f2)[8]) {
-        const double *raw = raw_all + (jb.blk + b) * 256, *vt = vt_all + (jb.blk + b) * 512;
+            for (int c = 0; c < CT; ++c)
 #pragma unroll
-        for (int ks = 0; ks < 8; ++ks) {
-            if (!TRANS) {
-                f1[ks] = raw[(lr * 15 + 4 * ks + g) & 255];  // V(4 ks + g, lr)
-                f2[ks] = vt[(4 * (ks & 3) + g) * 32 + 16 * (ks >> 2) + lr];
-            } else {
-                f1[ks] = vt[lr * 32 + 4 * ks + g];
-                f2[ks] = raw[((4 * (ks & 3) + g) * 15 + 16 * (ks >> 2) + lr) & 255];
-            }
+                for (int r = 0; r < 4; ++r)
+                    if (16 * t + 1 + 4 * g + r < m && cok[c]) y[c][16 * t + r] = x[c][r];
         }
     };
-    auto mask = [&](double (&f1)[8], double (&f2)[8]) {
-#pragma unroll
-        for (int ks = 0; ks < 8; ++ks) {
-            if (!TRANS) {
-                const int rel = 4 * ks + g - lr;
-                if (rel < 0 || rel > 15) f1[ks] = 0.0;
-            } else {
-                const int rel = 16 * (ks >> 2) + lr - (4 * (ks & 3) + g);
-                if (rel < 0 || rel > 15) f2[ks] = 0.0;
-            }
-        }
+    // block (G, k)'s operands: f1 (reflectors x rows, slice s: row 4 g + s of the
+    // low and the high tile), f2 (rows x reflectors, slice s: reflector 4 g + s)
+    const int pr = 4 * (lr & 3) + (lr >> 2);
+    const double *f1a = fac_all + jb.blk * 1024 + (TRANS ? 512 : 0) + 64 * g + pr;
+    const double *f2a = fac_all + jb.blk * 1024 + (TRANS ? 0 : 512) + 16 * pr + 4 * g;
+    struct Fac {
+        double f1[8], f2[8];
     };
-    const int ng = jb.ng;
-    double f1[8], f2[8], n1[8], n2[8];
-    fetch(TRANS ? q2_block(ng, 0, ng - 1) : q2_block(ng, ng - 1, 0), f1, f2);
-    for (int gi = 0; gi < ng; ++gi) {
-        const int G = TRANS ? gi : ng - 1 - gi;
-        const int nb = ng - G;
-        d4_t xa[CT], xb[CT], xn[CT];
-        load(TRANS ? G + nb : G, xa);
-        load(TRANS ? G + nb - 1 : G + 1, xb);
-        for (int ki = 0; ki < nb; ++ki) {
-            const int k = TRANS ? nb - 1 - ki : ki;
-            const bool last = ki + 1 == nb;
-            // the next block's operands and the next tile
-            const int G2 = last ? (TRANS ? min(G + 1, ng - 1) : max(G - 1, 0)) : G;
-            const int k2 = last ? (TRANS ? ng - G2 - 1 : 0) : (TRANS ? k - 1 : k + 1);
-            fetch(q2_block(ng, G2, k2), n1, n2);
-            const int tn = TRANS ? G + k - 1 : G + k + 2;
-            if (!last) load(tn, xn);
-            mask(f1, f2);
+    auto fetch = [&](int64_t b, Fac &f) {
+        const double *p1 = f1a + b * 1024;
+        const d2_t *p2 = reinterpret_cast<const d2_t *>(f2a + b * 1024);
 #pragma unroll
-            for (int c = 0; c < CT; ++c) {
-                d4_t &lo = TRANS ? xb[c] : xa[c], &hi = TRANS ? xa[c] : xb[c];
-                d4_t w = d4_t{0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-                for (int r = 0; r < 4; ++r) w = __builtin_amdgcn_mfma_f64_16x16x4f64(f1[r], lo[r], w, 0, 0, 0);
-#pragma unroll
-                for (int r = 0; r < 4; ++r) w = __builtin_amdgcn_mfma_f64_16x16x4f64(f1[4 + r], hi[r], w, 0, 0, 0);
-#pragma unroll
-                for (int r = 0; r < 4; ++r) lo = __builtin_amdgcn_mfma_f64_16x16x4f64(f2[r], w[r], lo, 0, 0, 0);
-#pragma unroll
-                for (int r = 0; r < 4; ++r) hi = __builtin_amdgcn_mfma_f64_16x16x4f64(f2[4 + r], w[r], hi, 0, 0, 0);
-            }
-            store(TRANS ? G + k + 1 : G + k, xa);
-#pragma unroll
-            for (int c = 0; c < CT; ++c) {
-                xa[c] = xb[c];
-                xb[c] = xn[c];
-            }
-#pragma unroll
-            for (int ks = 0; ks < 8; ++ks) {
-                f1[ks] = n1[ks];
-                f2[ks] = n2[ks];
-            }
-            if (last) store(TRANS ? G + k : G + k + 1, xa);
+        for (int s = 0; s < 4; ++s) {
+            f.f1[s] = p1[16 * s];
+            f.f1[4 + s] = p1[256 + 16 * s];
         }
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                const d2_t v = p2[128 * h + s];
+                f.f2[4 * h + 2 * s] = v[0];
+                f.f2[4 * h + 2 * s + 1] = v[1];
+            }
+    };
+    // A pass takes the groups A, A - 1, .. A - Q + 1 (TRANS in the other order; the
+    // last pass may reach below group 0).  At step i the window is k = i (TRANS:
+    // from the top), the h-th group's block touches the tiles met at positions
+    // i + Q - 1 - h and i + Q - h, and position i is finished.  Position o lives
+    // in buffer o mod S and the steps are unrolled by S, so that every buffer is
+    // a fixed set of registers (moving one would wait for its loads); Q more
+    // steps only store.
+    constexpr int Q = kQ2Groups, S = 8;
+    Fac F[2];
+    d4_t X[S][CT];
+    const int npass = (ng + Q - 1) / Q;
+    for (int pass = 0; pass < npass; ++pass) {
+        const int A = ng - 1 - Q * (TRANS ? npass - 1 - pass : pass);
+        const int n = ng - A + Q - 1;  // steps that hold blocks
+        auto tile = [&](int o) { return A - Q + 1 + (TRANS ? n + Q - 1 - o : o); };
+        auto group = [&](int h) { return TRANS ? A - Q + 1 + h : A - h; };
+        auto window = [&](int i) { return TRANS ? n - 1 - i : i; };
+        auto valid = [&](int i, int h) {
+            const int G = group(h), k = window(i);
+            return G >= 0 && k >= 0 && k < ng - G;
+        };
+        auto get = [&](int i, int h, Fac &f) {
+            const int G = max(group(h), 0), k = min(max(window(i), 0), ng - G - 1);
+            fetch(q2_block(ng, G, k), f);
+        };
+        get(0, 0, F[0]);
+        get(0, 1, F[1]);
+        [&]<int... O>(std::integer_sequence<int, O...>) {
+            ((O < n + Q ? load(tile(O), X[O]) : (void)0), ...);
+        }(std::make_integer_sequence<int, S>{});
+        auto step = [&](auto U, int i) {
+            constexpr int u = decltype(U)::value;
+            auto block = [&](auto H) {
+                constexpr int h = decltype(H)::value;
+                constexpr int o0 = (u + Q - 1 - h) % S, o1 = (u + Q - h) % S;
+                Fac &f = F[h & 1];
+                if (valid(i, h)) {
+#pragma unroll
+                    for (int c = 0; c < CT; ++c) {
+                        d4_t &lo = X[TRANS ? o1 : o0][c], &hi = X[TRANS ? o0 : o1][c];
+                        d4_t w = d4_t{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) w = __builtin_amdgcn_mfma_f64_16x16x4f64(f.f1[r], lo[r], w, 0, 0, 0);
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) w = __builtin_amdgcn_mfma_f64_16x16x4f64(f.f1[4 + r], hi[r], w, 0, 0, 0);
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            lo = __builtin_amdgcn_mfma_f64_16x16x4f64(f.f2[r], w[r], lo, 0, 0, 0);
+                            hi = __builtin_amdgcn_mfma_f64_16x16x4f64(f.f2[4 + r], w[r], hi, 0, 0, 0);
+                        }
+                    }
+                }
+                get(h + 2 < Q ? i : i + 1, (h + 2) % Q, f);
+            };
+            [&]<int... H>(std::integer_sequence<int, H...>) {
+                (block(std::integral_constant<int, H>{}), ...);
+            }(std::make_integer_sequence<int, Q>{});
+            store(tile(i), X[u]);
+            if (i + S < n + Q) load(tile(i + S), X[u]);
+        };
+        for (int i = 0; i < n + Q; i += S)
+            [&]<int... U>(std::integer_sequence<int, U...>) {
+                ((i + U < n + Q ? step(std::integral_constant<int, U>{}, i + U) : (void)0), ...);
+            }(std::make_integer_sequence<int, S>{});
     }
 }
 
@@ -889,7 +935,7 @@ int sytrd_band(ptbgpu_ctx *ctx, const std::vector<SubDesc> &desc, double *A, dou
                double *tau, QFactor &qf) {
     const int nsm = (int)desc.size();
     qf.q2blk.assign(nsm, -1);
-    qf.q2raw = qf.q2vt = nullptr;
+    qf.q2fac = nullptr;
     std::vector<int> order;
     for (int s = 0; s < nsm; ++s)
         if (desc[s].flags & kSubBand) order.push_back(s);
@@ -910,12 +956,11 @@ int sytrd_band(ptbgpu_ctx *ctx, const std::vector<SubDesc> &desc, double *A, dou
     auto *AB = static_cast<double *>(ws(ctx, "band_ab", sizeof(double) * ab));
     auto *raw = static_cast<double *>(ws(ctx, "band_q2raw", sizeof(double) * 256 * std::max<int64_t>(blk, 1)));
     auto *rtau = static_cast<double *>(ws(ctx, "band_q2tau", sizeof(double) * 16 * std::max<int64_t>(blk, 1)));
-    auto *vt = static_cast<double *>(ws(ctx, "band_q2vt", sizeof(double) * 512 * std::max<int64_t>(blk, 1)));
-    if (!PW || !AB || !raw || !rtau || !vt) return PTBGPU_E_NOMEM;
+    auto *fac = static_cast<double *>(ws(ctx, "band_q2fac", sizeof(double) * 1024 * std::max<int64_t>(blk, 1)));
+    if (!PW || !AB || !raw || !rtau || !fac) return PTBGPU_E_NOMEM;
     auto *ds = static_cast<BandSub *>(upload_table(ctx, "band_subs", subs.data(), sizeof(BandSub) * nb));
     if (!ds) return PTBGPU_E_NOMEM;
-    qf.q2raw = raw;
-    qf.q2vt = vt;
+    qf.q2fac = fac;
     hipStream_t st = ctx->stream;
     const int max_m = subs[0].m;
     // submatrices (largest first) of at least `rows` rows
@@ -1013,7 +1058,7 @@ int sytrd_band(ptbgpu_ctx *ctx, const std::vector<SubDesc> &desc, double *A, dou
         ProfScope prof_(ctx, "q2_prep");
         const int nblk = (int)band_blocks(max_m);
         hipLaunchKernelGGL(k_q2_prep, dim3(nb, (nblk + 4 * kPrepBlk - 1) / (4 * kPrepBlk)), dim3(256), 0, st,
-                           ds, raw, rtau, vt);
+                           ds, raw, rtau, fac);
         PTB_CHECK_LAUNCH(ctx);
     }
     return PTBGPU_OK;
@@ -1022,15 +1067,21 @@ int sytrd_band(ptbgpu_ctx *ctx, const std::vector<SubDesc> &desc, double *A, dou
 int apply_q2(ptbgpu_ctx *ctx, const std::vector<SubDesc> &desc, const QFactor &qf, double *Y,
              const std::vector<int64_t> &yoff, const std::vector<int> &ncols, bool trans,
              const char *tag) {
-    if (!qf.q2raw) return PTBGPU_OK;
+    if (!qf.q2fac) return PTBGPU_OK;
     ProfScope prof_(ctx, "apply_q2");
-    // two 16-column tiles per wavefront, except for a last piece of at most 16
+    // two 16-column tiles per wavefront (each factor feeds both) where that leaves
+    // a wavefront for every SIMD, else one; one for a last piece of at most 16, and
+    // for Q2^T (few columns; two tiles would spill registers there)
+    int64_t pairs = 0;
+    for (int s = 0; s < (int)desc.size(); ++s)
+        if (qf.q2blk[s] >= 0) pairs += (ncols[s] + 31) / 32;
+    const int step = !trans && pairs >= 4 * (int64_t)ctx->num_cus ? 32 : 16;
     std::vector<Q2Job> wide, narrow;
     for (int s = 0; s < (int)desc.size(); ++s) {
         const SubDesc &x = desc[s];
         if (qf.q2blk[s] < 0 || x.m < 3) continue;
-        for (int c = 0; c < ncols[s]; c += 32) {
-            const int nc = std::min(32, ncols[s] - c);
+        for (int c = 0; c < ncols[s]; c += step) {
+            const int nc = std::min(step, ncols[s] - c);
             (nc > 16 ? wide : narrow)
                 .push_back({yoff[s] + (int64_t)c * x.ld, qf.q2blk[s], x.m, x.ld, q2_groups(x.m), nc});
         }
@@ -1042,9 +1093,8 @@ int apply_q2(ptbgpu_ctx *ctx, const std::vector<SubDesc> &desc, const QFactor &q
             upload_table(ctx, (std::string(nm) + tag).c_str(), jobs.data(), sizeof(Q2Job) * jobs.size()));
         if (!dj) return PTBGPU_E_NOMEM;
         const dim3 grid((unsigned)((jobs.size() + 3) / 4));
-        auto kern = two ? (trans ? k_q2_apply<true, 2> : k_q2_apply<false, 2>)
-                        : (trans ? k_q2_apply<true, 1> : k_q2_apply<false, 1>);
-        hipLaunchKernelGGL(kern, grid, dim3(256), 0, ctx->stream, dj, (int)jobs.size(), qf.q2raw, qf.q2vt, Y);
+        auto kern = two ? k_q2_apply<false, 2> : trans ? k_q2_apply<true, 1> : k_q2_apply<false, 1>;
+        hipLaunchKernelGGL(kern, grid, dim3(256), 0, ctx->stream, dj, (int)jobs.size(), qf.q2fac, Y);
         PTB_CHECK_LAUNCH(ctx);
         return PTBGPU_OK;
     };

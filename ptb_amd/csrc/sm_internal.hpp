@@ -115,10 +115,9 @@ struct QFactor {
     double *T128 = nullptr;       // 128 x 128 factors of pairs of those (what apply_q uses)
     std::vector<int64_t> toff128;
     int maxblk128 = 0;
-    // band route: reflectors of the chase (16 x 16 per block) and -(V T) of
-    // every block (32 x 16); first block per submatrix (-1: not on that route)
-    const double *q2raw = nullptr;
-    const double *q2vt = nullptr;
+    // band route: factors of the chase's reflector blocks (V and -(V T), 32 x 16
+    // each); first block per submatrix (-1: not on that route)
+    const double *q2fac = nullptr;
     std::vector<int64_t> q2blk;
 };
 
