@@ -6,13 +6,16 @@
 // read and rewritten once per kBW columns by matrix-core products, and the band
 // (17 m doubles) is reduced inside one CU.
 //
-// Stage 1, per panel of kBW columns k0 .. k0 + 15 (rows from r0 = k0 + 16 on):
+// Stage 1, per panel p of kBW columns k0 .. k0 + 15 (rows from r0 = k0 + 16 on):
 //   k_band_qr    Householder QR of the panel below the band in registers;
 //                V into the matrix and the panel buffers, R into the band,
 //                the WY factor T;
-//   k_band_symm  X = A22 V from the lower triangle;
-//   k_band_w     W = X T - V (T^T (V^T X) T) / 2;
-//   then A22 -= [W V] [V W]^T (lower triangle) by the batched GEMM.
+//   k_band_step  the previous panel's update A22 -= V W^T + W V^T (lower
+//                triangle) and X = A22 V with the updated tiles, in one pass
+//                over the matrix;
+//   k_band_x     X summed from the tiles' parts;
+//   k_band_w     W = X T - V (T^T (V^T X) T) / 2, and this panel's update on the
+//                16 columns that the next panel factors.
 // The reflector of column c has its unit at row c + kBW.
 //
 // Stage 2 (k_chase): sweep s removes column s outside the tridiagonal with a
@@ -41,7 +44,8 @@ constexpr int kABL = kBW + 1;    // doubles per column of the band buffer
 // One submatrix of the band route (largest first).
 struct BandSub {
     int64_t off;   // matrix block in the arena
-    int64_t pw;    // panel buffers: [W V W] (ld x 48), V and X by rows (ld x 16 each), T (256)
+    int64_t pw;    // panel buffers by rows (ld x 16 each): V of even and odd panels, W, X; T (256)
+    int64_t px;    // parts of X: a 64 x 16 block per tile, then one per unit of k_band_step
     int64_t ab;    // band: column c at ab + 17 c, element d below the diagonal at + d
     int64_t blk;   // first block of its Q2 reflectors
     int m, ld, mapoff, ng;  // ng sweep groups
@@ -203,9 +207,8 @@ __global__ __launch_bounds__(NT, R == 4 ? 2 : 4) void k_band_qr(const BandSub *_
     column(std::integral_constant<int, 12>{}), column(std::integral_constant<int, 13>{});
     column(std::integral_constant<int, 14>{}), column(std::integral_constant<int, 15>{});
     __syncthreads();
-    double *pw = PW + d.pw;
-    double *vr = pw + (int64_t)48 * d.ld;
-    double *T = vr + (int64_t)32 * d.ld;
+    double *vr = PW + d.pw + (int64_t)(panel & 1) * 16 * d.ld;
+    double *T = PW + d.pw + (int64_t)64 * d.ld;
     // R into the band, T (wavefront 0; lane i holds row i)
     if (threadIdx.x < kBW) {
         const int i = threadIdx.x;
@@ -238,10 +241,7 @@ __global__ __launch_bounds__(NT, R == 4 ? 2 : 4) void k_band_qr(const BandSub *_
         for (int l = 0; l < kBW; ++l) {
             const double v = l >= nref ? 0.0 : i > l ? x[q][l] : i == l ? 1.0 : 0.0;
             x[q][l] = v;
-            if (i < n) {
-                if (l < nref) a[(unsigned)(l * d.ld) + (unsigned)i] = v;
-                pw[(unsigned)((kBW + l) * d.ld) + (unsigned)(r0 + i)] = v;
-            }
+            if (i < n && l < nref) a[(unsigned)(l * d.ld) + (unsigned)i] = v;
         }
         // by rows, zero up to the next multiple of 16 rows
         if (i < ((n + 15) & ~15)) {
@@ -255,99 +255,262 @@ __global__ __launch_bounds__(NT, R == 4 ? 2 : 4) void k_band_qr(const BandSub *_
     }
 }
 
-// X = A22 V (rows r0 .., V by rows): one wavefront per 16 rows, straight from
-// memory to v_mfma_f64_16x16x4 operands (no LDS, no barrier): the rows' part
-// left of the diagonal tile, the diagonal tile, and the part below it
-// transposed.  Every element of the lower triangle is read twice, once as row
-// and once as column; bound by that traffic.  A workgroup's four wavefronts
-// take 64 consecutive rows; a submatrix's workgroups run on one XCD.
-__global__ __launch_bounds__(256) void k_band_symm(const BandSub *__restrict__ subs, int nsub,
-                                                   const double *__restrict__ Aa,
-                                                   double *__restrict__ PW, int panel, int nblk) {
+// Units of k_band_step: strip i (64 rows) in chunks of kChunk 64-column tiles.
+// Strips 4 a .. 4 a + 3 have a + 1 chunks each.
+constexpr int kChunk = 4;
+__host__ __device__ inline int band_units(int ns) {  // of ns strips
+    const int a = ns / kChunk;
+    return 2 * a * (a + 1) + (ns - kChunk * a) * (a + 1);
+}
+__device__ inline int band_unit(int i, int q) { return band_units(i) + q; }
+
+// One pass over the lower triangle of the trailing matrix (rows and columns from
+// r0 = 16 (panel + 1) on): the previous panel's update (not for the first
+// panel) and the parts of X = A22 V of this panel.  A 256-thread workgroup takes
+// a strip of 64 rows and up to four 64 x 64 tiles of it, each wavefront 16 columns
+// of a tile.  A tile is loaded with a lane per row (coalesced), which is both the
+// result layout of v_mfma_f64_16x16x4 for A^T and its operand layout for A V, so
+// it is updated, stored and multiplied from the same registers; A^T V takes it
+// transposed through the wavefront's own LDS (no barrier).  Tile (i, j) gives rows
+// of strip i (summed over the unit's tiles) and of strip j, both to the part
+// buffers, summed by k_band_x in a fixed order.  Bound by HBM: the triangle is read
+// and written once, and parts of a quarter of it written and read (1.3e11 bytes at
+// 4.0 TB/s on the 512-water box), instead of three reads and a write: 38.8 ms per
+// build with k_band_x, against 47.0 for separate product and update kernels (39.7
+// against 42.6 on 256 molecules), and no host tables.  134 VGPRs and 42 KB of LDS
+// hold three workgroups per CU; with the next tile's loads in flight the kernel
+// spills (72 ms).  grid: 8 XCDs x (submatrices of an XCD x units); a submatrix's
+// units run on one XCD.
+template <bool UPD>
+__global__ __launch_bounds__(256, 3) void k_band_step(const BandSub *__restrict__ subs, int nsub,
+                                                      double *__restrict__ Aa,
+                                                      const double *__restrict__ PW,
+                                                      double *__restrict__ PXa, int panel, int nunit) {
     const unsigned lin = blockIdx.x, slot = lin >> 3;
-    const int si = (int)((slot / (unsigned)nblk) * 8 + (lin & 7));
+    const int si = (int)((slot / (unsigned)nunit) * 8 + (lin & 7));
     if (si >= nsub) return;
     const BandSub d = subs[si];
     const int r0 = panel * kBW + kBW;
     const int n = d.m - r0;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PTB_WAVE);
-    const int R0 = (int)(slot % (unsigned)nblk) * 64 + wave * 16;
-    if (n < 2 || R0 >= n) return;
-    const int lane = threadIdx.x % PTB_WAVE, lr = lane & 15, g = lane >> 4;
-    const unsigned ld = (unsigned)d.ld;
-    const double *a = Aa + d.off + (int64_t)r0 * d.ld + r0;
-    double *vr = PW + d.pw + (int64_t)48 * d.ld;
-    double *xr = vr + (int64_t)16 * d.ld;
-    const double *v = vr + (int64_t)r0 * kBW;
-    d4_t acc = d4_t{0.0, 0.0, 0.0, 0.0}, acc2 = acc;
-    // rows: A(R0 + i, k), k < R0 (slices of 4 columns); rows past the end
-    // clamped (their results are not used)
+    if (n < 2) return;
+    const int ns = (n + 63) / 64;
+    const int unit = (int)(slot % (unsigned)nunit);
+    if (unit >= band_units(ns)) return;
+    int i = 0, q = 0;
     {
-        const double *ar = a + (unsigned)min(R0 + lr, n - 1) + (unsigned)g * ld;
-        const double *vk = v + (unsigned)g * kBW + lr;
-        for (int k = 0; k < R0; k += 16) {
-            double av[4], bv[4];
+        int a = 0;
+        while (2 * (a + 1) * (a + 2) <= unit) ++a;
+        const int rem = unit - 2 * a * (a + 1);
+        i = kChunk * a + rem / (a + 1);
+        q = rem % (a + 1);
+    }
+    constexpr int LR = 66, LT = 34;
+    __shared__ double vs[16][LR], ws_[16][LR], vn[64][16];
+    __shared__ double tbuf[4][16][LT];
+    const int lane = threadIdx.x % PTB_WAVE, lr = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PTB_WAVE);
+    const unsigned ld = (unsigned)d.ld;
+    double *a = Aa + d.off + (int64_t)r0 * d.ld + r0;
+    const double *pw = PW + d.pw + (int64_t)r0 * kBW;
+    const double *vprev = pw + (int64_t)((panel + 1) & 1) * 16 * d.ld;
+    const double *vcur = pw + (int64_t)(panel & 1) * 16 * d.ld;
+    const double *wprev = pw + (int64_t)32 * d.ld;
+    double *px = PXa + d.px;
+    const int rb = 64 * i;
+    {
+        // the strip's rows of V and W (previous panel, by columns) and of this V
+        const int row = threadIdx.x >> 2, c = (threadIdx.x & 3) * 4;
+        const bool in = rb + row < n;
+        const unsigned at = (unsigned)min(rb + row, n - 1) * kBW + c;
+        const d4_t z = *reinterpret_cast<const d4_t *>(vcur + at);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) vn[row][c + u] = in ? z[u] : 0.0;
+        if (UPD) {
+            const d4_t x = *reinterpret_cast<const d4_t *>(vprev + at);
+            const d4_t y = *reinterpret_cast<const d4_t *>(wprev + at);
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
-                av[u] = ar[(unsigned)(4 * u) * ld];
-                bv[u] = vk[4 * u * kBW];
+                vs[c + u][row] = in ? x[u] : 0.0;
+                ws_[c + u][row] = in ? y[u] : 0.0;
             }
-            ar += 16u * ld;
-            vk += 16 * kBW;
-            acc = __builtin_amdgcn_mfma_f64_16x16x4f64(av[0], bv[0], acc, 0, 0, 0);
-            acc2 = __builtin_amdgcn_mfma_f64_16x16x4f64(av[1], bv[1], acc2, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f64_16x16x4f64(av[2], bv[2], acc, 0, 0, 0);
-            acc2 = __builtin_amdgcn_mfma_f64_16x16x4f64(av[3], bv[3], acc2, 0, 0, 0);
         }
     }
-    // the diagonal tile, from its lower triangle
+    __syncthreads();
+    d4_t xi[4];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-        const int i = R0 + lr, k = R0 + 4 * u + g;
-        const int hi = min(max(i, k), n - 1), lo = min(min(i, k), n - 1);
-        const double x = a[(unsigned)lo * ld + (unsigned)hi];
-        const double av = (i < n && k < n) ? x : 0.0;
-        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(av, v[(unsigned)k * kBW + lr], acc, 0, 0, 0);
+    for (int b = 0; b < 4; ++b) xi[b] = d4_t{0.0, 0.0, 0.0, 0.0};
+    // one tile's 16 columns: A^T by row blocks, and the operands of its columns
+    struct Tile {
+        d4_t t[4];
+        double wc[4], vc[4], vb[4];
+    };
+    const int j0 = kChunk * q;
+    // 32-bit byte offsets from uniform bases: one register per address
+    auto at = [](auto *base, unsigned bytes) {
+        return reinterpret_cast<decltype(base)>(reinterpret_cast<uintptr_t>(base) + bytes);
+    };
+    unsigned ro[4];  // the lane's rows, clamped
+#pragma unroll
+    for (int b = 0; b < 4; ++b) ro[b] = 8u * (unsigned)min(rb + 16 * b + lr, n - 1);
+    auto load = [&](int j, Tile &x) {
+        const int cb = 64 * j + 16 * wave;
+        const unsigned cl = 8u * ((unsigned)min(cb + lr, n - 1) * kBW + g);
+        const unsigned cv = 8u * ((unsigned)(cb + g) * kBW + lr);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const unsigned co = 8u * (unsigned)min(cb + 4 * r + g, n - 1) * ld;
+#pragma unroll
+            for (int b = 0; b < 4; ++b) x.t[b][r] = *at(a, co + ro[b]);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            if (UPD) {
+                x.wc[u] = *at(wprev, cl + 32 * u);
+                x.vc[u] = *at(vprev, cl + 32 * u);
+            }
+            x.vb[u] = *at(vcur, cv + 512 * u);  // zero past n
+        }
+    };
+    int zero = 0;
+    const int jl = min(j0 + kChunk - 1, i);
+    for (int j = j0; j <= jl && 64 * j + 16 * wave < n; ++j) {
+        asm volatile("" : "+v"(zero));  // (keeps the strip's operands in LDS)
+        Tile x;
+        load(j, x);
+        const int cb = 64 * j + 16 * wave;
+        const bool diag = j == i, edge = diag || rb + 64 > n;  // cut by the diagonal or the last row
+        if (UPD) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const double w = -x.wc[u], v = -x.vc[u];
+#pragma unroll
+                for (int b = 0; b < 4; ++b)
+                    x.t[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(w, vs[4 * u + g][16 * b + lr + zero], x.t[b], 0, 0, 0);
+#pragma unroll
+                for (int b = 0; b < 4; ++b)
+                    x.t[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(v, ws_[4 * u + g][16 * b + lr + zero], x.t[b], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);  // (else every operand is read ahead, and registers spill)
+            }
+        }
+        const unsigned so = 8u * ((unsigned)(cb + g) * ld + (unsigned)(rb + lr)), ld32 = 32u * ld;
+        d4_t xj = d4_t{0.0, 0.0, 0.0, 0.0}, xk = xj;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {  // 32 rows at a time through LDS
+            double e[2][4];
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    e[b][r] = x.t[2 * h + b][r];
+                    tbuf[wave][4 * r + g][16 * b + lr] = e[b][r];
+                }
+            if (edge) {
+#pragma unroll
+                for (int b = 0; b < 2; ++b)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int row = rb + 16 * (2 * h + b) + lr + zero, col = cb + 4 * r + g;
+                        const bool on = row < n && col < n && (!diag || row >= col);
+                        if (UPD && on) *at(a, so + r * ld32 + 128u * (2 * h + b)) = e[b][r];
+                        e[b][r] = on ? e[b][r] : 0.0;
+                        tbuf[wave][4 * r + g][16 * b + lr] = diag && row == col ? 0.0 : e[b][r];
+                    }
+            } else if (UPD) {
+#pragma unroll
+                for (int b = 0; b < 2; ++b)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) *at(a, so + r * ld32 + 128u * (2 * h + b)) = e[b][r];
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int b = 0; b < 2; ++b)
+                    xi[2 * h + b] = __builtin_amdgcn_mfma_f64_16x16x4f64(e[b][r], x.vb[r], xi[2 * h + b], 0, 0, 0);
+#pragma unroll
+            for (int u = 0; u < 8; u += 2) {
+                xj = __builtin_amdgcn_mfma_f64_16x16x4f64(tbuf[wave][lr][4 * u + g], vn[32 * h + 4 * u + g][lr + zero],
+                                                          xj, 0, 0, 0);
+                xk = __builtin_amdgcn_mfma_f64_16x16x4f64(tbuf[wave][lr][4 * u + 4 + g],
+                                                          vn[32 * h + 4 * u + 4 + g][lr + zero], xk, 0, 0, 0);
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        double *p = px + (int64_t)(i * (i + 1) / 2 + j) * 1024 + (16 * wave + g) * 16 + lr;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) p[64 * r] = xj[r] + xk[r];
     }
-    // columns: A(k, R0 + i), k >= R0 + 16, 16 rows at a time, lane group g
-    // holding rows 4 g .. 4 g + 3 (slice u: k = 4 g + u in both operands)
-    if (R0 + 16 < n) {
-        const double *ac = a + (unsigned)(R0 + lr) * ld;
-        for (int k = R0 + 16; k < n; k += 16) {
-            const d2_t *p = reinterpret_cast<const d2_t *>(ac + k + 4 * g);
-            const d2_t p0 = p[0], p1 = p[1];
-            const double *vk = v + (unsigned)(k + 4 * g) * kBW + lr;
-            double av[4] = {p0[0], p0[1], p1[0], p1[1]}, bv[4];
+    // the strip's own rows: the wavefronts' parts in fixed order, 32 rows at a time
+    double *xs = &tbuf[0][0][0];  // [wave][32 x 16]
+    const int ns0 = (d.m - kBW + 63) / 64;
+    double *o = px + (int64_t)(ns0 * (ns0 + 1) / 2 + unit) * 1024;
 #pragma unroll
-            for (int u = 0; u < 4; ++u) bv[u] = vk[u * kBW];
-            if (k + 16 > n)
+    for (int h = 0; h < 2; ++h) {
+        __syncthreads();
 #pragma unroll
-                for (int u = 0; u < 4; ++u) av[u] = k + 4 * g + u < n ? av[u] : 0.0;
-            acc = __builtin_amdgcn_mfma_f64_16x16x4f64(av[0], bv[0], acc, 0, 0, 0);
-            acc2 = __builtin_amdgcn_mfma_f64_16x16x4f64(av[1], bv[1], acc2, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f64_16x16x4f64(av[2], bv[2], acc, 0, 0, 0);
-            acc2 = __builtin_amdgcn_mfma_f64_16x16x4f64(av[3], bv[3], acc2, 0, 0, 0);
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) xs[wave * 512 + (16 * b + 4 * r + g) * 16 + lr] = xi[2 * h + b][r];
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const int l = threadIdx.x + 256 * e;
+            o[512 * h + l] = ((xs[l] + xs[512 + l]) + xs[1024 + l]) + xs[1536 + l];
         }
     }
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-        xr[(unsigned)(r0 + R0 + 4 * r + g) * kBW + lr] = acc[r] + acc2[r];
 }
 
-// W = X T - V S, S = T^T (V^T X) T / 2, by columns into the panel buffer
-// (columns 0 .. 15 and 32 .. 47).  One workgroup per submatrix: V^T X on the
-// matrix cores (wavefronts on alternate 16-row tiles), the 16 x 16 products in
-// LDS, then W^T tile by tile.
+// X (by rows) of one 64-row strip from its parts: the strip's own chunks, then
+// the tiles below it in its columns, in order.  grid: (submatrix, strip)
+__global__ __launch_bounds__(256) void k_band_x(const BandSub *__restrict__ subs,
+                                                const double *__restrict__ PXa, double *__restrict__ PW,
+                                                int panel) {
+    const BandSub d = subs[blockIdx.x];
+    const int r0 = panel * kBW + kBW;
+    const int n = d.m - r0, i = blockIdx.y;
+    if (n < 2 || 64 * i >= n) return;
+    const int ns = (n + 63) / 64, ns0 = (d.m - kBW + 63) / 64;
+    const double *px = PXa + d.px;
+    const double *own = px + (int64_t)(ns0 * (ns0 + 1) / 2 + band_unit(i, 0)) * 1024;
+    const int nq = i / kChunk + 1;
+    double *x = PW + d.pw + (int64_t)48 * d.ld + (int64_t)(r0 + 64 * i) * kBW;
+    const int rows = min(64, ((n + 15) & ~15) - 64 * i);
+    double s[4] = {0.0, 0.0, 0.0, 0.0};
+    for (int q = 0; q < nq; ++q)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[e] += own[(int64_t)q * 1024 + threadIdx.x + 256 * e];
+#pragma unroll 4
+    for (int j = i; j < ns; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            s[e] += px[(int64_t)(j * (j + 1) / 2 + i) * 1024 + threadIdx.x + 256 * e];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int l = threadIdx.x + 256 * e;
+        if (l < 16 * rows) x[l] = 64 * i + (l >> 4) < n ? s[e] : 0.0;
+    }
+}
+
+// W = X T - V S, S = T^T (V^T X) T / 2, by rows, and the panel's update
+// A -= V W^T + W V^T on the next 16 columns (rows and columns from r0 on), which
+// the next panel's QR reads.  One workgroup per submatrix: V^T X on the matrix
+// cores (wavefronts on alternate 16-row tiles), the 16 x 16 products in LDS, then
+// W^T and the columns tile by tile (lane = row; W^T's result layout is the operand
+// layout of the update).
 __global__ __launch_bounds__(256) void k_band_w(const BandSub *__restrict__ subs,
-                                                double *__restrict__ PW, int panel) {
+                                                double *__restrict__ Aa, double *__restrict__ PW,
+                                                int panel) {
     const BandSub d = subs[blockIdx.x];
     const int r0 = panel * kBW + kBW;
     const int n = d.m - r0;
     if (n < 2) return;
     double *pw = PW + d.pw;
-    const double *vr = pw + (int64_t)48 * d.ld + (int64_t)r0 * kBW;
-    const double *xr = vr + (int64_t)16 * d.ld;
-    const double *T = pw + (int64_t)80 * d.ld;
+    const double *vr = pw + (int64_t)(panel & 1) * 16 * d.ld + (int64_t)r0 * kBW;
+    double *wr = pw + (int64_t)32 * d.ld + (int64_t)r0 * kBW;
+    const double *xr = pw + (int64_t)48 * d.ld + (int64_t)r0 * kBW;
+    const double *T = pw + (int64_t)64 * d.ld;
+    double *a = Aa + d.off + (int64_t)r0 * d.ld + r0;
     __shared__ double gs[4][16][17], ts[16][17], ms[16][17], ss[16][17];
     const int lane = threadIdx.x % PTB_WAVE, wave = threadIdx.x / PTB_WAVE;
     const int lr = lane & 15, g = lane >> 4;
@@ -367,10 +530,7 @@ __global__ __launch_bounds__(256) void k_band_w(const BandSub *__restrict__ subs
     const int ti = threadIdx.x & 15, tj = threadIdx.x >> 4;
     ts[ti][tj] = T[tj * kBW + ti];
     __syncthreads();
-    {
-        const double s = ((gs[0][ti][tj] + gs[1][ti][tj]) + gs[2][ti][tj]) + gs[3][ti][tj];
-        ss[ti][tj] = s;
-    }
+    ss[ti][tj] = ((gs[0][ti][tj] + gs[1][ti][tj]) + gs[2][ti][tj]) + gs[3][ti][tj];
     __syncthreads();
     {
         double s = 0.0;  // M = G T
@@ -393,8 +553,8 @@ __global__ __launch_bounds__(256) void k_band_w(const BandSub *__restrict__ subs
         ta[u] = ts[4 * u + g][lr];
         sa[u] = -ss[4 * u + g][lr];
     }
-    for (int k = 16 * wave; k < n; k += 64) {
-        double xb[4], vb[4];
+    auto make_w = [&](int k, double (&vb)[4]) {
+        double xb[4];
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             xb[u] = xr[(unsigned)(k + lr) * kBW + 4 * u + g];
@@ -406,13 +566,37 @@ __global__ __launch_bounds__(256) void k_band_w(const BandSub *__restrict__ subs
             w = __builtin_amdgcn_mfma_f64_16x16x4f64(ta[u], xb[u], w, 0, 0, 0);
             w = __builtin_amdgcn_mfma_f64_16x16x4f64(sa[u], vb[u], w, 0, 0, 0);
         }
-        if (k + lr < n)
+        return w;
+    };
+    // rows r0 .. r0 + 15 of V and W, the update's column operands
+    double v0[4];
+    const d4_t w0 = make_w(0, v0);
+    for (int k = 16 * wave; k < n; k += 64) {
+        const int row = k + lr;
+        d4_t t;
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            t[r] = a[(unsigned)min(4 * r + g, n - 1) * (unsigned)d.ld + (unsigned)min(row, n - 1)];
+        double vb[4];
+        const d4_t w = make_w(k, vb);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            t = __builtin_amdgcn_mfma_f64_16x16x4f64(-w0[u], vb[u], t, 0, 0, 0);
+            t = __builtin_amdgcn_mfma_f64_16x16x4f64(-v0[u], w[u], t, 0, 0, 0);
+        }
+        if (row < n)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                double *o = pw + (unsigned)((4 * r + g) * d.ld) + (unsigned)(r0 + k + lr);
-                o[0] = w[r];
-                o[(unsigned)(32 * d.ld)] = w[r];
+                wr[(unsigned)row * kBW + 4 * r + g] = w[r];
+                if (4 * r + g <= row) a[(unsigned)(4 * r + g) * (unsigned)d.ld + (unsigned)row] = t[r];
             }
+        if (n == kBW + 1 && k == kBW) {  // no next panel: the last diagonal element
+            double s = 0.0;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) s += vb[u] * w[u];
+            s = rows_sum(s);
+            if (lane == 0) a[(unsigned)kBW * (unsigned)d.ld + kBW] -= 2.0 * s;
+        }
     }
 }
 
@@ -931,6 +1115,11 @@ int64_t band_blocks(int m) {
     return ng * (ng + 1) / 2;
 }
 
+int64_t band_parts(int m) {
+    const int64_t ns = m > kBW ? (m - kBW + 63) / 64 : 0;
+    return 1024 * (ns * (ns + 1) / 2 + band_units((int)ns));
+}
+
 int sytrd_band(ptbgpu_ctx *ctx, const std::vector<SubDesc> &desc, double *A, double *d, double *e,
                double *tau, QFactor &qf) {
     const int nsm = (int)desc.size();
@@ -943,21 +1132,23 @@ int sytrd_band(ptbgpu_ctx *ctx, const std::vector<SubDesc> &desc, double *A, dou
     if (nb == 0) return PTBGPU_OK;
     std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return desc[a].m > desc[b].m; });
     std::vector<BandSub> subs(nb);
-    int64_t pw = 0, ab = 0, blk = 0;
+    int64_t pw = 0, px = 0, ab = 0, blk = 0;
     for (int i = 0; i < nb; ++i) {
         const SubDesc &x = desc[order[i]];
-        subs[i] = {x.off, pw, ab, blk, x.m, x.ld, x.mapoff, q2_groups(x.m)};
+        subs[i] = {x.off, pw, px, ab, blk, x.m, x.ld, x.mapoff, q2_groups(x.m)};
         qf.q2blk[order[i]] = blk;
-        pw += (int64_t)x.ld * 80 + 256;
+        pw += (int64_t)x.ld * 64 + 256;
+        px += band_parts(x.m);
         ab += ((int64_t)x.m * kABL + 15) & ~15;
         blk += band_blocks(x.m);
     }
     auto *PW = static_cast<double *>(ws(ctx, "band_pw", sizeof(double) * pw));
+    auto *PX = static_cast<double *>(ws(ctx, "band_px", sizeof(double) * std::max<int64_t>(px, 1)));
     auto *AB = static_cast<double *>(ws(ctx, "band_ab", sizeof(double) * ab));
     auto *raw = static_cast<double *>(ws(ctx, "band_q2raw", sizeof(double) * 256 * std::max<int64_t>(blk, 1)));
     auto *rtau = static_cast<double *>(ws(ctx, "band_q2tau", sizeof(double) * 16 * std::max<int64_t>(blk, 1)));
     auto *fac = static_cast<double *>(ws(ctx, "band_q2fac", sizeof(double) * 1024 * std::max<int64_t>(blk, 1)));
-    if (!PW || !AB || !raw || !rtau || !fac) return PTBGPU_E_NOMEM;
+    if (!PW || !PX || !AB || !raw || !rtau || !fac) return PTBGPU_E_NOMEM;
     auto *ds = static_cast<BandSub *>(upload_table(ctx, "band_subs", subs.data(), sizeof(BandSub) * nb));
     if (!ds) return PTBGPU_E_NOMEM;
     qf.q2fac = fac;
@@ -970,31 +1161,10 @@ int sytrd_band(ptbgpu_ctx *ctx, const std::vector<SubDesc> &desc, double *A, dou
     };
     // panels: at least two rows below the band
     const int npanel = max_m >= kBW + 2 ? (max_m - kBW - 2) / kBW + 1 : 0;
-    std::vector<GemmDesc> g;
-    std::vector<int> start(npanel + 1, 0);
-    for (int p = 0; p < npanel; ++p) {
-        start[p] = (int)g.size();
-        const int r0 = (p + 1) * kBW, na = count(r0 + 2);
-        for (int i = 0; i < na; ++i) {
-            const BandSub &x = subs[i];
-            double *w = PW + x.pw + r0, *C = A + x.off + (int64_t)r0 * x.ld + r0;
-            g.push_back({w, w + (int64_t)kBW * x.ld, C, x.m - r0, x.m - r0, 2 * kBW, x.ld, x.ld, x.ld,
-                         -1.0, 1.0, 1, 0});
-        }
-    }
-    start[npanel] = (int)g.size();
-    GemmDesc *dg = nullptr;
-    TileList tl;
-    if (npanel > 0) {
-        dg = static_cast<GemmDesc *>(upload_table(ctx, "band_g", g.data(), sizeof(GemmDesc) * g.size()));
-        if (!dg) return PTBGPU_E_NOMEM;
-        for (int p = 0; p < npanel; ++p) tl.add(g.data() + start[p], start[p + 1] - start[p]);
-        PTB_TRY(tl.upload(ctx, "band_w"));
-    }
     {
         ProfScope prof_(ctx, "band_reduce");
         for (int p = 0; p < npanel; ++p) {
-            const int r0 = (p + 1) * kBW, na = start[p + 1] - start[p];
+            const int r0 = (p + 1) * kBW, na = count(r0 + 2);
             const int n = max_m - r0;  // the tallest panel
             {
                 ProfScope kprof_(ctx, "band_qr");
@@ -1010,19 +1180,27 @@ int sytrd_band(ptbgpu_ctx *ctx, const std::vector<SubDesc> &desc, double *A, dou
                     hipLaunchKernelGGL((k_band_qr<256, 1>), dim3(na - big), dim3(256), 0, st, ds, A, PW, AB, tau, big, p);
                 PTB_CHECK_LAUNCH(ctx);
             }
+            const int ns = (n + 63) / 64;
             {
-                ProfScope kprof_(ctx, "band_symm");
-                const int nblk = (n + 63) / 64;
-                hipLaunchKernelGGL(k_band_symm, dim3((unsigned)((na + 7) / 8 * 8 * nblk)), dim3(256), 0, st,
-                                   ds, na, A, PW, p, nblk);
+                ProfScope kprof_(ctx, "band_step");
+                const int nunit = band_units(ns);
+                const dim3 grid((unsigned)((na + 7) / 8 * 8 * nunit));
+                if (p == 0)
+                    hipLaunchKernelGGL(k_band_step<false>, grid, dim3(256), 0, st, ds, na, A, PW, PX, p, nunit);
+                else
+                    hipLaunchKernelGGL(k_band_step<true>, grid, dim3(256), 0, st, ds, na, A, PW, PX, p, nunit);
+                PTB_CHECK_LAUNCH(ctx);
+            }
+            {
+                ProfScope kprof_(ctx, "band_x");
+                hipLaunchKernelGGL(k_band_x, dim3(na, ns), dim3(256), 0, st, ds, PX, PW, p);
                 PTB_CHECK_LAUNCH(ctx);
             }
             {
                 ProfScope kprof_(ctx, "band_w");
-                hipLaunchKernelGGL(k_band_w, dim3(na), dim3(256), 0, st, ds, PW, p);
+                hipLaunchKernelGGL(k_band_w, dim3(na), dim3(256), 0, st, ds, A, PW, p);
                 PTB_CHECK_LAUNCH(ctx);
             }
-            PTB_TRY(tl.launch(ctx, p, false, true, dg + start[p], "sytrd"));
         }
         hipLaunchKernelGGL(k_band_extract, dim3(nb, (max_m + kBW - 1) / kBW), dim3(256), 0, st, ds, A, AB,
                            kQBlk);

@@ -377,7 +377,7 @@ int refine_occupied(ptbgpu_ctx *ctx, const std::vector<SubDesc> &desc, const Sub
 const char *const kChunkBufs[] = {"sm_A",      "sm_B",       "sm_Z",  "sm_W",   "sm_X",
                                   "sm_Li",     "sm_K32",     "sm_V",  "sm_R",   "sm_xa",
                                   "sm_f",      "sytrd_pw",   "sytrd_pw32", "q_T", "q_T64",
-                                  "q_T128",    "q_t128_gm", "band_pw",   "band_ab",
+                                  "q_T128",    "q_t128_gm", "band_pw",   "band_px", "band_ab",
                                   "band_q2raw", "band_q2tau", "band_q2fac"};
 
 // Device bytes the per-submatrix arenas of one chunk may take: the free
@@ -640,7 +640,8 @@ int sm_density_batch_device(ptbgpu_ctx *ctx, const std::vector<MolIn> &mols, int
                              2 * sizeof(double) * (size_t)desc[s].ld * 2 * (desc[s].gend - desc[s].gbeg) +
                              sizeof(double) * (size_t)desc[s].ld * (96 + 32 + 64 + 128) +
                              (desc[s].flags & kSubBand
-                                  ? sizeof(double) * (256 + 16 + 1024) * (size_t)ptb::band_blocks(desc[s].m)
+                                  ? sizeof(double) * ((256 + 16 + 1024) * (size_t)ptb::band_blocks(desc[s].m) +
+                                                      (size_t)ptb::band_parts(desc[s].m))
                                   : 0);
             if (used > 0 && used + c > budget) {
                 cb.push_back(s);

@@ -230,6 +230,8 @@ int apply_q(ptbgpu_ctx *ctx, const std::vector<SubDesc> &desc, const QFactor &qf
 // band.hip
 // blocks of chase reflectors of one submatrix of m rows
 int64_t band_blocks(int m);
+// doubles of part sums its band reduction takes
+int64_t band_parts(int m);
 // FP64 tridiagonalisation of the submatrices flagged kSubBand (lower triangle
 // of A): d and e, the reflectors and tau of the band reduction in A, and the
 // chase's in qf
