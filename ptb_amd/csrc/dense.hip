@@ -2,8 +2,8 @@
 //
 // * k_gemm:     C = alpha op(A) op(B) + beta C for a variable-size batch whose
 //               shapes and pointers come from device descriptors (so a kernel
-//               earlier in the stream can size the next product).  64x64 (or
-//               128x128) output tile per workgroup, 16-deep k slices staged in
+//               earlier in the stream can size the next product).  64x64 (32x32,
+//               128x128) output tile per workgroup, k slices staged in
 //               LDS with the next slice prefetched into registers.
 // * k_potrf_panel: one 32-column panel of the lower Cholesky S = L L^T: the
 //               diagonal block factored and inverted in LDS, the panel below as
@@ -32,7 +32,7 @@ typedef double d4_t __attribute__((ext_vector_type(4)));
 template <typename T>
 using gmem = __attribute__((address_space(1))) T;
 
-// TE x TE output tile per 256-thread workgroup (TE = 64 or 128); each
+// TE x TE output tile per 256-thread workgroup (TE = 32, 64 or 128); each
 // wavefront owns a TE/2 x TE/2 quarter as (TE/32)^2 blocks of
 // v_mfma_f64_16x16x4.  MFMA operand layout: lane l supplies A(l%16, l/16) of
 // a 16x4 slice and B(l/16, l%16) of a 4x16 slice; result value r of lane l is
@@ -53,12 +53,13 @@ constexpr int kKS = 32;  // k depth up to which a product counts as one slice (k
 
 template <int TE>
 struct GemmTileShape {
-    static constexpr int KS = 16;         // k slice
+    static constexpr int KS = TE == 32 ? 64 : 16;  // k slice
     static constexpr int NL = TE * KS / 256;  // elements of A (and of B) per thread per slice
     static constexpr int BW = TE / 32;    // 16 x 16 blocks along a wavefront's quarter
     static constexpr int LD = TE + 4;     // row stride of the LDS slices
     static constexpr int CLD = TE + 1;    // column stride of the epilogue's LDS columns
     static constexpr int CW = 32;         // columns of the tile per epilogue pass
+    static constexpr int RW = TE < 64 ? TE : 64;  // rows of a column per wavefront instruction
     static constexpr int SMEM = 2 * KS * LD > CW * CLD ? 2 * KS * LD : CW * CLD;
 };
 
@@ -76,7 +77,7 @@ struct GemmTileShape {
 // With a tile list (work != nullptr) workgroup b computes the tile work[b],
 // already dealt to XCDs by the host; the grid is the list's length.
 template <bool TA, bool TB, typename T, int TE>
-__global__ __attribute__((amdgpu_flat_work_group_size(1, kT), amdgpu_waves_per_eu(TE == 64 ? 5 : 2)))
+__global__ __attribute__((amdgpu_flat_work_group_size(1, kT), amdgpu_waves_per_eu(TE == 64 ? 5 : TE == 32 ? 3 : 2)))
 void k_gemm(const GemmDesc *__restrict__ descs, int count, int tiles,
             const GemmTile *__restrict__ work) {
     using S = GemmTileShape<TE>;
@@ -108,7 +109,8 @@ void k_gemm(const GemmDesc *__restrict__ descs, int count, int tiles,
         if (tile >= tM * tN) return;
         m0 = (tile % max(tM, 1)) * TE;
         n0 = (tile / max(tM, 1)) * TE;
-        if (descs[gi].uplo && n0 > m0 + TE - 1) return;  // tile strictly above the diagonal
+        const int up = descs[gi].uplo;  // tile strictly above the diagonal
+        if (up && (TE == 32 && up == 2 ? (n0 >> 6) > (m0 >> 6) : n0 > m0 + TE - 1)) return;
     }
     const GemmDesc g = descs[gi];
     // (a list may hold tiles of a bound on a shape the device fills in)
@@ -231,16 +233,18 @@ void k_gemm(const GemmDesc *__restrict__ descs, int count, int tiles,
                     Ct[(wn - CW * h + 16 * j + lr) * CLD + wm + 16 * i + 4 * r + lk] = acc[i][j][r];
         }
         __syncthreads();
-        for (int cc = wave; cc < CW; cc += kT / 64) {
+        constexpr int RW = S::RW, NC = 64 / RW;  // NC columns per instruction
+        const int row = lane & (RW - 1);
+        for (int cc = NC * wave + lane / RW; cc < CW; cc += NC * (kT / 64)) {
             const int gn = n0 + CW * h + cc;
 #pragma unroll
-            for (int rr = 0; rr < TE; rr += 64) {
-                const int gm = m0 + rr + lane;
+            for (int rr = 0; rr < TE; rr += RW) {
+                const int gm = m0 + rr + row;
                 if (gm >= g.M || gn >= g.N || (g.uplo == 1 && gm < gn) ||
                     (g.uplo == 2 && (gm >> 6) < (gn >> 6)))
                     continue;
                 auto *c = gC + (int64_t)gn * g.ldc + gm;
-                const double v = Ct[cc * CLD + rr + lane];
+                const double v = Ct[cc * CLD + rr + row];
                 const T r = (T)(g.beta == 0.0 ? g.alpha * v : g.alpha * v + g.beta * (double)*c);
                 *c = r;
                 if (g.C32) ((gmem<float> *)(void *)g.C32)[(int64_t)gn * g.ldc + gm] = (float)r;
@@ -978,7 +982,7 @@ static void launch_gemm_te(ptbgpu_ctx *ctx, bool ta, bool tb, dim3 grid, const G
     else hipLaunchKernelGGL((k_gemm<true, true, double, TE>), grid, dim3(kT), 0, ctx->stream, ddesc, count, tiles, work);
 }
 
-// edge: 64 or 128 (double storage only)
+// edge: 64, or 32 or 128 (double storage only); the brackets count 32 with 64
 static int launch_gemm(ptbgpu_ctx *ctx, bool ta, bool tb, bool f32, dim3 grid, const GemmDesc *ddesc,
                        int count, int tiles, const GemmTile *work, int edge) {
     ProfScope eprof_(ctx, edge == 128 ? "gemm_tile128" : "gemm_tile64");
@@ -988,6 +992,8 @@ static int launch_gemm(ptbgpu_ctx *ctx, bool ta, bool tb, bool f32, dim3 grid, c
         hipLaunchKernelGGL((k_gemm<false, true, float, 64>), grid, dim3(kT), 0, ctx->stream, ddesc, count, tiles, work);
     } else if (edge == 128) {
         launch_gemm_te<128>(ctx, ta, tb, grid, ddesc, count, tiles, work);
+    } else if (edge == 32) {
+        launch_gemm_te<32>(ctx, ta, tb, grid, ddesc, count, tiles, work);
     } else {
         launch_gemm_te<64>(ctx, ta, tb, grid, ddesc, count, tiles, work);
     }
@@ -995,8 +1001,8 @@ static int launch_gemm(ptbgpu_ctx *ctx, bool ta, bool tb, bool f32, dim3 grid, c
     return PTBGPU_OK;
 }
 
-// Tile edge of an FP64 launch of `count` products from its 128 x 128 tile
-// count and the multiply-adds its tiles issue at both edges (padded output
+constexpr int64_t kSmallTiles = 2;
+// Tile edge of an FP64 launch of `count` products from its tile counts and the multiply-adds its tiles issue at both edges (padded output
 // times the k range of each tile): the gemm_tile knob forces 64 or 128; else
 // 128 x 128 tiles only for launches of fewer products than XCDs (single large
 // products, spread over the chip) with at least 4 such tiles per CU and at
@@ -1004,9 +1010,15 @@ static int launch_gemm(ptbgpu_ctx *ctx, bool ta, bool tb, bool f32, dim3 grid, c
 // one 4096^3 product against 50; on the batches of ragged, partly triangular
 // submatrix products (m about 100 to 1000) their coarser padding costs more
 // than the halved operand traffic saves, so those stay at 64.
-static int gemm_edge(int64_t mode, int num_cus, int count, int64_t tiles128, double work64,
-                     double work128) {
+// 32 x 32 tiles for launches of at most kSmallTiles 64 x 64 tiles per CU: with one
+// 64 x 64 tile per CU every SIMD holds one wavefront, which waits for each slice
+// in turn, and most CUs may hold none.  A 621^3 product (100 such tiles) takes
+// 25.5 us with 400 small tiles of 64-deep slices against 45.6, the 1472-row dense
+// solve's products of 128 rows (k up to 1472) 16.8 us against 39.
+static int gemm_edge(int64_t mode, int num_cus, int count, int64_t tiles64, int64_t tiles128,
+                     double work64, double work128) {
     if (mode == 64 || mode == 128) return (int)mode;
+    if (tiles64 <= kSmallTiles * (int64_t)std::max(num_cus, 1)) return 32;
     return count < 8 && tiles128 >= 4 * (int64_t)std::max(num_cus, 1) && work128 <= 1.03 * work64
                ? 128
                : 64;
@@ -1043,7 +1055,7 @@ int gemm_vbatch(ptbgpu_ctx *ctx, bool ta, bool tb, const GemmDesc *ddesc, int co
     auto tiles_at = [&](int te) { return (int64_t)((max_m + te - 1) / te) * ((max_n + te - 1) / te); };
     // (the k extent and triangles are on the device: padded outputs only)
     const int edge = f32 ? 64
-                         : gemm_edge(ctx->gemm_tile, ctx->num_cus, count, count * tiles_at(128),
+                         : gemm_edge(ctx->gemm_tile, ctx->num_cus, count, count * tiles_at(64), count * tiles_at(128),
                                      4096.0 * tiles_at(64), 16384.0 * tiles_at(128));
     const int64_t tiles = tiles_at(edge);
     // fewer products than XCDs: each product's tiles over the whole chip
@@ -1064,7 +1076,7 @@ int gemm_tiles(ptbgpu_ctx *ctx, bool ta, bool tb, const GemmDesc *ddesc, const G
     ProfScope prof_(ctx, "gemm");
     ProfScope sprof_(ctx, site ? (std::string("gemm_") + site).c_str() : "gemm_other");
     if (nwork <= 0) return PTBGPU_OK;
-    if (edge != 64 && (edge != 128 || f32 || lowp != kLowpNone))
+    if (edge != 64 && ((edge != 128 && edge != 32) || f32 || lowp != kLowpNone))
         return fail(ctx, PTBGPU_E_ARG, "GEMM tile edge %d is for FP64 products on double storage", edge);
     if (lowp != kLowpNone) {
         ProfScope lprof_(ctx, lowp == kLowpBF16 ? "gemm_bf16" : "gemm_bf16x3");
@@ -1081,6 +1093,11 @@ int gemm_tiles(ptbgpu_ctx *ctx, bool ta, bool tb, const GemmDesc *ddesc, const G
     return launch_gemm(ctx, ta, tb, f32, grid, ddesc, 0, 1, dwork, edge);
 }
 
+// first tile row of tile column tn that holds output
+static int first_tile(int te, int uplo, int tn) {
+    return uplo == 0 ? 0 : te == 32 && uplo == 2 ? tn & ~1 : tn;
+}
+
 int TileList::add(const GemmDesc *h, int count, bool fp64) {
     sig_.push_back(count);
     sig_.push_back(fp64 ? 1 : 0);
@@ -1092,7 +1109,7 @@ int TileList::add(const GemmDesc *h, int count, bool fp64) {
 }
 
 // Every launch: the tile edge (128 for an FP64 launch where gemm_edge says
-// so, else 64); products largest first (longest-processing-time order), each
+// so, 32 for small launches, else 64); products largest first (longest-processing-time order), each
 // dealt whole to the XCD with the fewest tiles so far (in a launch of fewer
 // products than XCDs, a product larger than an XCD's even share in runs of
 // tiles instead); entry 8 k + x of the launch's block is XCD x's k-th tile
@@ -1113,13 +1130,16 @@ void TileList::build(std::vector<GemmTile> &work, int64_t tile_mode, int num_cus
             const int64_t tM = (M + te - 1) / te, tN = (N + te - 1) / te;
             if (!sh[5 * i + 3]) return tM * tN;
             const int64_t c = std::min(tM, tN);  // columns tn < c hold tM - tn tiles
-            return c * tM - c * (c - 1) / 2;
+            // (uplo = 2 writes 64-wide diagonal blocks whole: at edge 32 the tile
+            // above an odd column's diagonal too)
+            return c * tM - c * (c - 1) / 2 + (te == 32 && sh[5 * i + 3] == 2 ? c / 2 : 0);
         };
         bool one = true;
-        int64_t t128 = 0;
+        int64_t t64 = 0, t128 = 0;
         for (int i = 0; i < count; ++i) {
             if (tiles_of(i, 64) == 0) continue;
             one = one && sh[5 * i + 2] <= kKS && sh[5 * i + 4] == 0;
+            t64 += tiles_of(i, 64);
             t128 += tiles_of(i, 128);
         }
         int te = 64;
@@ -1131,7 +1151,7 @@ void TileList::build(std::vector<GemmTile> &work, int64_t tile_mode, int num_cus
                     w64 += tile_work(d[0], d[1], d[2], d[3], d[4], 64);
                     w128 += tile_work(d[0], d[1], d[2], d[3], d[4], 128);
                 }
-            te = gemm_edge(tile_mode, num_cus, count, t128, w64, w128);
+            te = gemm_edge(tile_mode, num_cus, count, t64, t128, w64, w128);
         }
         std::vector<int> ord(count);
         std::vector<int64_t> area(count);
@@ -1156,7 +1176,7 @@ void TileList::build(std::vector<GemmTile> &work, int64_t tile_mode, int num_cus
             int64_t k = 0;
             int x = 0;
             for (int tn = 0; tn < tN; ++tn)
-                for (int tm = sh[5 * i + 3] ? tn : 0; tm < tM; ++tm, ++k) {
+                for (int tm = first_tile(te, sh[5 * i + 3], tn); tm < tM; ++tm, ++k) {
                     if (k % run == 0) {
                         x = 0;
                         for (int y = 1; y < 8; ++y)
@@ -1172,7 +1192,7 @@ void TileList::build(std::vector<GemmTile> &work, int64_t tile_mode, int num_cus
         for (int x = 0; x < 8; ++x)
             for (size_t k = 0; k < q[x].size(); ++k) work[base + 8 * k + x] = q[x][k];
         start_.push_back((int64_t)work.size());
-        flags_.push_back((char)((one ? kOne : 0) | (te == 128 ? kEdge128 : 0)));
+        flags_.push_back((char)((one ? kOne : 0) | (te == 128 ? kEdge128 : te == 32 ? kEdge32 : 0)));
     }
 }
 
@@ -1234,7 +1254,7 @@ int TileList::launch(ptbgpu_ctx *ctx, int i, bool ta, bool tb, const GemmDesc *d
     if (n == 0) return PTBGPU_OK;
     if (!dwork_) return fail(ctx, PTBGPU_E_ARG, "GEMM tile list launched before upload");
     return gemm_tiles(ctx, ta, tb, ddesc, dwork_ + start_[i], n, site, f32, (flags_[i] & kOne) != 0,
-                      lowp, (flags_[i] & kEdge128) ? 128 : 64);
+                      lowp, (flags_[i] & kEdge128) ? 128 : (flags_[i] & kEdge32) ? 32 : 64);
 }
 
 // X = L^-1 B (trans=false) or L^-T B (trans=true), all m columns, blocked by

@@ -191,6 +191,7 @@ class TileList {
     void build(std::vector<GemmTile> &work, int64_t tile_mode, int num_cus);
     static constexpr char kOne = 1;       // every product is one k slice (K <= 32, no tri)
     static constexpr char kEdge128 = 2;   // 128 x 128 tiles
+    static constexpr char kEdge32 = 4;    // 32 x 32 tiles
     std::vector<int> sig_;        // per launch: count, fp64, then M, N, K, uplo, tri per product
     int nlaunch_ = 0;
     std::vector<int64_t> start_;  // per launch: first entry in the table (+ the total)

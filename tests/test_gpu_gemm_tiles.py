@@ -187,3 +187,42 @@ def test_chip_wide_merges_identical(engine, precision):
     finally:
         engine.set_tuning("dc_global_min", saved)
     assert np.array_equal(Ps[0], Ps[64])
+
+
+@pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True), (True, True)])
+@pytest.mark.parametrize("m,n,k", [(1, 1, 1), (31, 33, 63), (32, 32, 64), (33, 65, 65), (95, 97, 129),
+                                   (64, 1, 200), (621, 130, 621)])
+def test_small_launch_tiles_identical(engine, m, n, k, ta, tb):
+    """A launch of few 64 x 64 tiles runs on 32 x 32 ones (knob 0): the same
+    bits as with 64 x 64 tiles, and the FP64 bound against torch."""
+    import torch
+    gen = np.random.default_rng(m + 7 * n + 31 * k)
+    A = _mat(k, m, gen) if ta else _mat(m, k, gen)
+    B = _mat(n, k, gen) if tb else _mat(k, n, gen)
+    C0 = _mat(m, n, gen)
+    a, b = (A if ta else A.t()), (B if tb else B.t())
+    out = {}
+    for edge in (0, 64):
+        C = C0.clone()
+        with _tile(engine, edge):
+            engine.gemm_batch_dev("fp64", ta, tb, [A], [B], [C], -1.25, 0.5)
+        torch.cuda.synchronize()
+        out[edge] = C
+    assert torch.equal(out[0], out[64])
+    scale = 1.25 * (a.abs() @ b.abs()) + 0.5 * C0.t().abs()
+    err = ((out[0].t() - (-1.25 * (a @ b) + 0.5 * C0.t())).abs() / scale.clamp_min(1e-300)).max().item()
+    assert err <= 1e-13
+
+
+@pytest.mark.parametrize("kind,size,cols", [("water", (2, 2, 2), 3), ("water", (2, 1, 1), 2), ("alkane", 8, 3)])
+def test_small_builds_identical(engine, kind, size, cols):
+    """Triangular factors and lower-triangle products of small builds (32 x 32
+    tiles at knob 0): the same density bits as with 64 x 64 tiles."""
+    mol, H, S = small_system(kind, size, 3)
+    out = {}
+    for edge in (0, 64):
+        P = np.zeros_like(H)
+        with _tile(engine, edge):
+            engine.sm_stupid_simple(mol.ndim, mol.nel, H, S, P, mol.n, mol.xyz, mol.aoat, cols, 2)
+        out[edge] = P
+    assert np.array_equal(out[0], out[64])
