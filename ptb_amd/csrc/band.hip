@@ -74,6 +74,28 @@ __device__ __forceinline__ double row_sum(double v) {
     v = dpp_add<0x141>(v);
     return dpp_add<0x140>(v);
 }
+template <int CTRL>
+__device__ __forceinline__ double dpp_mov(double v) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+// sums over the 16 lanes of a row of four values, times a, in every lane: two
+// halving exchanges (quad_perm 1032, 2301) leave one value per lane, summed over
+// the quads by rotations of 8 and 4 lanes and broadcast within each quad
+__device__ __forceinline__ void row_sum4(const double (&p)[4], double a, int i, double (&z)[4]) {
+    const bool b0 = i & 1, b1 = i & 2;
+    const double h0 = (b0 ? p[2] : p[0]) + dpp_mov<0xB1>(b0 ? p[0] : p[2]);
+    const double h1 = (b0 ? p[3] : p[1]) + dpp_mov<0xB1>(b0 ? p[1] : p[3]);
+    double v = (b1 ? h1 : h0) + dpp_mov<0x4E>(b1 ? h0 : h1);
+    v = dpp_add<0x128>(v);
+    v = dpp_add<0x124>(v) * a;
+    z[0] = dpp_mov<0x00>(v);
+    z[1] = dpp_mov<0xAA>(v);
+    z[2] = dpp_mov<0x55>(v);
+    z[3] = dpp_mov<0xFF>(v);
+}
 // sum over the four 16-lane rows, in every lane
 __device__ __forceinline__ double rows_sum(double v) {
     {
@@ -119,6 +141,25 @@ __device__ __forceinline__ Reflector reflector(double alpha, double sigma) {
     if (sigma == 0.0) return {alpha, 0.0, 0.0};
     const double beta = -copysign(sqrt(alpha * alpha + sigma), alpha);
     return {beta, (beta - alpha) / beta, 1.0 / (alpha - beta)};
+}
+// The same for the chase, where it is on the serial chain of every step: the norm
+// and its reciprocal from one hardware estimate of 1 / sqrt (coupled Newton
+// steps), the scale from one of 1 / x, each refined to rounding level.
+__device__ __forceinline__ Reflector reflector_fast(double alpha, double sigma) {
+    if (sigma == 0.0) return {alpha, 0.0, 0.0};
+    const double n2 = alpha * alpha + sigma, y = __builtin_amdgcn_rsq(n2);
+    double g = n2 * y, h = 0.5 * y;
+    double e = fma(-h, g, 0.5);
+    g = fma(g, e, g), h = fma(h, e, h);
+    e = fma(-h, g, 0.5);
+    g = fma(g, e, g), h = fma(h, e, h);
+    g = fma(fma(-g, g, n2), h, g);  // sqrt(n2), 2 h its reciprocal
+    h = fma(h, fma(-2.0 * h, g, 1.0), h);
+    const double q = fabs(alpha) + g;
+    double r = __builtin_amdgcn_rcp(q);
+    r = fma(r, fma(-q, r, 1.0), r);
+    r = fma(r, fma(-q, r, 1.0), r);
+    return {-copysign(g, alpha), fma(2.0 * h, fabs(alpha), 1.0), copysign(r, alpha)};
 }
 
 // ---- stage 1 ------------------------------------------------------------------
@@ -662,21 +703,26 @@ __device__ __forceinline__ void chase_step(double (&D)[4], double (&B)[4], int k
             B[c] = cc ? bcol : rf ? 0.0 : B[c];
         }
     }
+    const bool pivot = i == f;
+    // where the reflectors of this step go (those the sweep has)
+    const bool last = s >= m - 2;
+    const unsigned ro = (unsigned)((i - f) & 15);
+    const int64_t blk = q2_block(ng, s >> 4, k);
     if (k == 0) {
         // the sweep's first reflector: column s below its diagonal
         const double dia = L.cm[fo];
         const double x = i == fo ? L.bm[0] : L.cm[i];
-        const Reflector h = reflector(read_lane(x, f), row_sum(i == f ? 0.0 : x * x));
-        const double u = i == f ? 1.0 : x * h.scale;
+        const Reflector h = reflector_fast(read_lane(x, f), row_sum(pivot ? 0.0 : x * x));
+        const double u = pivot ? 1.0 : x * h.scale;
         if (g == 0) {
             L.vm[i] = u;
-            if (s < m - 2) raw[q2_block(ng, s >> 4, 0) * 256 + (s & 15) * 16 + ((i - f) & 15)] = u;
+            if (!last) (raw + blk * 256 + (s & 15) * 16)[ro] = u;
         }
         if (lane == 0) {
             L.tm[0] = h.tau;
             dv[s] = dia;
             ev[s] = s < m - 1 ? h.beta : 0.0;
-            if (s < m - 2) rtau[q2_block(ng, s >> 4, 0) * 16 + (s & 15)] = h.tau;
+            if (!last) rtau[blk * 16 + (s & 15)] = h.tau;
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     }
@@ -684,6 +730,9 @@ __device__ __forceinline__ void chase_step(double (&D)[4], double (&B)[4], int k
     double vc[4];
 #pragma unroll
     for (int c = 0; c < 4; ++c) vc[c] = L.vm[k * 16 + 4 * g + c];
+    const int gf = f >> 2, cf = f & 3;
+    const double b0 = cf & 1 ? B[1] : B[0], b1 = cf & 1 ? B[3] : B[2];
+    // p = D v, y = B v and B's first column, by rows
     double p = D[0] * vc[0], y = B[0] * vc[0];
 #pragma unroll
     for (int c = 1; c < 4; ++c) {
@@ -692,22 +741,27 @@ __device__ __forceinline__ void chase_step(double (&D)[4], double (&B)[4], int k
     }
     p = tau * rows_sum(p);
     y = tau * rows_sum(y);
-    const double w = p - (0.5 * tau * row_sum(p * vr)) * vr;
+    // (v is 1 at the pivot, so the column after B <- B H is x = B(:, f) - y)
+    const double x = rows_sum(g == gf ? (cf & 2 ? b1 : b0) : 0.0) - y;
+    const double pv = row_sum(p * vr), sig = row_sum(pivot ? 0.0 : x * x);
+    const double w = p - (0.5 * tau * pv) * vr;
     if (g == 0) L.wsc[i] = w;
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    // B <- B H, then the reflector of its first column
-#pragma unroll
-    for (int c = 0; c < 4; ++c) B[c] -= y * vc[c];
-    const int gf = f >> 2, cf = f & 3;
-    const double b0 = cf & 1 ? B[1] : B[0], b1 = cf & 1 ? B[3] : B[2];
-    const double x = rows_sum(g == gf ? (cf & 2 ? b1 : b0) : 0.0);
-    const Reflector h = reflector(read_lane(x, f), row_sum(i == f ? 0.0 : x * x));
-    const double u = i == f ? 1.0 : x * h.scale;
+    const Reflector h = reflector_fast(read_lane(x, f), sig);
+    const double u = pivot ? 1.0 : x * h.scale;
+    // B <- H' B H, its first column beta e
+    double q[4], z[4];
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
-        const double z = h.tau * row_sum(u * B[c]);
-        const double t = B[c] - u * z;
-        B[c] = 4 * g + c == f ? (i == f ? h.beta : 0.0) : t;
+        B[c] -= y * vc[c];
+        q[c] = u * B[c];
+    }
+    row_sum4(q, h.tau, i, z);
+    const double xf = pivot ? h.beta : 0.0;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        const double t = B[c] - u * z[c];
+        B[c] = 4 * g + c == f ? xf : t;
     }
     // D <- H D H
 #pragma unroll
@@ -716,42 +770,42 @@ __device__ __forceinline__ void chase_step(double (&D)[4], double (&B)[4], int k
         D[c] -= vr * wc;
         D[c] -= w * vc[c];
     }
+    const bool next = !last && s + 1 + 16 * (k + 1) <= m - 2;
     if (g == 0) {
         L.vm[(k + 1) * 16 + i] = u;
-        if (s < m - 2 && s + 1 + 16 * (k + 1) <= m - 2)
-            raw[q2_block(ng, s >> 4, k + 1) * 256 + (s & 15) * 16 + ((i - f) & 15)] = u;
+        if (next) (raw + (blk + 1) * 256 + (s & 15) * 16)[ro] = u;
     }
     if (lane == 0) {
         L.tm[k + 1] = h.tau;
         L.bm[k] = h.beta;
-        if (s < m - 2 && s + 1 + 16 * (k + 1) <= m - 2)
-            rtau[q2_block(ng, s >> 4, k + 1) * 16 + (s & 15)] = h.tau;
+        if (next) rtau[(blk + 1) * 16 + (s & 15)] = h.tau;
     }
-    if (g == gf) {
-        const double d0 = cf & 1 ? D[1] : D[0], d1 = cf & 1 ? D[3] : D[2];
-        L.cm[k * 16 + i] = cf & 2 ? d1 : d0;
-    }
-    if (i == f)
+    // the first rows of D (its first column, D being symmetric) and of B
+    if (pivot)
 #pragma unroll
-        for (int c = 0; c < 4; ++c) L.rm[k * 16 + 4 * g + c] = B[c];
+        for (int c = 0; c < 4; ++c) {
+            L.cm[k * 16 + 4 * g + c] = D[c];
+            L.rm[k * 16 + 4 * g + c] = B[c];
+        }
 }
 
-// Bulge chasing of one submatrix per workgroup of NW wavefronts.  Step (s, k)
+// Bulge chasing of one submatrix by a workgroup of NW wavefronts.  Step (s, k)
 // needs (s, k - 1) and (s - 1, k + 1), so at time t = 2 s + k all windows of one
 // parity step at once; a barrier ends each time step.  Wavefront w owns the
 // windows 2 w and 2 w + 1 (mod 2 NW), so the work stays even as the band
-// shortens.  MEM false: the windows live in registers (P per wavefront, 16 VGPRs
-// each), up to 16 NW P rows; MEM true: in device memory (state), for larger m.
+// shortens, and ends when they have left it.  P windows per wavefront live in
+// registers (16 VGPRs each), up to 16 NW P rows; MEM: those above that in device
+// memory (state), which they need for the first sweeps only.
+// Bound by instruction issue of the CU (about 390 vector instructions a step; with
+// IEEE square root and divisions, and one row sum per column of B, it was 430).
+// One window of each parity per wavefront where 16 hold them: a step's chain is the
+// time step.  512-water box 21.6 -> 17.3 ms, 256 molecules 46.4 -> 32.0, one
+// 1472-row matrix (every window in memory before) 14.0 -> 11.7.
 template <int NW, int P, bool MEM>
-__global__ __launch_bounds__(NW * 64) void k_chase(const BandSub *__restrict__ subs, int first,
-                                                   const double *__restrict__ ABa,
-                                                   double *__restrict__ raw_all,
-                                                   double *__restrict__ rtau_all,
-                                                   double *__restrict__ d_all,
-                                                   double *__restrict__ e_all,
-                                                   double *__restrict__ state) {
-    extern __shared__ double sm[];
-    const BandSub b = subs[first + blockIdx.x];
+__device__ __forceinline__ void chase(const BandSub &b, double *sm, const double *__restrict__ ABa,
+                                      double *__restrict__ raw_all, double *__restrict__ rtau_all,
+                                      double *__restrict__ d_all, double *__restrict__ e_all,
+                                      double *__restrict__ state) {
     const int m = b.m;
     const int K = max((m - 1 + kBW - 1) / kBW, 1);  // windows
     const int lane = threadIdx.x % PTB_WAVE;
@@ -775,7 +829,6 @@ __global__ __launch_bounds__(NW * 64) void k_chase(const BandSub *__restrict__ s
     }
     double *raw = raw_all + b.blk * 256, *rtau = rtau_all + b.blk * 16;
     double *dv = d_all + b.mapoff, *ev = e_all + b.mapoff;
-    double *st = MEM ? state + b.pw : nullptr;  // (the panel buffers are free by now)
     const int i = lane & 15, g = lane >> 4;
     auto load_window = [&](int k, double (&D)[4], double (&B)[4]) {
         const int r = 1 + 16 * k + ((i - 1) & 15);
@@ -788,50 +841,73 @@ __global__ __launch_bounds__(NW * 64) void k_chase(const BandSub *__restrict__ s
         }
     };
     auto active = [&](int k, int s) { return s >= 0 && s < m && (k == 0 || s + 1 + 16 * k < m); };
-    const int T2 = m - 1;  // every step (s, k) has s + k / 2 <= m - 1
-    if constexpr (!MEM) {
-        double D[P][4], B[P][4];
+    // (the panel buffers are free by now)
+    auto stored = [&](int k) {
+        return reinterpret_cast<d4_t *>(state + b.pw) + ((int64_t)k * 64 + lane) * 2;
+    };
+    double D[P][4], B[P][4];
 #pragma unroll
-        for (int q = 0; q < P; ++q) {
-            const int k = 2 * wave + 2 * NW * (q / 2) + (q & 1);
-            load_window(k, D[q], B[q]);
+    for (int q = 0; q < P; ++q) load_window(2 * wave + 2 * NW * (q / 2) + (q & 1), D[q], B[q]);
+    if constexpr (MEM)
+        for (int k = 2 * wave + P * NW; k < K; k = k & 1 ? k + 2 * NW - 1 : k + 1) {
+            double Dk[4], Bk[4];
+            load_window(k, Dk, Bk);
+            stored(k)[0] = d4_t{Dk[0], Dk[1], Dk[2], Dk[3]};
+            stored(k)[1] = d4_t{Bk[0], Bk[1], Bk[2], Bk[3]};
         }
-        __syncthreads();
-        for (int t = 0; t <= T2; ++t) {
+    __syncthreads();
+    if (2 * wave >= K) return;
+    // the last step of window 2 w: sweep m - 1 of window 0, else s + 1 + 32 w = m - 1
+    const int T2 = wave == 0 ? m - 1 : m - 2 - 31 * wave;
+    for (int t = 0; t <= T2; ++t) {
 #pragma unroll
-            for (int par = 0; par < 2; ++par) {
+        for (int par = 0; par < 2; ++par) {
 #pragma unroll
-                for (int q = par; q < P; q += 2) {
-                    const int k = 2 * wave + 2 * NW * (q / 2) + par, s = t - wave - NW * (q / 2);
-                    if (active(k, s)) chase_step(D[q], B[q], k, s, m, b.ng, L, raw, rtau, dv, ev, lane);
-                }
-                __syncthreads();
+            for (int q = par; q < P; q += 2) {
+                const int k = 2 * wave + 2 * NW * (q / 2) + par, s = t - wave - NW * (q / 2);
+                if (active(k, s)) chase_step(D[q], B[q], k, s, m, b.ng, L, raw, rtau, dv, ev, lane);
             }
-        }
-    } else {
-        for (int k = wave; k < K; k += NW) {
-            double D[4], B[4];
-            load_window(k, D, B);
-            d4_t *p = reinterpret_cast<d4_t *>(st) + ((int64_t)k * 64 + lane) * 2;
-            p[0] = d4_t{D[0], D[1], D[2], D[3]};
-            p[1] = d4_t{B[0], B[1], B[2], B[3]};
-        }
-        __syncthreads();
-        for (int t = 0; t <= T2; ++t)
-            for (int par = 0; par < 2; ++par) {
-                for (int j = 0; 2 * wave + par + 2 * NW * j < K; ++j) {
+            if constexpr (MEM)
+                for (int j = P / 2; 2 * wave + par + 2 * NW * j < K; ++j) {
                     const int k = 2 * wave + par + 2 * NW * j, s = t - wave - NW * j;
-                    if (!active(k, s)) continue;
-                    d4_t *p = reinterpret_cast<d4_t *>(st) + ((int64_t)k * 64 + lane) * 2;
-                    const d4_t p0 = p[0], p1 = p[1];
-                    double D[4] = {p0[0], p0[1], p0[2], p0[3]}, B[4] = {p1[0], p1[1], p1[2], p1[3]};
-                    chase_step(D, B, k, s, m, b.ng, L, raw, rtau, dv, ev, lane);
-                    p[0] = d4_t{D[0], D[1], D[2], D[3]};
-                    p[1] = d4_t{B[0], B[1], B[2], B[3]};
+                    if (!active(k, s)) break;  // (nor are the windows above)
+                    const d4_t p0 = stored(k)[0], p1 = stored(k)[1];
+                    double Dk[4] = {p0[0], p0[1], p0[2], p0[3]}, Bk[4] = {p1[0], p1[1], p1[2], p1[3]};
+                    chase_step(Dk, Bk, k, s, m, b.ng, L, raw, rtau, dv, ev, lane);
+                    stored(k)[0] = d4_t{Dk[0], Dk[1], Dk[2], Dk[3]};
+                    stored(k)[1] = d4_t{Bk[0], Bk[1], Bk[2], Bk[3]};
                 }
-                __syncthreads();
-            }
+            __syncthreads();
+        }
     }
+}
+
+template <int NW, int P, bool MEM>
+__global__ __launch_bounds__(NW * 64) void k_chase(const BandSub *__restrict__ subs, int first,
+                                                   const double *__restrict__ ABa,
+                                                   double *__restrict__ raw_all,
+                                                   double *__restrict__ rtau_all,
+                                                   double *__restrict__ d_all,
+                                                   double *__restrict__ e_all,
+                                                   double *__restrict__ state) {
+    extern __shared__ double sm[];
+    const BandSub b = subs[first + blockIdx.x];
+    chase<NW, P, MEM>(b, sm, ABa, raw_all, rtau_all, d_all, e_all, state);
+}
+
+// All submatrices of a small batch (a CU each) in one launch, 16 wavefronts each:
+// the size classes overlap (192 submatrices of 64 waters: 5.3 ms one class after
+// the other, 3.4 so); a larger batch fills the chip with each class.
+__global__ __launch_bounds__(1024) void k_chase_few(const BandSub *__restrict__ subs,
+                                                    const double *__restrict__ ABa,
+                                                    double *__restrict__ raw_all,
+                                                    double *__restrict__ rtau_all,
+                                                    double *__restrict__ d_all,
+                                                    double *__restrict__ e_all) {
+    extern __shared__ double sm[];
+    const BandSub b = subs[blockIdx.x];
+    if (b.m > 513) chase<16, 4, false>(b, sm, ABa, raw_all, rtau_all, d_all, e_all, nullptr);
+    else chase<16, 2, false>(b, sm, ABa, raw_all, rtau_all, d_all, e_all, nullptr);
 }
 
 // ---- application of Q2 ---------------------------------------------------------
@@ -1225,11 +1301,19 @@ int sytrd_band(ptbgpu_ctx *ctx, const std::vector<SubDesc> &desc, double *A, dou
         }                                                                                             \
     } while (0)
         PTB_CHASE(16, 2, true, 1026);
-        PTB_CHASE(16, 4, false, 514);
-        PTB_CHASE(8, 4, false, 258);
-        PTB_CHASE(4, 4, false, 130);
-        PTB_CHASE(4, 2, false, 66);
-        PTB_CHASE(2, 2, false, 0);
+        if (nb - done <= ctx->num_cus) {
+            if (nb > done) {
+                hipLaunchKernelGGL(k_chase_few, dim3(nb - done), dim3(1024), lds(subs[done].m, 16), st,
+                                   ds + done, AB, raw, rtau, d, e);
+                PTB_CHECK_LAUNCH(ctx);
+            }
+        } else {
+            PTB_CHASE(16, 4, false, 514);
+            PTB_CHASE(16, 2, false, 258);
+            PTB_CHASE(8, 2, false, 130);
+            PTB_CHASE(4, 2, false, 66);
+            PTB_CHASE(2, 2, false, 0);
+        }
 #undef PTB_CHASE
     }
     if (blk > 0) {

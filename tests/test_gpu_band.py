@@ -64,3 +64,23 @@ def test_build_through_every_size_class(engine, cols):
     rep = engine.sm_stupid_simple(mol.ndim, mol.nel, H, S, P, mol.n, mol.xyz, mol.aoat, cols, 2)
     assert np.abs(P - ref.P).max() < 1e-8
     assert rep["mu"] == ref.mu and rep["muiter"] == ref.muiter
+
+
+@pytest.mark.parametrize("n", [1472, 2047, 2048])
+def test_windows_in_memory(engine, n):
+    """Above 1025 rows part of the chase's windows live in memory: the first
+    sizes with two and three of them per wavefront, and the largest."""
+    _check(engine, _matrix(n, "dense"))
+
+
+def test_more_submatrices_than_compute_units(engine):
+    """Single-column submatrices of 27 waters (621 of several size classes, a
+    launch per class) against the oracle."""
+    from conftest import small_system
+    from oracle import ptb_oracle as O
+    mol, H, S = small_system("water", (3, 3, 3), 4)
+    ref = O.sm_stupid_simple(mol.ndim, mol.nel, H, S, mol.n, mol.xyz, mol.aoat, 1, 2)
+    P = np.full_like(H, np.nan)
+    rep = engine.sm_stupid_simple(mol.ndim, mol.nel, H, S, P, mol.n, mol.xyz, mol.aoat, 1, 2)
+    assert np.abs(P - ref.P).max() < 1e-8
+    assert rep["mu"] == ref.mu and rep["muiter"] == ref.muiter
