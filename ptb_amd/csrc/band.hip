@@ -1006,9 +1006,11 @@ __global__ __launch_bounds__(256, 4) void k_q2_prep(const BandSub *__restrict__ 
     }
 }
 
-constexpr int kQ2Groups = 4;  // sweep groups per pass of k_q2_apply (even)
+constexpr int kQ2Groups = 4;  // sweep groups per pass of k_q2_apply, a wavefront each
 
-// A chunk of columns of one submatrix's right-hand sides.
+constexpr int64_t kQ2Wide = 2;  // 32-column jobs per CU from which they are taken (what a CU holds)
+
+// A chunk of columns of one submatrix's right-hand sides (m = 0: none).
 struct Q2Job {
     int64_t y;    // first element (row 0 of the first column)
     int64_t blk;  // the submatrix's first block
@@ -1016,7 +1018,7 @@ struct Q2Job {
 };
 
 // Y <- Q2 Y (TRANS false: groups descending, windows ascending) or Q2^T Y (the
-// reverse) for up to 16 CT columns per wavefront.  The 32 rows a block touches sit
+// reverse) for up to 16 CT columns per workgroup.  The 32 rows a block touches sit
 // in registers as two 16 x 16 tiles per 16 columns, in the layout in which
 // v_mfma_f64_16x16x4 takes its B operand and leaves its result, so nothing moves
 // between the two products of a block; the next block shares one tile.  The
@@ -1025,21 +1027,26 @@ struct Q2Job {
 // 16-byte accesses), and for reflector 4 g + r between the products, so the
 // second factor is read 32 bytes per lane.
 //
-// Q groups run in one pass over the rows, group after group one window behind
-// the previous one: a window's step applies Q blocks to Q + 1 tiles, and each tile is
-// read and written once per Q groups.  On the 512-water box (1.5e6 blocks, 126
-// columns on average) one group per pass moved 43 GB of right-hand sides beside
-// 12 GB of factors and took 24.5 ms for both applications; four take 15.7.
-// Factors are fetched two blocks ahead, tiles three windows ahead.
+// kQ2Groups groups run in one pass over the rows, a wavefront each: a wavefront
+// keeps the tile that its next block shares, hands the finished one to the next
+// wavefront through LDS (the last one stores it) and takes a new one from the
+// wavefront before (the first one loads it), one barrier per step.  So a job's
+// chain is a quarter of its blocks long and every SIMD of a CU has one of its
+// wavefronts.  Against one wavefront per job that takes the four groups in turn:
+// one 1472-row matrix, all columns, 3.57 -> 1.27 ms; both applications of 64 waters
+// 2.67 -> 1.21, C400H802 2.9 -> 0.9, 8 waters 0.23 -> 0.08, the 512-water box (whose
+// products alone fill the matrix cores for 5.5 ms) 15.0 -> 13.1.
+// Factors and the first wavefront's tiles are fetched three steps ahead.
 template <bool TRANS, int CT>
-__global__ __launch_bounds__(256, 2) void k_q2_apply(const Q2Job *__restrict__ jobs, int njobs,
+__global__ __launch_bounds__(256, 2) void k_q2_apply(const Q2Job *__restrict__ jobs,
                                                      const double *__restrict__ fac_all,
                                                      double *__restrict__ Ya) {
     typedef double d2u_t __attribute__((ext_vector_type(2), aligned(8)));
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PTB_WAVE);
-    const int ji = blockIdx.x * 4 + wave;
-    if (ji >= njobs) return;
-    const Q2Job jb = jobs[ji];
+    constexpr int Q = kQ2Groups, S = 3;
+    __shared__ d2_t hand[2][Q - 1][CT][2][PTB_WAVE];
+    const int h = __builtin_amdgcn_readfirstlane(threadIdx.x / PTB_WAVE);
+    const Q2Job jb = jobs[blockIdx.x];
+    if (jb.m == 0) return;
     const int lane = threadIdx.x % PTB_WAVE, lr = lane & 15, g = lane >> 4;
     const int m = jb.m, ng = jb.ng;
     double *y[CT];
@@ -1049,12 +1056,9 @@ __global__ __launch_bounds__(256, 2) void k_q2_apply(const Q2Job *__restrict__ j
         cok[c] = 16 * c + lr < jb.nc;
         y[c] = Ya + jb.y + (int64_t)min(16 * c + lr, jb.nc - 1) * jb.ld + 1 + 4 * g;
     }
-    // tile t: rows 16 t + 1 .. 16 t + 16, the last one cut at m (t < 0: none)
+    // tile t: rows 16 t + 1 .. 16 t + 16, cut at m
     auto load = [&](int t, d4_t (&x)[CT]) {
-        if (t < 0) {
-#pragma unroll
-            for (int c = 0; c < CT; ++c) x[c] = d4_t{0.0, 0.0, 0.0, 0.0};
-        } else if (16 * t + 17 <= m) {
+        if (16 * t + 17 <= m) {
 #pragma unroll
             for (int c = 0; c < CT; ++c) {
                 const d2u_t *p = reinterpret_cast<const d2u_t *>(y[c] + 16 * t);
@@ -1073,7 +1077,6 @@ __global__ __launch_bounds__(256, 2) void k_q2_apply(const Q2Job *__restrict__ j
         }
     };
     auto store = [&](int t, const d4_t (&x)[CT]) {
-        if (t < 0) return;
         if (16 * t + 17 <= m) {
 #pragma unroll
             for (int c = 0; c < CT; ++c)
@@ -1107,54 +1110,75 @@ __global__ __launch_bounds__(256, 2) void k_q2_apply(const Q2Job *__restrict__ j
             f.f1[4 + s] = p1[256 + 16 * s];
         }
 #pragma unroll
-        for (int h = 0; h < 2; ++h)
+        for (int q = 0; q < 2; ++q)
 #pragma unroll
             for (int s = 0; s < 2; ++s) {
-                const d2_t v = p2[128 * h + s];
-                f.f2[4 * h + 2 * s] = v[0];
-                f.f2[4 * h + 2 * s + 1] = v[1];
+                const d2_t v = p2[128 * q + s];
+                f.f2[4 * q + 2 * s] = v[0];
+                f.f2[4 * q + 2 * s + 1] = v[1];
             }
     };
-    // A pass takes the groups A, A - 1, .. A - Q + 1 (TRANS in the other order; the
-    // last pass may reach below group 0).  At step i the window is k = i (TRANS:
-    // from the top), the h-th group's block touches the tiles met at positions
-    // i + Q - 1 - h and i + Q - h, and position i is finished.  Position o lives
-    // in buffer o mod S and the steps are unrolled by S, so that every buffer is
-    // a fixed set of registers (moving one would wait for its loads); Q more
-    // steps only store.
-    constexpr int Q = kQ2Groups, S = 8;
-    Fac F[2];
-    d4_t X[S][CT];
+    Fac F[S];
+    d4_t X[S][CT];  // the first wavefront's tiles
+    d4_t keep[CT];
     const int npass = (ng + Q - 1) / Q;
     for (int pass = 0; pass < npass; ++pass) {
-        const int A = ng - 1 - Q * (TRANS ? npass - 1 - pass : pass);
-        const int n = ng - A + Q - 1;  // steps that hold blocks
-        auto tile = [&](int o) { return A - Q + 1 + (TRANS ? n + Q - 1 - o : o); };
-        auto group = [&](int h) { return TRANS ? A - Q + 1 + h : A - h; };
-        auto window = [&](int i) { return TRANS ? n - 1 - i : i; };
-        auto valid = [&](int i, int h) {
-            const int G = group(h), k = window(i);
-            return G >= 0 && k >= 0 && k < ng - G;
+        // the pass' first group; wavefront h takes the h-th one after it
+        const int A = TRANS ? Q * pass : ng - 1 - Q * pass;
+        const int nq = min(Q, TRANS ? ng - A : A + 1);
+        const bool on = h < nq;
+        const int G = !on ? 0 : TRANS ? A + h : A - h;
+        const int nb = ng - G;  // its blocks
+        // Block j of group G (window j, TRANS: from the top) is step j + lag.  It
+        // needs the tile that the wavefront before finished one step earlier: in
+        // its block j, TRANS: j + 1
+        const int lag = TRANS ? 2 * h : h;
+        const int steps = TRANS ? ng - A + nq - 1 : ng - A + 2 * nq - 1;
+        auto tile_in = [&](int j) { return TRANS ? ng - 1 - j : G + j + 1; };
+        auto get = [&](int j, Fac &f) {
+            const int jc = min(max(j, 0), nb - 1);
+            fetch(q2_block(ng, G, TRANS ? nb - 1 - jc : jc), f);
         };
-        auto get = [&](int i, int h, Fac &f) {
-            const int G = max(group(h), 0), k = min(max(window(i), 0), ng - G - 1);
-            fetch(q2_block(ng, G, k), f);
-        };
-        get(0, 0, F[0]);
-        get(0, 1, F[1]);
-        [&]<int... O>(std::integer_sequence<int, O...>) {
-            ((O < n + Q ? load(tile(O), X[O]) : (void)0), ...);
-        }(std::make_integer_sequence<int, S>{});
-        auto step = [&](auto U, int i) {
+        if (on) {
+            if (h == 0)
+                [&]<int... U>(std::integer_sequence<int, U...>) {
+                    ((U < nb ? load(tile_in(U), X[U]) : (void)0), ...);
+                }(std::make_integer_sequence<int, S>{});
+            if (!TRANS) load(G, keep);
+            else if (h == 0) load(ng, keep);
+            get(-lag, F[0]);
+            get(1 - lag, F[1]);
+            get(2 - lag, F[2]);
+        }
+        auto step = [&](auto U, int t) {
             constexpr int u = decltype(U)::value;
-            auto block = [&](auto H) {
-                constexpr int h = decltype(H)::value;
-                constexpr int o0 = (u + Q - 1 - h) % S, o1 = (u + Q - h) % S;
-                Fac &f = F[h & 1];
-                if (valid(i, h)) {
+            const int j = t - lag;
+            auto take = [&](d4_t (&x)[CT]) {
+#pragma unroll
+                for (int c = 0; c < CT; ++c) {
+                    const d2_t a = hand[(t - 1) & 1][h - 1][c][0][lane], b = hand[(t - 1) & 1][h - 1][c][1][lane];
+                    x[c] = d4_t{a[0], a[1], b[0], b[1]};
+                }
+            };
+            auto pass_on = [&](int tile, const d4_t (&x)[CT]) {
+                if (h == nq - 1) {
+                    store(tile, x);
+                    return;
+                }
+#pragma unroll
+                for (int c = 0; c < CT; ++c) {
+                    hand[t & 1][h][c][0][lane] = d2_t{x[c][0], x[c][1]};
+                    hand[t & 1][h][c][1][lane] = d2_t{x[c][2], x[c][3]};
+                }
+            };
+            if (on) {
+                if (j >= 0 && j < nb) {
+                    if (h > 0) take(X[u]);
+                    Fac &f = F[u];
+                    d4_t done[CT];
 #pragma unroll
                     for (int c = 0; c < CT; ++c) {
-                        d4_t &lo = X[TRANS ? o1 : o0][c], &hi = X[TRANS ? o0 : o1][c];
+                        d4_t &lo = TRANS ? X[u][c] : keep[c], &hi = TRANS ? keep[c] : X[u][c];
                         d4_t w = d4_t{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
                         for (int r = 0; r < 4; ++r) w = __builtin_amdgcn_mfma_f64_16x16x4f64(f.f1[r], lo[r], w, 0, 0, 0);
@@ -1165,19 +1189,24 @@ __global__ __launch_bounds__(256, 2) void k_q2_apply(const Q2Job *__restrict__ j
                             lo = __builtin_amdgcn_mfma_f64_16x16x4f64(f.f2[r], w[r], lo, 0, 0, 0);
                             hi = __builtin_amdgcn_mfma_f64_16x16x4f64(f.f2[4 + r], w[r], hi, 0, 0, 0);
                         }
+                        done[c] = keep[c];
+                        keep[c] = X[u][c];
                     }
+                    pass_on(TRANS ? ng - j : G + j, done);
+                    if (h == 0 && j + S < nb) load(tile_in(j + S), X[u]);
+                    if (TRANS && j == nb - 1) store(G, keep);
+                } else if (TRANS && j == -1) {
+                    take(keep);  // (h > 0: the top tile)
+                } else if (!TRANS && j == nb) {
+                    pass_on(ng, keep);
                 }
-                get(h + 2 < Q ? i : i + 1, (h + 2) % Q, f);
-            };
-            [&]<int... H>(std::integer_sequence<int, H...>) {
-                (block(std::integral_constant<int, H>{}), ...);
-            }(std::make_integer_sequence<int, Q>{});
-            store(tile(i), X[u]);
-            if (i + S < n + Q) load(tile(i + S), X[u]);
+                get(j + S, F[u]);
+            }
+            __syncthreads();
         };
-        for (int i = 0; i < n + Q; i += S)
+        for (int t = 0; t < steps; t += S)
             [&]<int... U>(std::integer_sequence<int, U...>) {
-                ((i + U < n + Q ? step(std::integral_constant<int, U>{}, i + U) : (void)0), ...);
+                ((t + U < steps ? step(std::integral_constant<int, U>{}, t + U) : (void)0), ...);
             }(std::make_integer_sequence<int, S>{});
     }
 }
@@ -1331,37 +1360,49 @@ int apply_q2(ptbgpu_ctx *ctx, const std::vector<SubDesc> &desc, const QFactor &q
              const char *tag) {
     if (!qf.q2fac) return PTBGPU_OK;
     ProfScope prof_(ctx, "apply_q2");
-    // two 16-column tiles per wavefront (each factor feeds both) where that leaves
-    // a wavefront for every SIMD, else one; one for a last piece of at most 16, and
-    // for Q2^T (few columns; two tiles would spill registers there)
+    // two 16-column tiles per workgroup (each factor feeds both) where that leaves
+    // kQ2Wide workgroups per CU, else one; one for a last piece of at most 16
     int64_t pairs = 0;
     for (int s = 0; s < (int)desc.size(); ++s)
         if (qf.q2blk[s] >= 0) pairs += (ncols[s] + 31) / 32;
-    const int step = !trans && pairs >= 4 * (int64_t)ctx->num_cus ? 32 : 16;
-    std::vector<Q2Job> wide, narrow;
-    for (int s = 0; s < (int)desc.size(); ++s) {
-        const SubDesc &x = desc[s];
-        if (qf.q2blk[s] < 0 || x.m < 3) continue;
-        for (int c = 0; c < ncols[s]; c += step) {
-            const int nc = std::min(step, ncols[s] - c);
-            (nc > 16 ? wide : narrow)
-                .push_back({yoff[s] + (int64_t)c * x.ld, qf.q2blk[s], x.m, x.ld, q2_groups(x.m), nc});
+    const int step = pairs >= kQ2Wide * (int64_t)ctx->num_cus ? 32 : 16;
+    std::vector<int> order;
+    for (int s = 0; s < (int)desc.size(); ++s)
+        if (qf.q2blk[s] >= 0 && desc[s].m >= 3 && ncols[s] > 0) order.push_back(s);
+    std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return desc[a].m > desc[b].m; });
+    // largest submatrices first, each one's jobs on one XCD (whose L2 holds its
+    // factors): entry 8 k + x is XCD x's k-th job
+    auto run = [&](const char *nm, bool two) -> int {
+        std::vector<Q2Job> q[8];
+        for (int s : order) {
+            const SubDesc &x = desc[s];
+            int to = 0;
+            for (int i = 1; i < 8; ++i)
+                if (q[i].size() < q[to].size()) to = i;
+            for (int c = 0; c < ncols[s]; c += step) {
+                const int nc = std::min(step, ncols[s] - c);
+                if ((nc > 16) != two) continue;
+                q[order.size() < 8 ? (c / step) & 7 : to].push_back(
+                    {yoff[s] + (int64_t)c * x.ld, qf.q2blk[s], x.m, x.ld, q2_groups(x.m), nc});
+            }
         }
-    }
-    auto run = [&](std::vector<Q2Job> &jobs, const char *nm, bool two) -> int {
-        if (jobs.empty()) return PTBGPU_OK;
-        std::stable_sort(jobs.begin(), jobs.end(), [](const Q2Job &a, const Q2Job &b) { return a.m > b.m; });
+        size_t len = 0;
+        for (const auto &l : q) len = std::max(len, l.size());
+        if (len == 0) return PTBGPU_OK;
+        std::vector<Q2Job> jobs(8 * len, Q2Job{});
+        for (int x = 0; x < 8; ++x)
+            for (size_t k = 0; k < q[x].size(); ++k) jobs[8 * k + x] = q[x][k];
         auto *dj = static_cast<Q2Job *>(
             upload_table(ctx, (std::string(nm) + tag).c_str(), jobs.data(), sizeof(Q2Job) * jobs.size()));
         if (!dj) return PTBGPU_E_NOMEM;
-        const dim3 grid((unsigned)((jobs.size() + 3) / 4));
-        auto kern = two ? k_q2_apply<false, 2> : trans ? k_q2_apply<true, 1> : k_q2_apply<false, 1>;
-        hipLaunchKernelGGL(kern, grid, dim3(256), 0, ctx->stream, dj, (int)jobs.size(), qf.q2fac, Y);
+        auto kern = two ? (trans ? k_q2_apply<true, 2> : k_q2_apply<false, 2>)
+                        : (trans ? k_q2_apply<true, 1> : k_q2_apply<false, 1>);
+        hipLaunchKernelGGL(kern, dim3((unsigned)jobs.size()), dim3(256), 0, ctx->stream, dj, qf.q2fac, Y);
         PTB_CHECK_LAUNCH(ctx);
         return PTBGPU_OK;
     };
-    PTB_TRY(run(wide, "q2_jw_", true));
-    return run(narrow, "q2_jn_", false);
+    PTB_TRY(run("q2_jw_", true));
+    return run("q2_jn_", false);
 }
 
 }  // namespace ptb

@@ -84,3 +84,20 @@ def test_more_submatrices_than_compute_units(engine):
     rep = engine.sm_stupid_simple(mol.ndim, mol.nel, H, S, P, mol.n, mol.xyz, mol.aoat, 1, 2)
     assert np.abs(P - ref.P).max() < 1e-8
     assert rep["mu"] == ref.mu and rep["muiter"] == ref.muiter
+
+
+@pytest.mark.parametrize("m", [3, 18, 19, 34, 66, 83, 98, 530])
+def test_sweep_groups_of_every_remainder(engine, m):
+    """One to five sweep groups and more (a pass of four wavefronts full, cut short,
+    followed by another), last column pieces of several widths: solve2's
+    eigenvectors are S-orthonormal and solve the pencil."""
+    rng = np.random.default_rng(10 * m)
+    A = _matrix(m, "dense")
+    B = rng.normal(size=(m, m))
+    S = np.eye(m) + 0.05 * (B + B.T) / np.sqrt(m)
+    iu = np.tril_indices(m)
+    P, e, focc, U, fail = engine.solve2(1, m, 2, 0, 300.0, A[iu].copy(), S[iu].copy())
+    assert not fail
+    tol = 100 * max(m, 8) * np.finfo(float).eps
+    assert np.abs(U.T @ S @ U - np.eye(m)).max() < tol
+    assert np.abs(A @ U - (S @ U) * e).max() < tol * np.abs(e).max()
