@@ -6,8 +6,8 @@
 //               128x128) output tile per workgroup, k slices staged in
 //               LDS with the next slice prefetched into registers.
 // * k_potrf_panel: one 32-column panel of the lower Cholesky S = L L^T: the
-//               diagonal block factored and inverted in LDS, the panel below as
-//               X = P L_kk^-T; the trailing update is a batched GEMM.  A
+//               diagonal block factored in a wavefront's registers, the panel
+//               below as X = P L_kk^-T; the trailing update is a batched GEMM.  A
 //               non-positive pivot sets flags bit 0 (dsygvd would report INFO>0).
 // * k_diag_inv: inverses of the 64x64 diagonal blocks of L, for the blocked
 //               triangular solves (one GEMM update + one GEMM with the
@@ -50,6 +50,14 @@ using gmem = __attribute__((address_space(1))) T;
 // GEMM time than 32-deep slices at four per SIMD, and 64-deep slices at two
 // per SIMD cost 20 % more.
 constexpr int kKS = 32;  // k depth up to which a product counts as one slice (k_gemm_nt1)
+
+// a wavefront lane's value, in scalar registers
+__device__ __forceinline__ double lane_value(double v, int lane) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_readlane((int)b, lane);
+    const int hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
 
 template <int TE>
 struct GemmTileShape {
@@ -384,87 +392,100 @@ __global__ __launch_bounds__(kT, sizeof(T) == 4 ? 6 : 4) void k_gemm_nt1(
     }
 }
 
-// One 32-column panel of the lower Cholesky factor of every submatrix: factor
-// the diagonal block in LDS, invert it, and form the panel below as
-// X = P L_kk^-T (rows independent).  The trailing update that follows is a
-// batched GEMM.  A non-positive pivot sets flags bit 0 (dsygvd: INFO > 0).
+// One 32-column panel of the lower Cholesky factor of every submatrix: the
+// diagonal block's factor and the panel below as X = P L_kk^-T (rows
+// independent).  The trailing update that follows is a batched GEMM.  A
+// non-positive pivot sets flags bit 0 (dsygvd: INFO > 0).
+//
+// A panel is a serial chain (32 square roots and divisions), so one wavefront
+// keeps the block in registers (lane = row; a column reaches the other lanes
+// through scalar registers, no barrier) while the others load their rows below;
+// these are then solved by substitution, a thread per row, the factor read from
+// LDS (one address per wavefront).  With four wavefronts and three barriers per
+// column, the block's inverse and X = P L_kk^-T by it: 55 us for the rows below and
+// 21 for the block of one 1472-row matrix, now 23 and 5; a panel of the 512-water
+// box 120 us, now 71.
 //
 // mode 0: the whole panel (grid (submatrix, 1)).  For few submatrices the
 // panel is split: mode 1 forms the rows below the diagonal block, sliced over
-// grid.y (each workgroup factors the block in LDS for itself), then mode 2
-// writes the factored diagonal block and the flag (the rows read the block
-// unfactored, so they go first).
+// grid.y (each workgroup factors the block for itself), then mode 2 (one
+// wavefront) writes the factored diagonal block and the flag (the rows read the
+// block unfactored, so they go first).
 __global__ __launch_bounds__(kT) void k_potrf_panel(const SubDesc *__restrict__ desc,
                                                     double *__restrict__ Aa,
                                                     int *__restrict__ flags, int panel, int mode) {
     const SubDesc d = desc[blockIdx.x];
-    const int m = d.m, ld = d.ld;
+    const int m = d.m;
+    const unsigned ld = (unsigned)d.ld;
     const int k0 = panel * 32;
     if (k0 >= m) return;
-    double *a = Aa + d.off;
+    double *a = Aa + d.off + (int64_t)k0 * ld;  // the panel's columns
     const int kb = min(32, m - k0);
-    __shared__ double Lk[32][33], Li[32][33];
-    __shared__ int bad;
-    if (threadIdx.x == 0) bad = 0;
-    for (int l = threadIdx.x; l < 1024; l += kT) {
-        const int r = l & 31, c = l >> 5;
-        double v;
-        if (r < kb && c < kb) v = r >= c ? a[(int64_t)(k0 + c) * ld + k0 + r] : 0.0;
-        else v = (r == c) ? 1.0 : 0.0;  // identity padding
-        Lk[r][c] = v;
-        Li[r][c] = 0.0;
-    }
-    __syncthreads();
-    for (int j = 0; j < kb; ++j) {
-        if (threadIdx.x == 0) {
-            double p = Lk[j][j];
-            if (!(p > 0.0)) {
-                bad = 1;
-                p = 1.0;
+    __shared__ double Lc[32][32], rinv[32];  // Lc[c][r] = L(r, c)
+    double p[32];
+    // a row of the panel below (there are none unless kb = 32)
+    auto load = [&](int i) {
+#pragma unroll
+        for (int t = 0; t < 32; ++t) p[t] = a[(unsigned)t * ld + (unsigned)i];
+    };
+    int i = k0 + 32 + blockIdx.y * kT + threadIdx.x;
+    if (threadIdx.x < PTB_WAVE) {
+        const int r = threadIdx.x & 31;
+        double x[32];
+#pragma unroll
+        for (int c = 0; c < 32; ++c)
+            x[c] = a[(unsigned)min(c, kb - 1) * ld + (unsigned)(k0 + min(r, kb - 1))];
+#pragma unroll
+        for (int c = 0; c < 32; ++c) x[c] = r < kb && c < kb ? (r >= c ? x[c] : 0.0) : r == c ? 1.0 : 0.0;
+        bool bad = false;
+        double diag = 1.0;
+#pragma unroll
+        for (int j = 0; j < 32; ++j) {
+            double q = lane_value(x[j], j);
+            if (!(q > 0.0)) {
+                bad = true;
+                q = 1.0;
             }
-            Lk[j][j] = sqrt(p);
+            const double sq = sqrt(q), l = r == j ? sq : x[j] / sq;
+            x[j] = l;
+            diag = r == j ? sq : diag;
+#pragma unroll
+            for (int c = j + 1; c < 32; ++c) x[c] -= l * lane_value(l, c);
         }
-        __syncthreads();
-        if ((int)threadIdx.x > j && (int)threadIdx.x < kb) Lk[threadIdx.x][j] /= Lk[j][j];
-        __syncthreads();
-        for (int l = threadIdx.x; l < 1024; l += kT) {
-            const int r = l & 31, c = l >> 5;
-            if (c > j && r >= c && r < kb) Lk[r][c] -= Lk[r][j] * Lk[c][j];
+        if (mode != 1) {
+            if (threadIdx.x < 32)
+#pragma unroll
+                for (int c = 0; c < 32; ++c)
+                    if (r < kb && c <= r) a[(unsigned)c * ld + (unsigned)(k0 + r)] = x[c];
+            if (threadIdx.x == 0 && bad) flags[blockIdx.x] |= 1;
         }
-        __syncthreads();
-    }
-    if (mode != 1)
-        for (int l = threadIdx.x; l < 1024; l += kT) {
-            const int r = l & 31, c = l >> 5;
-            if (r < kb && c < kb && r >= c) a[(int64_t)(k0 + c) * ld + k0 + r] = Lk[r][c];
+        if (mode == 2) return;
+        if (threadIdx.x < 32) {
+#pragma unroll
+            for (int c = 0; c < 32; ++c) Lc[c][r] = x[c];
+            rinv[r] = 1.0 / diag;
         }
-    if (mode == 2) {
-        if (threadIdx.x == 0 && bad) flags[blockIdx.x] |= 1;
-        return;
-    }
-    // Li = Lk^-1, column c by thread c (forward substitution)
-    if (threadIdx.x < 32) {
-        const int c = threadIdx.x;
-        for (int r = c; r < 32; ++r) {
-            double sacc = (r == c) ? 1.0 : 0.0;
-            for (int t = c; t < r; ++t) sacc -= Lk[r][t] * Li[t][c];
-            Li[r][c] = sacc / Lk[r][r];
-        }
+        if (i < m) load(i);
+    } else if (i < m) {
+        load(i);
     }
     __syncthreads();
-    // X(i, c) = sum_{t<=c} P(i, t) Li(c, t)
-    for (int i = k0 + kb + blockIdx.y * kT + threadIdx.x; i < m; i += gridDim.y * kT) {
-        double p[32];
+    // p <- p L^-T, column by column
+    int zero = 0;
+    while (i < m) {
+        asm volatile("" : "+v"(zero));  // (keeps the factor in LDS)
 #pragma unroll
-        for (int t = 0; t < 32; ++t) p[t] = t < kb ? a[(int64_t)(k0 + t) * ld + i] : 0.0;
-        for (int c = 0; c < kb; ++c) {
-            double sacc = 0.0;
+        for (int c = 0; c < 32; ++c) {
+            p[c] *= rinv[c + zero];
 #pragma unroll
-            for (int t = 0; t < 32; ++t) sacc += p[t] * Li[c][t];
-            a[(int64_t)(k0 + c) * ld + i] = sacc;
+            for (int t = c + 1; t < 32; ++t) p[t] -= p[c] * Lc[c][t + zero];
+            if (c & 1) __builtin_amdgcn_sched_barrier(0);  // (nor read all of it ahead)
         }
+#pragma unroll
+        for (int c = 0; c < 32; ++c) a[(unsigned)c * ld + (unsigned)i] = p[c];
+        i += gridDim.y * kT;
+        if (i < m) load(i);
     }
-    if (mode == 0 && threadIdx.x == 0 && bad) flags[blockIdx.x] |= 1;
 }
 
 // L = I (lower triangle) for the submatrices whose Cholesky met a
@@ -1392,7 +1413,7 @@ int potrf_batch(ptbgpu_ctx *ctx, const std::vector<SubDesc> &desc, const SubDesc
             hipLaunchKernelGGL(k_potrf_panel, dim3(nsm), dim3(kT), 0, ctx->stream, ddesc, A, flags, p, 0);
         } else {
             hipLaunchKernelGGL(k_potrf_panel, dim3(nsm, ny), dim3(kT), 0, ctx->stream, ddesc, A, flags, p, 1);
-            hipLaunchKernelGGL(k_potrf_panel, dim3(nsm), dim3(kT), 0, ctx->stream, ddesc, A, flags, p, 2);
+            hipLaunchKernelGGL(k_potrf_panel, dim3(nsm), dim3(PTB_WAVE), 0, ctx->stream, ddesc, A, flags, p, 2);
         }
         PTB_CHECK_LAUNCH(ctx);
         return PTBGPU_OK;
