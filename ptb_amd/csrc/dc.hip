@@ -177,12 +177,55 @@ __device__ __forceinline__ double rcp64(double x) {
     return fma(r, e, r);
 }
 
+// Lanes that share a root or a Loewner entry of a node of kLanesMin rows or more
+// (a thread's chain of O(K) terms is an eighth as long).  The number depends on the
+// node alone, so a density does not depend on what else is in the batch.  Merges of
+// 512 rows and more of the 512-water box 4.9 -> 4.5 ms, of 256 to 511 3.2 -> 2.8.
+constexpr int kRootLanes = 8, kLanesMin = 256;
+template <int CTRL>
+__device__ __forceinline__ double dpp_mov(double v) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+// op over the eight lanes of a group, the same value in each (quad_perm 1032 and
+// 2301, then the mirror within 8)
+template <typename F>
+__device__ __forceinline__ double group_reduce(double v, F op) {
+    v = op(v, dpp_mov<0xB1>(v));
+    v = op(v, dpp_mov<0x4E>(v));
+    return op(v, dpp_mov<0x141>(v));
+}
+
 // s = sum_{i0 <= i < i1} q_i, ds = sum q_i r_i with r_i = 1 / ((d_i - dorg) - t),
 // q_i = w2_i r_i: the secular function's pole terms and their derivatives.
 // Four interleaved partial sums, so that the terms' dependent chains
-// (reciprocal, Newton steps, accumulation) overlap.
+// (reciprocal, Newton steps, accumulation) overlap.  L = 8: lane l of a group of
+// eight takes every eighth term (two partial sums), and every lane gets the sums.
+template <int L>
 __device__ __forceinline__ void secular_sums(const double *dl, const double *w2, int i0, int i1,
-                                             double dorg, double t, double &s, double &ds) {
+                                             double dorg, double t, int l, double &s, double &ds) {
+    if constexpr (L == kRootLanes) {
+        double a0 = 0.0, a1 = 0.0, b0 = 0.0, b1 = 0.0;
+        int i = i0 + l;
+        for (; i + L < i1; i += 2 * L) {
+            const double r0 = rcp64((dl[i] - dorg) - t), r1 = rcp64((dl[i + L] - dorg) - t);
+            const double q0 = w2[i] * r0, q1 = w2[i + L] * r1;
+            a0 += q0;
+            a1 += q1;
+            b0 += q0 * r0;
+            b1 += q1 * r1;
+        }
+        if (i < i1) {
+            const double r = rcp64((dl[i] - dorg) - t), q = w2[i] * r;
+            a0 += q;
+            b0 += q * r;
+        }
+        s = group_reduce(a0 + a1, [](double x, double y) { return x + y; });
+        ds = group_reduce(b0 + b1, [](double x, double y) { return x + y; });
+        return;
+    }
     double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0, b0 = 0.0, b1 = 0.0, b2 = 0.0, b3 = 0.0;
     int i = i0;
     for (; i + 4 <= i1; i += 4) {
@@ -229,15 +272,17 @@ __device__ __forceinline__ void copy_column(double *__restrict__ dst,
 }
 
 // Secular root j of a merge with K poles dl (ascending), weights w and
-// w2 = rho w^2: the root's origin pole org[j] and offset tau[j].
+// w2 = rho w^2: the root's origin pole org[j] and offset tau[j].  One thread, or
+// a group of L lanes (l this one's) in step.
+template <int L>
 __device__ void dc_root(int j, int K, const double *dl, const double *w2, const double *w,
-                        double rho, int *org, double *tau) {
+                        double rho, int *org, double *tau, int l = 0) {
     int o;
     double lo, hi;
     if (j < K - 1) {
         const double mid = 0.5 * (dl[j + 1] - dl[j]);
         double fs, fds;
-        secular_sums(dl, w2, 0, K, dl[j], mid, fs, fds);
+        secular_sums<L>(dl, w2, 0, K, dl[j], mid, l, fs, fds);
         const double f = 1.0 + fs;
         if (f >= 0.0) {
             o = j;
@@ -251,7 +296,8 @@ __device__ void dc_root(int j, int K, const double *dl, const double *w2, const 
     } else {
         o = j;
         double s2 = 0.0;
-        for (int i = 0; i < K; ++i) s2 += w[i] * w[i];
+        for (int i = l; i < K; i += L) s2 += w[i] * w[i];
+        if constexpr (L > 1) s2 = group_reduce(s2, [](double x, double y) { return x + y; });
         lo = 0.0;
         hi = rho * s2;
     }
@@ -269,8 +315,8 @@ __device__ void dc_root(int j, int K, const double *dl, const double *w2, const 
     double t = 0.5 * (lo + hi);
     for (int it = 0; it < 200; ++it) {
         double psi, dpsi, phi, dphi;
-        secular_sums(dl, w2, 0, j + 1, dorg, t, psi, dpsi);
-        secular_sums(dl, w2, j + 1, K, dorg, t, phi, dphi);
+        secular_sums<L>(dl, w2, 0, j + 1, dorg, t, l, psi, dpsi);
+        secular_sums<L>(dl, w2, j + 1, K, dorg, t, l, phi, dphi);
         const double f = 1.0 + psi + phi;
         if (f == 0.0 || fabs(f) <= 8.0 * kEps * (double)K * (1.0 + fabs(psi) + fabs(phi))) {
             lo = hi = t;
@@ -306,20 +352,25 @@ __device__ void dc_root(int j, int K, const double *dl, const double *w2, const 
         if (tn == t || tn == lo || tn == hi) break;
         t = tn;
     }
-    org[j] = o;
-    tau[j] = (lo == hi) ? lo : t;
+    if (l == 0) {
+        org[j] = o;
+        tau[j] = (lo == hi) ? lo : t;
+    }
 }
 
 // Loewner vector entry i: rho zhat_i^2 = (lam_i - d_i) prod_{j != i} (lam_j - d_i)/(d_j - d_i)
+// (by one thread, or by a group of L lanes, l this one's)
+template <int L>
 __device__ double dc_loewner(int i, int K, const double *dl, const int *org, const double *tau,
-                             const double *w, double rho) {
+                             const double *w, double rho, int l = 0) {
     const double di = dl[i];
-    double prod = -((di - dl[org[i]]) - tau[i]);
-    for (int j = 0; j < K; ++j) {
+    double prod = l == 0 ? -((di - dl[org[i]]) - tau[i]) : 1.0;
+    for (int j = l; j < K; j += L) {
         if (j == i) continue;
         const double dlt = (di - dl[org[j]]) - tau[j];  // d_i - lam_j
         prod *= (-dlt) * rcp64(dl[j] - di);
     }
+    if constexpr (L > 1) prod = group_reduce(prod, [](double x, double y) { return x * y; });
     return copysign(sqrt(fmax(prod, 0.0) / rho), w[i]);
 }
 
@@ -376,10 +427,13 @@ __device__ int block_scan_excl(int v, int *wsum, int *total) {
 // kernel writes both descriptors, gd[2 node] and gd[2 node + 1].
 //
 // The per-node vectors (6 doubles and 4 ints per row, padded to the power of
-// two npow) live in LDS up to npow = 2048; larger nodes (kGlobal) keep them
+// two npow) live in LDS up to npow = 2048; larger nodes (kDcGlobal) keep them
 // in a device scratch of 8 npow doubles per node at gscr, which only this
-// workgroup touches (its barriers order the accesses as they do in LDS).
-template <bool kGlobal, int NT>
+// workgroup touches (its barriers order the accesses as they do in LDS).  With
+// kDcSpread they go from LDS to that scratch once the slots are known, and the
+// columns and the O(K^2) phases are left to kernels over the whole chip.
+constexpr int kDcLds = 0, kDcGlobal = 1, kDcSpread = 2;
+template <int MODE, int NT>
 __global__ __launch_bounds__(NT) void k_dc_merge(const SubDesc *__restrict__ desc,
                                                   const DcNode *__restrict__ nodes, int npow,
                                                   const double *__restrict__ e_all,
@@ -389,6 +443,7 @@ __global__ __launch_bounds__(NT) void k_dc_merge(const SubDesc *__restrict__ des
                                                   double *__restrict__ rot_all,
                                                   GemmDesc *__restrict__ gd, double *gscr,
                                                   int *gK) {
+    constexpr bool kGlobal = MODE == kDcGlobal;
     extern __shared__ double shm_[];
     double *shm;
     if constexpr (kGlobal) shm = gscr + (size_t)blockIdx.x * 8 * (size_t)npow;
@@ -421,7 +476,7 @@ __global__ __launch_bounds__(NT) void k_dc_merge(const SubDesc *__restrict__ des
     constexpr int kWaves = NT / PTB_WAVE;
 
     if (rho == 0.0) {  // decoupled: children are already eigenpairs of T
-        if (kGlobal && threadIdx.x == 0) gK[blockIdx.x] = 0;
+        if (MODE != kDcLds && threadIdx.x == 0) gK[4 * blockIdx.x] = gK[4 * blockIdx.x + 1] = 0;
         if (threadIdx.x < 2) {
             g[threadIdx.x].M = 0;
             g[threadIdx.x].N = 0;
@@ -602,6 +657,30 @@ __global__ __launch_bounds__(NT) void k_dc_merge(const SubDesc *__restrict__ des
         __syncthreads();
     }
     const int KL = sKL, KD = sKD;
+    if constexpr (MODE == kDcSpread) {
+        double *b = gscr + (size_t)blockIdx.x * 8 * (size_t)npow;
+        int *gmask = reinterpret_cast<int *>(b), *gi = reinterpret_cast<int *>(b + 6 * (size_t)npow);
+        for (int j = threadIdx.x; j < n; j += NT) {
+            gmask[j] = cmask[j];
+            gi[j] = ix[j];
+            gi[npow + j] = slot[j];
+            if (slot[j] >= K) D[nd.lo + slot[j]] = Dk[j];
+        }
+        for (int i = threadIdx.x; i < K; i += NT) {
+            b[2 * (size_t)npow + i] = dl[i];
+            b[3 * (size_t)npow + i] = w[i];
+            b[5 * (size_t)npow + i] = rho * w[i] * w[i];
+            gi[3 * (size_t)npow + i] = prow[i];
+        }
+        if (threadIdx.x == 0) {
+            int *o = gK + 4 * blockIdx.x;
+            o[0] = K;
+            o[1] = n;  // columns to place
+            o[2] = nr;
+            o[3] = KL | (KD << 16);
+        }
+    }
+    if constexpr (MODE != kDcSpread) {
     // sorted, compacted eigenvector columns into W: W(:, slot[j]) = Z(:, lo+ix[j]),
     // one column per wavefront.  A child's column is nonzero only on the
     // child's rows, which are the only rows read.  Left-only and right-only
@@ -636,8 +715,8 @@ __global__ __launch_bounds__(NT) void k_dc_merge(const SubDesc *__restrict__ des
     for (int j = threadIdx.x; j < n; j += NT)
         if (slot[j] >= K) D[nd.lo + slot[j]] = Dk[j];
     __syncthreads();
-    double *w2 = zh;
-    for (int i = threadIdx.x; i < K; i += NT) w2[i] = rho * w[i] * w[i];
+    for (int i = threadIdx.x; i < K; i += NT) zh[i] = rho * w[i] * w[i];
+    }
     if (threadIdx.x < 2) {
         // 0: rows above the split from slots [0, KL + KD); 1: rows below it
         // from slots [KL, K)
@@ -661,16 +740,26 @@ __global__ __launch_bounds__(NT) void k_dc_merge(const SubDesc *__restrict__ des
     }
     // a node from device scratch leaves the O(K^2) phases to three kernels
     // over the whole chip (k_dc_roots_big, k_dc_loewner_big, k_dc_vectors_big)
-    if constexpr (kGlobal) {
-        if (threadIdx.x == 0) gK[blockIdx.x] = K;
-        return;
-    }
+    if constexpr (kGlobal)
+        if (threadIdx.x == 0) gK[4 * blockIdx.x] = K;
+    if constexpr (MODE != kDcLds) return;
     __syncthreads();
-    // secular roots, one thread per root
-    for (int j = threadIdx.x; j < K; j += NT) dc_root(j, K, dl, w2, w, rho, org, tau);
+    // secular roots, one thread or kRootLanes lanes per root
+    const int rl = threadIdx.x % kRootLanes;
+    if (n >= kLanesMin)
+        for (int j = threadIdx.x / kRootLanes; j < K; j += NT / kRootLanes)
+            dc_root<kRootLanes>(j, K, dl, zh, w, rho, org, tau, rl);
+    else
+        for (int j = threadIdx.x; j < K; j += NT) dc_root<1>(j, K, dl, zh, w, rho, org, tau);
     __syncthreads();
     // Loewner vector: rho zhat_i^2 = (lam_i - d_i) prod_{j != i} (lam_j - d_i)/(d_j - d_i)
-    for (int i = threadIdx.x; i < K; i += NT) zh[i] = dc_loewner(i, K, dl, org, tau, w, rho);
+    if (n >= kLanesMin)
+        for (int i = threadIdx.x / kRootLanes; i < K; i += NT / kRootLanes) {
+            const double v = dc_loewner<kRootLanes>(i, K, dl, org, tau, w, rho, rl);
+            if (rl == 0) zh[i] = v;
+        }
+    else
+        for (int i = threadIdx.x; i < K; i += NT) zh[i] = dc_loewner<1>(i, K, dl, org, tau, w, rho);
     __syncthreads();
     // U(:, j) = zhat ./ (d - lam_j), normalised; eigenvalues lam_j.  One
     // column per wavefront: its norm, then the column (lanes on rows).
@@ -688,7 +777,7 @@ struct BigNode {
     double *zh;
     int *org, *prow;
     double rho;
-    int K;
+    int K, n;
 };
 
 __device__ BigNode big_node(const SubDesc *desc, const DcNode *nodes, int npow,
@@ -705,26 +794,9 @@ __device__ BigNode big_node(const SubDesc *desc, const DcNode *nodes, int npow,
     g.org = ib + 2 * (size_t)npow;
     g.prow = ib + 3 * (size_t)npow;
     g.rho = 2.0 * fabs(e_all[ds.mapoff + nd.sp - 1]);
-    g.K = gK[node];
+    g.K = gK[4 * (size_t)node];
+    g.n = nd.hi - nd.lo;
     return g;
-}
-
-__global__ __launch_bounds__(kMT) void k_dc_roots_big(const SubDesc *__restrict__ desc,
-                                                      const DcNode *__restrict__ nodes, int npow,
-                                                      const double *__restrict__ e_all,
-                                                      double *gscr, const int *__restrict__ gK) {
-    BigNode g = big_node(desc, nodes, npow, e_all, gscr, gK, blockIdx.y);
-    const int j = blockIdx.x * kMT + threadIdx.x;
-    if (j < g.K) dc_root(j, g.K, g.dl, g.zh, g.w, g.rho, g.org, const_cast<double *>(g.tau));
-}
-
-__global__ __launch_bounds__(kMT) void k_dc_loewner_big(const SubDesc *__restrict__ desc,
-                                                        const DcNode *__restrict__ nodes, int npow,
-                                                        const double *__restrict__ e_all,
-                                                        double *gscr, const int *__restrict__ gK) {
-    BigNode g = big_node(desc, nodes, npow, e_all, gscr, gK, blockIdx.y);
-    const int i = blockIdx.x * kMT + threadIdx.x;
-    if (i < g.K) g.zh[i] = dc_loewner(i, g.K, g.dl, g.org, g.tau, g.w, g.rho);
 }
 
 __global__ __launch_bounds__(kMT) void k_dc_vectors_big(const SubDesc *__restrict__ desc,
@@ -741,6 +813,100 @@ __global__ __launch_bounds__(kMT) void k_dc_vectors_big(const SubDesc *__restric
     if (j < g.K)
         dc_vector(j, lane, g.K, g.dl, g.org, g.tau, g.zh, g.prow,
                   Xa + ds.off + (int64_t)(nd.lo + j) * ds.ld + nd.lo, D_all + ds.mapoff + nd.lo);
+}
+
+// After the front of a merge (kDcGlobal, kDcSpread): its vectors in gscr, the node's
+// counts in gK; grid (blocks, node).
+//
+// Secular roots (the first nroot blocks); after kDcSpread also the sorted, compacted
+// columns into W, one per wavefront (see k_dc_merge).
+constexpr int kRootsPerBlock = kMT / kRootLanes;
+__global__ __launch_bounds__(kMT) void k_dc_roots_columns(const SubDesc *__restrict__ desc,
+                                                          const DcNode *__restrict__ nodes, int npow,
+                                                          const double *__restrict__ e_all,
+                                                          const double *__restrict__ Za,
+                                                          double *__restrict__ Wa, double *gscr,
+                                                          const int *__restrict__ gK, int nroot) {
+    const int node = blockIdx.y;
+    if ((int)blockIdx.x < nroot) {
+        BigNode g = big_node(desc, nodes, npow, e_all, gscr, gK, node);
+        double *tau = const_cast<double *>(g.tau);
+        if (g.n >= kLanesMin) {
+            const int j = blockIdx.x * kRootsPerBlock + threadIdx.x / kRootLanes;
+            if (j < g.K)
+                dc_root<kRootLanes>(j, g.K, g.dl, g.zh, g.w, g.rho, g.org, tau, threadIdx.x % kRootLanes);
+        } else {
+            const int j = blockIdx.x * kMT + threadIdx.x;
+            if (j < g.K) dc_root<1>(j, g.K, g.dl, g.zh, g.w, g.rho, g.org, tau);
+        }
+        return;
+    }
+    const int lane = threadIdx.x % PTB_WAVE, wid = threadIdx.x / PTB_WAVE;
+    const int j = (blockIdx.x - nroot) * (kMT / PTB_WAVE) + wid;
+    const int K = gK[4 * node], n = gK[4 * node + 1];
+    if (j >= n) return;
+    const int KL = gK[4 * node + 3] & 0xffff, KD = gK[4 * node + 3] >> 16;
+    const DcNode nd = nodes[node];
+    const SubDesc ds = desc[nd.s];
+    const int n1 = nd.sp - nd.lo, ld = ds.ld;
+    const double *b = gscr + (size_t)node * 8 * (size_t)npow;
+    const int *gi = reinterpret_cast<const int *>(b + 6 * (size_t)npow);
+    const int c = gi[j], sl = gi[npow + j], mask = reinterpret_cast<const int *>(b)[j];
+    const int cb = c < n1 ? 0 : n1, ce = c < n1 ? n1 : n;
+    const bool half = !(mask & 4) && (sl < KL || (sl >= KL + KD && sl < K));
+    copy_column(Wa + ds.off + (int64_t)(nd.lo + sl) * ld + nd.lo,
+                Za + ds.off + (int64_t)(nd.lo + c) * ld + nd.lo, half ? cb : 0, half ? ce : n, lane, cb, ce);
+}
+
+// Loewner entries (the first nroot blocks) and, after kDcSpread, 64 rows a block: the deflation rotations in order, then the deflated columns to their
+// final place.
+__global__ __launch_bounds__(kMT) void k_dc_loewner_deflated(const SubDesc *__restrict__ desc,
+                                                             const DcNode *__restrict__ nodes, int npow,
+                                                             const double *__restrict__ e_all,
+                                                             const double *__restrict__ rot_all,
+                                                             double *__restrict__ Za,
+                                                             double *__restrict__ Wa, double *gscr,
+                                                             const int *__restrict__ gK, int nroot) {
+    const int node = blockIdx.y;
+    if ((int)blockIdx.x < nroot) {
+        BigNode g = big_node(desc, nodes, npow, e_all, gscr, gK, node);
+        if (g.n >= kLanesMin) {
+            const int i = blockIdx.x * kRootsPerBlock + threadIdx.x / kRootLanes;
+            if (i >= g.K) return;
+            const double v =
+                dc_loewner<kRootLanes>(i, g.K, g.dl, g.org, g.tau, g.w, g.rho, threadIdx.x % kRootLanes);
+            if (threadIdx.x % kRootLanes == 0) g.zh[i] = v;
+        } else {
+            const int i = blockIdx.x * kMT + threadIdx.x;
+            if (i < g.K) g.zh[i] = dc_loewner<1>(i, g.K, g.dl, g.org, g.tau, g.w, g.rho);
+        }
+        return;
+    }
+    const int K = gK[4 * node], n = gK[4 * node + 1], nr = gK[4 * node + 2];
+    const int lane = threadIdx.x % PTB_WAVE, wid = threadIdx.x / PTB_WAVE;
+    const int r = (blockIdx.x - nroot) * PTB_WAVE + lane;
+    if ((int)(blockIdx.x - nroot) * PTB_WAVE >= n) return;
+    const DcNode nd = nodes[node];
+    const SubDesc ds = desc[nd.s];
+    const int ld = ds.ld;
+    double *W = Wa + ds.off + (int64_t)nd.lo * ld + nd.lo, *Z = Za + ds.off + (int64_t)nd.lo * ld + nd.lo;
+    if (nr > 0) {
+        const double *rot = rot_all + 4 * (int64_t)(ds.mapoff + nd.lo);
+        const int *slot = reinterpret_cast<const int *>(gscr + (size_t)node * 8 * (size_t)npow +
+                                                        6 * (size_t)npow) + npow;
+        if (wid == 0 && r < n)
+            for (int q = 0; q < nr; ++q) {
+                double *pp = W + (int64_t)slot[(int)rot[4 * q]] * ld + r;
+                double *pj = W + (int64_t)slot[(int)rot[4 * q + 1]] * ld + r;
+                const double c = rot[4 * q + 2], s = rot[4 * q + 3], qp = *pp, qj = *pj;
+                *pp = c * qp + s * qj;
+                *pj = c * qj - s * qp;
+            }
+        __syncthreads();
+    }
+    if (r >= n) return;
+#pragma unroll 4
+    for (int c = K + wid; c < n; c += kMT / PTB_WAVE) Z[(int64_t)c * ld + r] = W[(int64_t)c * ld + r];
 }
 
 }  // namespace
@@ -793,7 +959,34 @@ int dc_merge_level(ptbgpu_ctx *ctx, const SubDesc *ddesc, const DcNode *dnodes, 
             const int i1 = r + 1 < runs.size() ? runs[r + 1].first : count;
             const int np = runs[r].second;
             const bool global = !in_lds(np) || (ctx->dc_global_min > 0 && np >= ctx->dc_global_min);
-            if (!global) {
+            // No more nodes than CUs: each would hold one CU with a chain of O(n^2)
+            // phases while the others idle or finish early, so only the front of the
+            // merge stays one workgroup per node (all merges of one 1472-row matrix
+            // 4.9 ms in one workgroup each, 1.2 so; of 24 submatrices of 8 waters
+            // 0.81 and 0.52; a level of 192 nodes up to 811 rows 1.4 and 0.75)
+            // (np bounds the rows of every node of the run)
+            const int nroot = (np + kRootsPerBlock - 1) / kRootsPerBlock;
+            const bool spread = in_lds(np) && ctx->dc_global_min == 0 && i1 - i0 <= ctx->num_cus;
+            if (spread) {
+                const int nn = i1 - i0;
+                auto *scr = static_cast<double *>(
+                    ws(ctx, "dc_gscr", sizeof(double) * 8 * (size_t)np * (size_t)nn));
+                auto *gK = static_cast<int *>(ws(ctx, "dc_gK", 4 * sizeof(int) * (size_t)nn));
+                if (!scr || !gK) return PTBGPU_E_NOMEM;
+                const size_t shmem = (size_t)np * (6 * sizeof(double) + 4 * sizeof(int));
+                if (np <= 512)
+                    hipLaunchKernelGGL((k_dc_merge<kDcSpread, 256>), dim3(nn), dim3(256), shmem, ctx->stream, ddesc,
+                                       dnodes + i0, np, e, D, Z, W, X, rot, dgemm + 2 * i0, scr, gK);
+                else
+                    hipLaunchKernelGGL((k_dc_merge<kDcSpread, 512>), dim3(nn), dim3(512), shmem, ctx->stream, ddesc,
+                                       dnodes + i0, np, e, D, Z, W, X, rot, dgemm + 2 * i0, scr, gK);
+                hipLaunchKernelGGL(k_dc_roots_columns, dim3((unsigned)(nroot + (np + 3) / 4), nn), dim3(kMT), 0,
+                                   ctx->stream, ddesc, dnodes + i0, np, e, Z, W, scr, gK, nroot);
+                hipLaunchKernelGGL(k_dc_loewner_deflated, dim3((unsigned)(nroot + (np + 63) / 64), nn), dim3(kMT), 0,
+                                   ctx->stream, ddesc, dnodes + i0, np, e, rot, Z, W, scr, gK, nroot);
+                hipLaunchKernelGGL(k_dc_vectors_big, dim3((unsigned)((np + 3) / 4), nn), dim3(kMT), 0,
+                                   ctx->stream, ddesc, dnodes + i0, np, e, D, X, scr, gK);
+            } else if (!global) {
                 // a workgroup of min(max(np / 2, 64), 512) threads per node:
                 // the small nodes of the low levels leave fewer threads of a
                 // larger group idle at every barrier, and more of them fit
@@ -802,10 +995,10 @@ int dc_merge_level(ptbgpu_ctx *ctx, const SubDesc *ddesc, const DcNode *dnodes, 
                 // fill the CU's wavefront slots with 512 threads
                 const size_t shmem = (size_t)np * (6 * sizeof(double) + 4 * sizeof(int));
                 const int half = np / 2;
-                auto k = half <= 64    ? k_dc_merge<false, 64>
-                         : half <= 128 ? k_dc_merge<false, 128>
-                         : half <= 256 ? k_dc_merge<false, 256>
-                                       : k_dc_merge<false, 512>;
+                auto k = half <= 64    ? k_dc_merge<kDcLds, 64>
+                         : half <= 128 ? k_dc_merge<kDcLds, 128>
+                         : half <= 256 ? k_dc_merge<kDcLds, 256>
+                                       : k_dc_merge<kDcLds, 512>;
                 const int nt = half <= 64 ? 64 : (half <= 128 ? 128 : (half <= 256 ? 256 : 512));
                 hipLaunchKernelGGL(k, dim3(i1 - i0), dim3(nt), shmem, ctx->stream, ddesc, dnodes + i0,
                                    np, e, D, Z, W, X, rot, dgemm + 2 * i0, nullptr, nullptr);
@@ -813,15 +1006,14 @@ int dc_merge_level(ptbgpu_ctx *ctx, const SubDesc *ddesc, const DcNode *dnodes, 
                 const int nn = i1 - i0;
                 auto *scr = static_cast<double *>(
                     ws(ctx, "dc_gscr", sizeof(double) * 8 * (size_t)np * (size_t)nn));
-                auto *gK = static_cast<int *>(ws(ctx, "dc_gK", sizeof(int) * (size_t)nn));
+                auto *gK = static_cast<int *>(ws(ctx, "dc_gK", 4 * sizeof(int) * (size_t)nn));
                 if (!scr || !gK) return PTBGPU_E_NOMEM;
-                hipLaunchKernelGGL((k_dc_merge<true, kMT>), dim3(nn), dim3(kMT), 0, ctx->stream, ddesc,
+                hipLaunchKernelGGL((k_dc_merge<kDcGlobal, kMT>), dim3(nn), dim3(kMT), 0, ctx->stream, ddesc,
                                    dnodes + i0, np, e, D, Z, W, X, rot, dgemm + 2 * i0, scr, gK);
-                const unsigned nb = (unsigned)((np + kMT - 1) / kMT);
-                hipLaunchKernelGGL(k_dc_roots_big, dim3(nb, nn), dim3(kMT), 0, ctx->stream, ddesc,
-                                   dnodes + i0, np, e, scr, gK);
-                hipLaunchKernelGGL(k_dc_loewner_big, dim3(nb, nn), dim3(kMT), 0, ctx->stream, ddesc,
-                                   dnodes + i0, np, e, scr, gK);
+                hipLaunchKernelGGL(k_dc_roots_columns, dim3((unsigned)nroot, nn), dim3(kMT), 0, ctx->stream, ddesc,
+                                   dnodes + i0, np, e, Z, W, scr, gK, nroot);
+                hipLaunchKernelGGL(k_dc_loewner_deflated, dim3((unsigned)nroot, nn), dim3(kMT), 0, ctx->stream,
+                                   ddesc, dnodes + i0, np, e, rot, Z, W, scr, gK, nroot);
                 hipLaunchKernelGGL(k_dc_vectors_big, dim3((unsigned)((np + 3) / 4), nn), dim3(kMT), 0,
                                    ctx->stream, ddesc, dnodes + i0, np, e, D, X, scr, gK);
             }
