@@ -54,6 +54,52 @@ void ws_trim(ptbgpu_ctx *ctx, const char *name, size_t bytes) {
     ctx->shadow.erase(name);
 }
 
+// Tables go into one half of the ring after the other; a half is used again when
+// the copies out of it are done.  It starts small and grows (to kRingHalfMax) while
+// tables do not fit or the host would wait for it; larger tables are copied as
+// they are.
+int upload_async(ptbgpu_ctx *ctx, void *dst, const void *src, size_t bytes) {
+    constexpr size_t kRingHalfMin = (size_t)1 << 20, kRingHalfMax = (size_t)32 << 20;
+    const size_t need = (bytes + 255) & ~(size_t)255;
+    if (need > kRingHalfMax) {
+        PTB_HIP(ctx, hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, ctx->stream));
+        return PTBGPU_OK;
+    }
+    for (auto &e : ctx->ring_ev)
+        if (!e) PTB_HIP(ctx, hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    size_t half = std::max(ctx->ring_half, kRingHalfMin);
+    while (half < need) half *= 2;
+    if (half == ctx->ring_half && ctx->ring_pos + need > half) {
+        const int cur = ctx->ring_cur, next = cur ^ 1;
+        PTB_HIP(ctx, hipEventRecord(ctx->ring_ev[cur], ctx->stream));
+        ctx->ring_busy[cur] = true;
+        const bool wait = ctx->ring_busy[next] && hipEventQuery(ctx->ring_ev[next]) != hipSuccess;
+        if (wait) (void)hipGetLastError();
+        if (wait && half < kRingHalfMax) {
+            half *= 2;
+        } else {
+            if (wait) PTB_HIP(ctx, hipEventSynchronize(ctx->ring_ev[next]));
+            ctx->ring_busy[next] = false;
+            ctx->ring_cur = next;
+            ctx->ring_pos = 0;
+        }
+    }
+    if (half != ctx->ring_half) {
+        ctx->ring_half = 0;
+        // (hws waits for the stream before it gives the old ring back)
+        if (!hws(ctx, "table_ring", 2 * half)) return PTBGPU_E_NOMEM;
+        ctx->ring_half = half;
+        ctx->ring_pos = 0;
+        ctx->ring_cur = 0;
+        ctx->ring_busy[0] = ctx->ring_busy[1] = false;
+    }
+    char *p = static_cast<char *>(hws(ctx, "table_ring", 2 * half)) + half * ctx->ring_cur + ctx->ring_pos;
+    memcpy(p, src, bytes);
+    ctx->ring_pos += need;
+    PTB_HIP(ctx, hipMemcpyAsync(dst, p, bytes, hipMemcpyHostToDevice, ctx->stream));
+    return PTBGPU_OK;
+}
+
 void *upload_table(ptbgpu_ctx *ctx, const char *name_in, const void *src, size_t bytes) {
     // tables of a graph-held phase live under the graph's own prefix, so that
     // other builds do not overwrite what its replays read
@@ -69,9 +115,8 @@ void *upload_table(ptbgpu_ctx *ctx, const char *name_in, const void *src, size_t
         fail(ctx, PTBGPU_E_ARG, "table '%s' changed during a graph capture", name);
         return nullptr;
     }
-    if (hipMemcpyAsync(d, src, bytes, hipMemcpyHostToDevice, ctx->stream) != hipSuccess) {
+    if (upload_async(ctx, d, src, bytes) != PTBGPU_OK) {
         ctx->shadow.erase(name);
-        fail(ctx, PTBGPU_E_HIP, "upload of '%s' failed: %s", name, hipGetErrorString(hipGetLastError()));
         return nullptr;
     }
     const char *c = static_cast<const char *>(src);
@@ -262,6 +307,8 @@ int ptbgpu_finalize(ptbgpu_ctx *ctx) {
     for (auto &kv : ctx->host_bufs)
         if (kv.second.ptr) (void)hipHostFree(kv.second.ptr);
     for (auto &e : ctx->stage_ev)
+        if (e) (void)hipEventDestroy(e);
+    for (auto &e : ctx->ring_ev)
         if (e) (void)hipEventDestroy(e);
     (void)hipStreamDestroy(ctx->stream);
     delete ctx;

@@ -78,6 +78,12 @@ struct ptbgpu_ctx {
     // after each buffer's last device copy, and whether one is pending
     hipEvent_t stage_ev[2] = {nullptr, nullptr};
     bool stage_busy[2] = {false, false};
+    // pinned staging of the tables (upload_async): two halves of ring_half bytes, the
+    // one in use, its fill, and the event behind each half's last copy
+    size_t ring_half = 0, ring_pos = 0;
+    int ring_cur = 0;
+    hipEvent_t ring_ev[2] = {nullptr, nullptr};
+    bool ring_busy[2] = {false, false};
     // PTBGPU_POISON_ARENAS=1 at ptbgpu_init: the floating-point arenas of a
     // density build are filled with NaN before each (eager) use, so that a
     // read of an element the build did not write shows in the result (tests)
@@ -98,6 +104,11 @@ void ws_trim(ptbgpu_ctx *ctx, const char *name, size_t bytes);
 // (descriptor tables of repeated builds with the same structure).  Returns the
 // device pointer, or nullptr with the error recorded.
 void *upload_table(ptbgpu_ctx *ctx, const char *name, const void *src, size_t bytes);
+// Copies a host table to the device on the context's stream through pinned
+// memory, so that the host goes on at once: a copy from pageable memory waits for
+// the stream to reach it, and the tables of a large build are made while the
+// device works on the phase before.
+int upload_async(ptbgpu_ctx *ctx, void *dst, const void *src, size_t bytes);
 // Named pinned host buffer of at least `bytes`.
 void *hws(ptbgpu_ctx *ctx, const char *name, size_t bytes);
 // Copies between pageable host memory and the device, on the context's

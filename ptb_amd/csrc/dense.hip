@@ -1258,10 +1258,9 @@ int TileList::upload(ptbgpu_ctx *ctx, const char *name_in) {
     const size_t bytes = sizeof(GemmTile) * work.size();
     void *d = ws(ctx, name, bytes);
     if (!d) return PTBGPU_E_NOMEM;
-    if (hipMemcpyAsync(d, work.data(), bytes, hipMemcpyHostToDevice, ctx->stream) != hipSuccess) {
+    if (const int rc = upload_async(ctx, d, work.data(), bytes); rc != PTBGPU_OK) {
         ctx->shadow.erase(name);
-        return fail(ctx, PTBGPU_E_HIP, "upload of tile list '%s' failed: %s", name,
-                    hipGetErrorString(hipGetLastError()));
+        return rc;
     }
     ctx->shadow[name].assign(sb, sb + sn);
     ctx->shadow[mkey] = meta;
