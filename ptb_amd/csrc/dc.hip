@@ -177,11 +177,11 @@ __device__ __forceinline__ double rcp64(double x) {
     return fma(r, e, r);
 }
 
-// Lanes that share a root or a Loewner entry of a node of kLanesMin rows or more
-// (a thread's chain of O(K) terms is an eighth as long).  The number depends on the
-// node alone, so a density does not depend on what else is in the batch.  Merges of
-// 512 rows and more of the 512-water box 4.9 -> 4.5 ms, of 256 to 511 3.2 -> 2.8.
-constexpr int kRootLanes = 8, kLanesMin = 256;
+// Lanes that share a root or a Loewner entry: a thread's chain of O(K) terms is an
+// eighth as long, and fewer roots wait for the slowest of their wavefront.  The
+// merges of the 512-water box took 1-4 % less with eight than with one (in
+// workgroups too few to be latency-bound), the roots of 8 waters 0.38 -> 0.10 ms.
+constexpr int kRootLanes = 8;
 template <int CTRL>
 __device__ __forceinline__ double dpp_mov(double v) {
     const long long b = __double_as_longlong(v);
@@ -200,54 +200,29 @@ __device__ __forceinline__ double group_reduce(double v, F op) {
 
 // s = sum_{i0 <= i < i1} q_i, ds = sum q_i r_i with r_i = 1 / ((d_i - dorg) - t),
 // q_i = w2_i r_i: the secular function's pole terms and their derivatives.
-// Four interleaved partial sums, so that the terms' dependent chains
-// (reciprocal, Newton steps, accumulation) overlap.  L = 8: lane l of a group of
-// eight takes every eighth term (two partial sums), and every lane gets the sums.
-template <int L>
+// Lane l of a group of kRootLanes takes every eighth term, in two interleaved
+// partial sums (the terms' dependent chains of reciprocal, Newton steps and
+// accumulation overlap); every lane gets the sums.
 __device__ __forceinline__ void secular_sums(const double *dl, const double *w2, int i0, int i1,
                                              double dorg, double t, int l, double &s, double &ds) {
-    if constexpr (L == kRootLanes) {
-        double a0 = 0.0, a1 = 0.0, b0 = 0.0, b1 = 0.0;
-        int i = i0 + l;
-        for (; i + L < i1; i += 2 * L) {
-            const double r0 = rcp64((dl[i] - dorg) - t), r1 = rcp64((dl[i + L] - dorg) - t);
-            const double q0 = w2[i] * r0, q1 = w2[i + L] * r1;
-            a0 += q0;
-            a1 += q1;
-            b0 += q0 * r0;
-            b1 += q1 * r1;
-        }
-        if (i < i1) {
-            const double r = rcp64((dl[i] - dorg) - t), q = w2[i] * r;
-            a0 += q;
-            b0 += q * r;
-        }
-        s = group_reduce(a0 + a1, [](double x, double y) { return x + y; });
-        ds = group_reduce(b0 + b1, [](double x, double y) { return x + y; });
-        return;
-    }
-    double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0, b0 = 0.0, b1 = 0.0, b2 = 0.0, b3 = 0.0;
-    int i = i0;
-    for (; i + 4 <= i1; i += 4) {
-        const double r0 = rcp64((dl[i] - dorg) - t), r1 = rcp64((dl[i + 1] - dorg) - t);
-        const double r2 = rcp64((dl[i + 2] - dorg) - t), r3 = rcp64((dl[i + 3] - dorg) - t);
-        const double q0 = w2[i] * r0, q1 = w2[i + 1] * r1, q2 = w2[i + 2] * r2, q3 = w2[i + 3] * r3;
+    constexpr int L = kRootLanes;
+    double a0 = 0.0, a1 = 0.0, b0 = 0.0, b1 = 0.0;
+    int i = i0 + l;
+    for (; i + L < i1; i += 2 * L) {
+        const double r0 = rcp64((dl[i] - dorg) - t), r1 = rcp64((dl[i + L] - dorg) - t);
+        const double q0 = w2[i] * r0, q1 = w2[i + L] * r1;
         a0 += q0;
         a1 += q1;
-        a2 += q2;
-        a3 += q3;
         b0 += q0 * r0;
         b1 += q1 * r1;
-        b2 += q2 * r2;
-        b3 += q3 * r3;
     }
-    for (; i < i1; ++i) {
+    if (i < i1) {
         const double r = rcp64((dl[i] - dorg) - t), q = w2[i] * r;
         a0 += q;
         b0 += q * r;
     }
-    s = (a0 + a1) + (a2 + a3);
-    ds = (b0 + b1) + (b2 + b3);
+    s = group_reduce(a0 + a1, [](double x, double y) { return x + y; });
+    ds = group_reduce(b0 + b1, [](double x, double y) { return x + y; });
 }
 
 // dst(wb:we) = src(wb:we) for one column by one wavefront, 8 loads in flight
@@ -272,17 +247,16 @@ __device__ __forceinline__ void copy_column(double *__restrict__ dst,
 }
 
 // Secular root j of a merge with K poles dl (ascending), weights w and
-// w2 = rho w^2: the root's origin pole org[j] and offset tau[j].  One thread, or
-// a group of L lanes (l this one's) in step.
-template <int L>
+// w2 = rho w^2: the root's origin pole org[j] and offset tau[j], by a group of
+// kRootLanes lanes (l this one's) in step.
 __device__ void dc_root(int j, int K, const double *dl, const double *w2, const double *w,
-                        double rho, int *org, double *tau, int l = 0) {
+                        double rho, int *org, double *tau, int l) {
     int o;
     double lo, hi;
     if (j < K - 1) {
         const double mid = 0.5 * (dl[j + 1] - dl[j]);
         double fs, fds;
-        secular_sums<L>(dl, w2, 0, K, dl[j], mid, l, fs, fds);
+        secular_sums(dl, w2, 0, K, dl[j], mid, l, fs, fds);
         const double f = 1.0 + fs;
         if (f >= 0.0) {
             o = j;
@@ -296,8 +270,8 @@ __device__ void dc_root(int j, int K, const double *dl, const double *w2, const 
     } else {
         o = j;
         double s2 = 0.0;
-        for (int i = l; i < K; i += L) s2 += w[i] * w[i];
-        if constexpr (L > 1) s2 = group_reduce(s2, [](double x, double y) { return x + y; });
+        for (int i = l; i < K; i += kRootLanes) s2 += w[i] * w[i];
+        s2 = group_reduce(s2, [](double x, double y) { return x + y; });
         lo = 0.0;
         hi = rho * s2;
     }
@@ -315,8 +289,8 @@ __device__ void dc_root(int j, int K, const double *dl, const double *w2, const 
     double t = 0.5 * (lo + hi);
     for (int it = 0; it < 200; ++it) {
         double psi, dpsi, phi, dphi;
-        secular_sums<L>(dl, w2, 0, j + 1, dorg, t, l, psi, dpsi);
-        secular_sums<L>(dl, w2, j + 1, K, dorg, t, l, phi, dphi);
+        secular_sums(dl, w2, 0, j + 1, dorg, t, l, psi, dpsi);
+        secular_sums(dl, w2, j + 1, K, dorg, t, l, phi, dphi);
         const double f = 1.0 + psi + phi;
         if (f == 0.0 || fabs(f) <= 8.0 * kEps * (double)K * (1.0 + fabs(psi) + fabs(phi))) {
             lo = hi = t;
@@ -359,18 +333,17 @@ __device__ void dc_root(int j, int K, const double *dl, const double *w2, const 
 }
 
 // Loewner vector entry i: rho zhat_i^2 = (lam_i - d_i) prod_{j != i} (lam_j - d_i)/(d_j - d_i)
-// (by one thread, or by a group of L lanes, l this one's)
-template <int L>
+// (by a group of kRootLanes lanes, l this one's)
 __device__ double dc_loewner(int i, int K, const double *dl, const int *org, const double *tau,
-                             const double *w, double rho, int l = 0) {
+                             const double *w, double rho, int l) {
     const double di = dl[i];
     double prod = l == 0 ? -((di - dl[org[i]]) - tau[i]) : 1.0;
-    for (int j = l; j < K; j += L) {
+    for (int j = l; j < K; j += kRootLanes) {
         if (j == i) continue;
         const double dlt = (di - dl[org[j]]) - tau[j];  // d_i - lam_j
         prod *= (-dlt) * rcp64(dl[j] - di);
     }
-    if constexpr (L > 1) prod = group_reduce(prod, [](double x, double y) { return x * y; });
+    prod = group_reduce(prod, [](double x, double y) { return x * y; });
     return copysign(sqrt(fmax(prod, 0.0) / rho), w[i]);
 }
 
@@ -744,22 +717,16 @@ __global__ __launch_bounds__(NT) void k_dc_merge(const SubDesc *__restrict__ des
         if (threadIdx.x == 0) gK[4 * blockIdx.x] = K;
     if constexpr (MODE != kDcLds) return;
     __syncthreads();
-    // secular roots, one thread or kRootLanes lanes per root
+    // secular roots
     const int rl = threadIdx.x % kRootLanes;
-    if (n >= kLanesMin)
-        for (int j = threadIdx.x / kRootLanes; j < K; j += NT / kRootLanes)
-            dc_root<kRootLanes>(j, K, dl, zh, w, rho, org, tau, rl);
-    else
-        for (int j = threadIdx.x; j < K; j += NT) dc_root<1>(j, K, dl, zh, w, rho, org, tau);
+    for (int j = threadIdx.x / kRootLanes; j < K; j += NT / kRootLanes)
+        dc_root(j, K, dl, zh, w, rho, org, tau, rl);
     __syncthreads();
     // Loewner vector: rho zhat_i^2 = (lam_i - d_i) prod_{j != i} (lam_j - d_i)/(d_j - d_i)
-    if (n >= kLanesMin)
-        for (int i = threadIdx.x / kRootLanes; i < K; i += NT / kRootLanes) {
-            const double v = dc_loewner<kRootLanes>(i, K, dl, org, tau, w, rho, rl);
-            if (rl == 0) zh[i] = v;
-        }
-    else
-        for (int i = threadIdx.x; i < K; i += NT) zh[i] = dc_loewner<1>(i, K, dl, org, tau, w, rho);
+    for (int i = threadIdx.x / kRootLanes; i < K; i += NT / kRootLanes) {
+        const double v = dc_loewner(i, K, dl, org, tau, w, rho, rl);
+        if (rl == 0) zh[i] = v;
+    }
     __syncthreads();
     // U(:, j) = zhat ./ (d - lam_j), normalised; eigenvalues lam_j.  One
     // column per wavefront: its norm, then the column (lanes on rows).
@@ -777,7 +744,7 @@ struct BigNode {
     double *zh;
     int *org, *prow;
     double rho;
-    int K, n;
+    int K;
 };
 
 __device__ BigNode big_node(const SubDesc *desc, const DcNode *nodes, int npow,
@@ -795,7 +762,6 @@ __device__ BigNode big_node(const SubDesc *desc, const DcNode *nodes, int npow,
     g.prow = ib + 3 * (size_t)npow;
     g.rho = 2.0 * fabs(e_all[ds.mapoff + nd.sp - 1]);
     g.K = gK[4 * (size_t)node];
-    g.n = nd.hi - nd.lo;
     return g;
 }
 
@@ -830,15 +796,9 @@ __global__ __launch_bounds__(kMT) void k_dc_roots_columns(const SubDesc *__restr
     const int node = blockIdx.y;
     if ((int)blockIdx.x < nroot) {
         BigNode g = big_node(desc, nodes, npow, e_all, gscr, gK, node);
-        double *tau = const_cast<double *>(g.tau);
-        if (g.n >= kLanesMin) {
-            const int j = blockIdx.x * kRootsPerBlock + threadIdx.x / kRootLanes;
-            if (j < g.K)
-                dc_root<kRootLanes>(j, g.K, g.dl, g.zh, g.w, g.rho, g.org, tau, threadIdx.x % kRootLanes);
-        } else {
-            const int j = blockIdx.x * kMT + threadIdx.x;
-            if (j < g.K) dc_root<1>(j, g.K, g.dl, g.zh, g.w, g.rho, g.org, tau);
-        }
+        const int j = blockIdx.x * kRootsPerBlock + threadIdx.x / kRootLanes;
+        if (j < g.K)
+            dc_root(j, g.K, g.dl, g.zh, g.w, g.rho, g.org, const_cast<double *>(g.tau), threadIdx.x % kRootLanes);
         return;
     }
     const int lane = threadIdx.x % PTB_WAVE, wid = threadIdx.x / PTB_WAVE;
@@ -870,16 +830,10 @@ __global__ __launch_bounds__(kMT) void k_dc_loewner_deflated(const SubDesc *__re
     const int node = blockIdx.y;
     if ((int)blockIdx.x < nroot) {
         BigNode g = big_node(desc, nodes, npow, e_all, gscr, gK, node);
-        if (g.n >= kLanesMin) {
-            const int i = blockIdx.x * kRootsPerBlock + threadIdx.x / kRootLanes;
-            if (i >= g.K) return;
-            const double v =
-                dc_loewner<kRootLanes>(i, g.K, g.dl, g.org, g.tau, g.w, g.rho, threadIdx.x % kRootLanes);
-            if (threadIdx.x % kRootLanes == 0) g.zh[i] = v;
-        } else {
-            const int i = blockIdx.x * kMT + threadIdx.x;
-            if (i < g.K) g.zh[i] = dc_loewner<1>(i, g.K, g.dl, g.org, g.tau, g.w, g.rho);
-        }
+        const int i = blockIdx.x * kRootsPerBlock + threadIdx.x / kRootLanes;
+        if (i >= g.K) return;
+        const double v = dc_loewner(i, g.K, g.dl, g.org, g.tau, g.w, g.rho, threadIdx.x % kRootLanes);
+        if (threadIdx.x % kRootLanes == 0) g.zh[i] = v;
         return;
     }
     const int K = gK[4 * node], n = gK[4 * node + 1], nr = gK[4 * node + 2];
@@ -963,7 +917,7 @@ int dc_merge_level(ptbgpu_ctx *ctx, const SubDesc *ddesc, const DcNode *dnodes, 
             // phases while the others idle or finish early, so only the front of the
             // merge stays one workgroup per node (all merges of one 1472-row matrix
             // 4.9 ms in one workgroup each, 1.2 so; of 24 submatrices of 8 waters
-            // 0.81 and 0.52; a level of 192 nodes up to 811 rows 1.4 and 0.75)
+            // 0.81 and 0.23)
             // (np bounds the rows of every node of the run)
             const int nroot = (np + kRootsPerBlock - 1) / kRootsPerBlock;
             const bool spread = in_lds(np) && ctx->dc_global_min == 0 && i1 - i0 <= ctx->num_cus;

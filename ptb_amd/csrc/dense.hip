@@ -402,9 +402,8 @@ __global__ __launch_bounds__(kT, sizeof(T) == 4 ? 6 : 4) void k_gemm_nt1(
 // through scalar registers, no barrier) while the others load their rows below;
 // these are then solved by substitution, a thread per row, the factor read from
 // LDS (one address per wavefront).  With four wavefronts and three barriers per
-// column, the block's inverse and X = P L_kk^-T by it: 55 us for the rows below and
-// 21 for the block of one 1472-row matrix, now 23 and 5; a panel of the 512-water
-// box 120 us, now 71.
+// column, the block's inverse and X = P L_kk^-T by it, a panel of one 1472-row
+// matrix (modes 1 and 2) took 76 us, now 28; one of the 512-water box 120, now 71.
 //
 // mode 0: the whole panel (grid (submatrix, 1)).  For few submatrices the
 // panel is split: mode 1 forms the rows below the diagonal block, sliced over
