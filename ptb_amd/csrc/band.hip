@@ -45,7 +45,8 @@ constexpr int kABL = kBW + 1;    // doubles per column of the band buffer
 struct BandSub {
     int64_t off;   // matrix block in the arena
     int64_t pw;    // panel buffers by rows (ld x 16 each): V of even and odd panels, W, X; T (256)
-    int64_t px;    // parts of X: a 64 x 16 block per tile, then one per unit of k_band_step
+    int64_t px;    // parts of X: a 64 x 16 block per tile, then one per unit of k_band_step;
+                   // parts of V^T X: 1024 per strip
     int64_t ab;    // band: column c at ab + 17 c, element d below the diagonal at + d
     int64_t blk;   // first block of its Q2 reflectors
     int m, ld, mapoff, ng;  // ng sweep groups
@@ -303,6 +304,11 @@ __host__ __device__ inline int band_units(int ns) {  // of ns strips
     const int a = ns / kChunk;
     return 2 * a * (a + 1) + (ns - kChunk * a) * (a + 1);
 }
+// where a submatrix's parts of V^T X (1024 per strip) begin in its part buffer
+__host__ __device__ inline int64_t gram_at(int m) {
+    const int64_t ns = m > kBW ? (m - kBW + 63) / 64 : 0;
+    return 1024 * (ns * (ns + 1) / 2 + band_units((int)ns));
+}
 __device__ inline int band_unit(int i, int q) { return band_units(i) + q; }
 
 // One pass over the lower triangle of the trailing matrix (rows and columns from
@@ -503,16 +509,19 @@ __global__ __launch_bounds__(256, 3) void k_band_step(const BandSub *__restrict_
 }
 
 // X (by rows) of one 64-row strip from its parts: the strip's own chunks, then
-// the tiles below it in its columns, in order.  grid: (submatrix, strip)
+// the tiles below it in its columns, in order; SPLIT: and the strip's parts of
+// V^T X, one of 16 rows per wavefront, behind the parts of X.
+// grid: (submatrix, strip)
+template <bool SPLIT>
 __global__ __launch_bounds__(256) void k_band_x(const BandSub *__restrict__ subs,
-                                                const double *__restrict__ PXa, double *__restrict__ PW,
+                                                double *__restrict__ PXa, double *__restrict__ PW,
                                                 int panel) {
     const BandSub d = subs[blockIdx.x];
     const int r0 = panel * kBW + kBW;
     const int n = d.m - r0, i = blockIdx.y;
     if (n < 2 || 64 * i >= n) return;
     const int ns = (n + 63) / 64, ns0 = (d.m - kBW + 63) / 64;
-    const double *px = PXa + d.px;
+    double *px = PXa + d.px;
     const double *own = px + (int64_t)(ns0 * (ns0 + 1) / 2 + band_unit(i, 0)) * 1024;
     const int nq = i / kChunk + 1;
     double *x = PW + d.pw + (int64_t)48 * d.ld + (int64_t)(r0 + 64 * i) * kBW;
@@ -529,49 +538,85 @@ __global__ __launch_bounds__(256) void k_band_x(const BandSub *__restrict__ subs
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
         const int l = threadIdx.x + 256 * e;
-        if (l < 16 * rows) x[l] = 64 * i + (l >> 4) < n ? s[e] : 0.0;
+        s[e] = 64 * i + (l >> 4) < n ? s[e] : 0.0;
+        if (l < 16 * rows) x[l] = s[e];
     }
+    if constexpr (!SPLIT) return;
+    __shared__ double xs[1024];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) xs[threadIdx.x + 256 * e] = s[e];
+    __syncthreads();
+    const int lane = threadIdx.x % PTB_WAVE, wave = threadIdx.x / PTB_WAVE;
+    const int lr = lane & 15, g = lane >> 4, k = 64 * i + 16 * wave;
+    d4_t acc = d4_t{0.0, 0.0, 0.0, 0.0};
+    if (k < n) {  // (V is zero up to the next multiple of 16 rows)
+        const double *vr = PW + d.pw + (int64_t)(panel & 1) * 16 * d.ld + (int64_t)(r0 + k) * kBW;
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            acc = __builtin_amdgcn_mfma_f64_16x16x4f64(vr[(4 * u + g) * kBW + lr],
+                                                       xs[(16 * wave + 4 * u + g) * kBW + lr], acc, 0, 0, 0);
+    }
+    double *gp = px + gram_at(d.m) + 1024 * i + 256 * wave;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) gp[(4 * r + g) * kBW + lr] = acc[r];
 }
 
 // W = X T - V S, S = T^T (V^T X) T / 2, by rows, and the panel's update
 // A -= V W^T + W V^T on the next 16 columns (rows and columns from r0 on), which
-// the next panel's QR reads.  One workgroup per submatrix: V^T X on the matrix
-// cores (wavefronts on alternate 16-row tiles), the 16 x 16 products in LDS, then
-// W^T and the columns tile by tile (lane = row; W^T's result layout is the operand
-// layout of the update).
+// the next panel's QR reads: V^T X on the matrix cores (wavefronts on alternate
+// 16-row tiles, a sum of tile products each), the 16 x 16 products in LDS, then W^T
+// and the columns tile by tile (lane = row; W^T's result layout is the operand
+// layout of the update).  One workgroup per submatrix, or (SPLIT) one per strip of
+// 64 rows, each adding up the parts of V^T X that k_band_x left, in the same order:
+// the same bits.  SPLIT serves panels of no more submatrices than CUs (one of
+// 1472 rows 27 us with k_band_x -> 14, 192 of 64 waters 24 -> 20); beyond that the
+// parts cost more than the second workgroup gains (256 molecules: 328 us -> 393).
+template <bool SPLIT>
 __global__ __launch_bounds__(256) void k_band_w(const BandSub *__restrict__ subs,
                                                 double *__restrict__ Aa, double *__restrict__ PW,
-                                                int panel) {
+                                                const double *__restrict__ PXa, int panel) {
     const BandSub d = subs[blockIdx.x];
     const int r0 = panel * kBW + kBW;
     const int n = d.m - r0;
-    if (n < 2) return;
+    if (n < 2 || 64 * (int)blockIdx.y >= n) return;
     double *pw = PW + d.pw;
     const double *vr = pw + (int64_t)(panel & 1) * 16 * d.ld + (int64_t)r0 * kBW;
     double *wr = pw + (int64_t)32 * d.ld + (int64_t)r0 * kBW;
     const double *xr = pw + (int64_t)48 * d.ld + (int64_t)r0 * kBW;
     const double *T = pw + (int64_t)64 * d.ld;
     double *a = Aa + d.off + (int64_t)r0 * d.ld + r0;
-    __shared__ double gs[4][16][17], ts[16][17], ms[16][17], ss[16][17];
+    __shared__ double gs[SPLIT ? 1 : 4][16][17], ts[16][17], ms[16][17], ss[16][17];
     const int lane = threadIdx.x % PTB_WAVE, wave = threadIdx.x / PTB_WAVE;
     const int lr = lane & 15, g = lane >> 4;
-    d4_t acc = d4_t{0.0, 0.0, 0.0, 0.0};
-    for (int k = 16 * wave; k < n; k += 64) {
-        double av[4], bv[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            av[u] = vr[(unsigned)(k + 4 * u + g) * kBW + lr];
-            bv[u] = xr[(unsigned)(k + 4 * u + g) * kBW + lr];
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(av[u], bv[u], acc, 0, 0, 0);
-    }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) gs[wave][4 * r + g][lr] = acc[r];
     const int ti = threadIdx.x & 15, tj = threadIdx.x >> 4;
     ts[ti][tj] = T[tj * kBW + ti];
-    __syncthreads();
-    ss[ti][tj] = ((gs[0][ti][tj] + gs[1][ti][tj]) + gs[2][ti][tj]) + gs[3][ti][tj];
+    if constexpr (SPLIT) {
+        const double *gp = PXa + d.px + gram_at(d.m) + threadIdx.x;
+        double s[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 4
+        for (int i = 0; i < (n + 63) / 64; ++i)
+#pragma unroll
+            for (int w = 0; w < 4; ++w) s[w] += gp[1024 * i + 256 * w];
+        ss[tj][ti] = ((s[0] + s[1]) + s[2]) + s[3];
+    } else {
+        d4_t sum = d4_t{0.0, 0.0, 0.0, 0.0};
+        for (int k = 16 * wave; k < n; k += 64) {
+            double av[4], bv[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                av[u] = vr[(unsigned)(k + 4 * u + g) * kBW + lr];
+                bv[u] = xr[(unsigned)(k + 4 * u + g) * kBW + lr];
+            }
+            d4_t acc = d4_t{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+            for (int u = 0; u < 4; ++u) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(av[u], bv[u], acc, 0, 0, 0);
+            sum += acc;
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) gs[wave][4 * r + g][lr] = sum[r];
+        __syncthreads();
+        ss[ti][tj] = ((gs[0][ti][tj] + gs[1][ti][tj]) + gs[2][ti][tj]) + gs[3][ti][tj];
+    }
     __syncthreads();
     {
         double s = 0.0;  // M = G T
@@ -612,7 +657,7 @@ __global__ __launch_bounds__(256) void k_band_w(const BandSub *__restrict__ subs
     // rows r0 .. r0 + 15 of V and W, the update's column operands
     double v0[4];
     const d4_t w0 = make_w(0, v0);
-    for (int k = 16 * wave; k < n; k += 64) {
+    for (int k = 64 * blockIdx.y + 16 * wave; k < n; k += 64 * gridDim.y) {
         const int row = k + lr;
         d4_t t;
 #pragma unroll
@@ -1222,7 +1267,7 @@ int64_t band_blocks(int m) {
 
 int64_t band_parts(int m) {
     const int64_t ns = m > kBW ? (m - kBW + 63) / 64 : 0;
-    return 1024 * (ns * (ns + 1) / 2 + band_units((int)ns));
+    return gram_at(m) + 1024 * ns;
 }
 
 int sytrd_band(ptbgpu_ctx *ctx, const std::vector<SubDesc> &desc, double *A, double *d, double *e,
@@ -1286,6 +1331,7 @@ int sytrd_band(ptbgpu_ctx *ctx, const std::vector<SubDesc> &desc, double *A, dou
                 PTB_CHECK_LAUNCH(ctx);
             }
             const int ns = (n + 63) / 64;
+            const bool split = na <= ctx->num_cus;
             {
                 ProfScope kprof_(ctx, "band_step");
                 const int nunit = band_units(ns);
@@ -1298,12 +1344,13 @@ int sytrd_band(ptbgpu_ctx *ctx, const std::vector<SubDesc> &desc, double *A, dou
             }
             {
                 ProfScope kprof_(ctx, "band_x");
-                hipLaunchKernelGGL(k_band_x, dim3(na, ns), dim3(256), 0, st, ds, PX, PW, p);
+                hipLaunchKernelGGL(split ? k_band_x<true> : k_band_x<false>, dim3(na, ns), dim3(256), 0, st, ds, PX, PW, p);
                 PTB_CHECK_LAUNCH(ctx);
             }
             {
                 ProfScope kprof_(ctx, "band_w");
-                hipLaunchKernelGGL(k_band_w, dim3(na), dim3(256), 0, st, ds, A, PW, p);
+                hipLaunchKernelGGL(split ? k_band_w<true> : k_band_w<false>, dim3(na, split ? ns : 1), dim3(256), 0, st, ds,
+                                   A, PW, PX, p);
                 PTB_CHECK_LAUNCH(ctx);
             }
         }
