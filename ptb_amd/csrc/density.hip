@@ -70,6 +70,7 @@ __global__ __launch_bounds__(kT) void k_fe_proj(const SubDesc *__restrict__ desc
     const double *f = F + xoff[blockIdx.x] + k;
     double s = 0.0;
     if (!(d.flags & 1))
+#pragma unroll 8
         for (int g = 0; g < c; ++g) s += f[(int64_t)g * d.ld] * f[(int64_t)(c + g) * d.ld];
     fe_all[d.mapoff + k] = s;
 }
@@ -115,32 +116,24 @@ __global__ __launch_bounds__(kT) void k_nel_partial(const double *__restrict__ e
     }
 }
 
-// One pass, part 2 (one thread per molecule): nel = the partials summed in
-// fixed order, then the reference's step (source/sm.f90:365-383): a pass after
-// convergence is the final one (its nel is reported); otherwise log (mu, nel),
+// The reference's step after a pass that gave nel (source/sm.f90:365-383): a pass
+// after convergence is the final one (its nel is reported); otherwise log (mu, nel),
 // test |mua-mub| < 1e-3 or |nel-nelref| < 1e-5 (REAL(4) literals), move the
 // bracket and bisect.  At most 100 passes, as the reference's loop.
-// out (per molecule, kBisStride): [0] mu, [1] nel, [2] logged passes,
-// [3] converged, then (mu, nel) of every logged pass.
-__global__ void k_bisect_step(BisState *__restrict__ st, const double *__restrict__ partial,
-                              int nblk, const int64_t *__restrict__ nelref, int nmol,
-                              double *__restrict__ out_all, int *__restrict__ ndone) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nmol) return;
-    BisState s = st[i];
-    if (s.done) return;
+// out (per molecule, kBisStride; NULL: not written): [0] mu, [1] nel, [2] logged
+// passes, [3] converged, then (mu, nel) of every logged pass.
+// True when that was the last pass.
+__device__ __forceinline__ bool bisect_next(BisState &s, double nel, double ref, double *out) {
     const float tol_mu = 1e-3f, tol_nel = 1e-5f;  // REAL(4) literals of the reference
-    double *out = out_all + (size_t)i * kBisStride;
-    double nel = 0.0;
-    for (int b = 0; b < nblk; ++b) nel += partial[(int64_t)i * nblk + b];
-    const double ref = (double)nelref[i];
     s.iter += 1;
     bool finish = false;
     if (s.finaliter) {
         finish = true;
     } else {
-        out[4 + 2 * s.logged] = s.mu;
-        out[5 + 2 * s.logged] = nel;
+        if (out) {
+            out[4 + 2 * s.logged] = s.mu;
+            out[5 + 2 * s.logged] = nel;
+        }
         s.logged += 1;
         if (fabs(s.mua - s.mub) < (double)tol_mu || fabs(nel - ref) < (double)tol_nel) {
             s.finaliter = 1;
@@ -152,23 +145,81 @@ __global__ void k_bisect_step(BisState *__restrict__ st, const double *__restric
         finish = s.iter >= 100;
     }
     if (finish) {
-        out[0] = s.mu;
-        out[1] = nel;
-        out[2] = (double)s.logged;
-        out[3] = s.finaliter ? 1.0 : 0.0;
+        if (out) {
+            out[0] = s.mu;
+            out[1] = nel;
+            out[2] = (double)s.logged;
+            out[3] = s.finaliter ? 1.0 : 0.0;
+        }
         s.done = 1;
-        atomicAdd(ndone, 1);
     } else {
         s.mu = (s.mua + s.mub) / 2.0;
     }
+    return finish;
+}
+
+// One pass, part 2 (one thread per molecule): nel = the partials summed in
+// fixed order, then the reference's step.
+__global__ void k_bisect_step(BisState *__restrict__ st, const double *__restrict__ partial,
+                              int nblk, const int64_t *__restrict__ nelref, int nmol,
+                              double *__restrict__ out_all, int *__restrict__ ndone) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= nmol) return;
+    BisState s = st[i];
+    if (s.done) return;
+    double nel = 0.0;
+    for (int b = 0; b < nblk; ++b) nel += partial[(int64_t)i * nblk + b];
+    if (bisect_next(s, nel, (double)nelref[i], out_all + (size_t)i * kBisStride)) atomicAdd(ndone, 1);
     st[i] = s;
+}
+
+// The whole bisection of molecules of at most kBisRows states, a workgroup each:
+// the states stay in its registers, and a pass costs a reduction instead of two
+// launches (8 waters: 48 launches of 2.5 us and the host's wait for them).  The
+// sums are those of k_nel_partial with one chunk.
+constexpr int kBisRows = 4096;
+__global__ __launch_bounds__(kT) void k_bisect_whole(const double *__restrict__ e,
+                                                     const double *__restrict__ fe,
+                                                     const int64_t *__restrict__ rbeg,
+                                                     const int64_t *__restrict__ nelref,
+                                                     double *__restrict__ out_all) {
+    constexpr int kN = kBisRows / kT;
+    __shared__ double red[kT / PTB_WAVE];
+    const int i = blockIdx.x;
+    const int64_t lo = rbeg[i], n = rbeg[i + 1] - lo;
+    double ev[kN], fv[kN];
+#pragma unroll
+    for (int q = 0; q < kN; ++q) {
+        const int64_t k = threadIdx.x + (int64_t)kT * q;
+        const bool in = k < n;
+        ev[q] = in ? e[lo + k] : 0.0;
+        fv[q] = in ? fe[lo + k] : 0.0;
+    }
+    const double ref = (double)nelref[i];
+    double *out = threadIdx.x == 0 ? out_all + (size_t)i * kBisStride : nullptr;
+    BisState s{-10.0, 10.0, 0.0, 0, 0, 0, 0};
+    for (int pass = 0; pass < 101; ++pass) {
+        double part = 0.0;
+#pragma unroll
+        for (int q = 0; q < kN; ++q) {
+            if (threadIdx.x + (int64_t)kT * q < n) part += fv[q] * occ_of(ev[q], s.mu);
+        }
+        part = wave_sum(part);
+        if (threadIdx.x % PTB_WAVE == 0) red[threadIdx.x / PTB_WAVE] = part;
+        __syncthreads();
+        double nel = 0.0;
+        for (int w = 0; w < kT / PTB_WAVE; ++w) nel += red[w];
+        __syncthreads();
+        if (bisect_next(s, nel, ref, out)) break;
+    }
 }
 
 // Occupied states of each submatrix at the final mu, in ascending state
 // order: weights occ(e_k) (2, or 1 for e_k == mu) into wocc at the submatrix's
 // row offset, their count into nocc, and the eigenvector columns Z(:, k) copied
-// to the first nocc columns of Zo.  One workgroup per submatrix; a submatrix
-// whose overlap block failed the Cholesky contributes no states.
+// to the first nocc columns of Zo, a column per wavefront.  grid: (submatrix,
+// slices of its columns; each finds the states for itself); a submatrix whose
+// overlap block failed the Cholesky contributes no states.
 __global__ __launch_bounds__(kT) void k_occ_compact(const SubDesc *__restrict__ desc,
                                                     const double *__restrict__ eig_all,
                                                     const double *__restrict__ mu_p,
@@ -197,8 +248,10 @@ __global__ __launch_bounds__(kT) void k_occ_compact(const SubDesc *__restrict__ 
         for (int q = 0; q < wid; ++q) off += wtot[q];
         if (w != 0.0) {
             occk[off + before] = k;
-            wocc[d.mapoff + off + before] = w;
-            if (oidx) oidx[d.mapoff + off + before] = k;
+            if (blockIdx.y == 0) {
+                wocc[d.mapoff + off + before] = w;
+                if (oidx) oidx[d.mapoff + off + before] = k;
+            }
         }
         __syncthreads();
         if (threadIdx.x == 0) {
@@ -209,13 +262,15 @@ __global__ __launch_bounds__(kT) void k_occ_compact(const SubDesc *__restrict__ 
         __syncthreads();
     }
     const int n = base;
-    if (threadIdx.x == 0) nocc[blockIdx.x] = n;
+    if (threadIdx.x == 0 && blockIdx.y == 0) nocc[blockIdx.x] = n;
     const double *Z = Za + d.off;
     double *Y = Zo + d.off;
-    for (int t = 0; t < n; ++t) {
+    constexpr int kW = kT / PTB_WAVE;
+    for (int t = kW * blockIdx.y + wid; t < n; t += kW * gridDim.y) {
         const double *src = Z + (int64_t)occk[t] * d.ld;
         double *dst = Y + (int64_t)t * d.ld;
-        for (int r = threadIdx.x; r < d.m; r += kT) dst[r] = src[r];
+#pragma unroll 4
+        for (int r = lane; r < d.m; r += PTB_WAVE) dst[r] = src[r];
     }
 }
 
@@ -386,6 +441,11 @@ int fe_proj(ptbgpu_ctx *ctx, const SubDesc *ddesc, int nsm, int max_m, const int
 int bisect_batch(ptbgpu_ctx *ctx, const double *e, const double *fe, const int64_t *drbeg,
                  const int64_t *dnelref, int nmol, int64_t max_rows, double *dout) {
     ProfScope prof_(ctx, "bisect");
+    if (max_rows <= kBisRows) {
+        hipLaunchKernelGGL(k_bisect_whole, dim3(nmol), dim3(kT), 0, ctx->stream, e, fe, drbeg, dnelref, dout);
+        PTB_CHECK_LAUNCH(ctx);
+        return PTBGPU_OK;
+    }
     auto *st = static_cast<BisState *>(ws(ctx, "bis_state", sizeof(BisState) * nmol));
     auto *ndone = static_cast<int *>(ws(ctx, "bis_done", sizeof(int)));
     const int nblk = (int)std::max<int64_t>(1, std::min<int64_t>(256, (max_rows + 4095) / 4096));
@@ -419,7 +479,10 @@ int occ_compact(ptbgpu_ctx *ctx, const SubDesc *ddesc, int nsm, int max_m, const
                 const double *dmu, const double *Z, double *Zo, double *wocc, int *nocc,
                 int *oidx) {
     ProfScope prof_(ctx, "occ_compact");
-    hipLaunchKernelGGL(k_occ_compact, dim3(nsm), dim3(kT), sizeof(int) * (size_t)max_m,
+    // (four workgroups per CU where the submatrices alone are fewer, and a column
+    // per wavefront at least)
+    const int ny = std::max(1, std::min(4 * ctx->num_cus / nsm, (max_m + 7) / 8));
+    hipLaunchKernelGGL(k_occ_compact, dim3(nsm, ny), dim3(kT), sizeof(int) * (size_t)max_m,
                        ctx->stream, ddesc, eig, dmu, Z, Zo, wocc, nocc, oidx);
     PTB_CHECK_LAUNCH(ctx);
     return PTBGPU_OK;

@@ -54,6 +54,7 @@ __global__ __launch_bounds__(kThreads) void k_group_union(const uint32_t *__rest
     for (int64_t w = (int64_t)blockIdx.y * kThreads + threadIdx.x; w < words;
          w += (int64_t)gridDim.y * kThreads) {
         uint32_t acc = 0;
+#pragma unroll 8
         for (int g = g0; g < g1; ++g) acc |= bits[(int64_t)gcols[g] * words + w];
         uni[w] = acc;
         pc += __popc(acc);
