@@ -723,12 +723,51 @@ struct ChaseLds {
     double *vm, *tm, *cm, *bm, *rm, *wsc;
 };
 
+// element c (the same in every lane) of a lane's four, by scalar branches (the empty
+// statements keep them from becoming selects)
+__device__ __forceinline__ void set_slot(double (&A)[4], int c, double v) {
+    if (c == 0) {
+        asm volatile("");
+        A[0] = v;
+    } else if (c == 1) {
+        asm volatile("");
+        A[1] = v;
+    } else if (c == 2) {
+        asm volatile("");
+        A[2] = v;
+    } else {
+        asm volatile("");
+        A[3] = v;
+    }
+}
+__device__ __forceinline__ double get_slot(const double (&A)[4], int c) {
+    double v;
+    if (c == 0) {
+        asm volatile("");
+        v = A[0];
+    } else if (c == 1) {
+        asm volatile("");
+        v = A[1];
+    } else if (c == 2) {
+        asm volatile("");
+        v = A[2];
+    } else {
+        asm volatile("");
+        v = A[3];
+    }
+    return v;
+}
+
 // One step of the chase: window k of sweep s.  A wavefront holds the window's
 // diagonal block D and the block B below it (rows of window k + 1), 16 x 16, in
 // cyclic slots: row or column r sits in slot r mod 16, so moving from sweep s - 1
 // to sweep s replaces one slot and shifts nothing.  Lane l holds row slot l % 16
 // and column slots 4 (l / 16) + c.  f = (s + 1) mod 16 is the slot of every
-// window's first row.
+// window's first row.  BRANCH: slots are replaced under scalar and lane branches, 35
+// vector instructions fewer than selects, where several windows per wavefront keep
+// the CU's issue busy (512-water box 15.2 -> 14.3 ms, 1472 rows 11.6 -> 10.2); a
+// wavefront with one window of each parity waits for the branches instead (4-9 %).
+template <bool BRANCH>
 __device__ __forceinline__ void chase_step(double (&D)[4], double (&B)[4], int k, int s, int m, int ng,
                                            const ChaseLds &L, double *__restrict__ raw,
                                            double *__restrict__ rtau, double *__restrict__ dv,
@@ -741,11 +780,26 @@ __device__ __forceinline__ void chase_step(double (&D)[4], double (&B)[4], int k
         const double cmv = L.cm[(k + 1) * 16 + i], bmv = L.bm[k + 1], rmv = L.rm[k * 16 + i];
         const bool rf = i == fo;
         const double dcol = rf ? cmv : rmv, bcol = rf ? bmv : cmv;
+        if constexpr (BRANCH) {
+            if (rf) {
+                asm volatile("");
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            const bool cc = 4 * g + c == fo;
-            D[c] = cc ? dcol : rf ? B[c] : D[c];
-            B[c] = cc ? bcol : rf ? 0.0 : B[c];
+                for (int c = 0; c < 4; ++c) {
+                    D[c] = B[c];
+                    B[c] = 0.0;
+                }
+            }
+            if (g == fo >> 2) {
+                set_slot(D, fo & 3, dcol);
+                set_slot(B, fo & 3, bcol);
+            }
+        } else {
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const bool cc = 4 * g + c == fo;
+                D[c] = cc ? dcol : rf ? B[c] : D[c];
+                B[c] = cc ? bcol : rf ? 0.0 : B[c];
+            }
         }
     }
     const bool pivot = i == f;
@@ -776,7 +830,13 @@ __device__ __forceinline__ void chase_step(double (&D)[4], double (&B)[4], int k
 #pragma unroll
     for (int c = 0; c < 4; ++c) vc[c] = L.vm[k * 16 + 4 * g + c];
     const int gf = f >> 2, cf = f & 3;
-    const double b0 = cf & 1 ? B[1] : B[0], b1 = cf & 1 ? B[3] : B[2];
+    double bf = 0.0;
+    if constexpr (BRANCH) {
+        if (g == gf) bf = get_slot(B, cf);
+    } else {
+        const double b0 = cf & 1 ? B[1] : B[0], b1 = cf & 1 ? B[3] : B[2];
+        bf = g == gf ? (cf & 2 ? b1 : b0) : 0.0;
+    }
     // p = D v, y = B v and B's first column, by rows
     double p = D[0] * vc[0], y = B[0] * vc[0];
 #pragma unroll
@@ -787,7 +847,7 @@ __device__ __forceinline__ void chase_step(double (&D)[4], double (&B)[4], int k
     p = tau * rows_sum(p);
     y = tau * rows_sum(y);
     // (v is 1 at the pivot, so the column after B <- B H is x = B(:, f) - y)
-    const double x = rows_sum(g == gf ? (cf & 2 ? b1 : b0) : 0.0) - y;
+    const double x = rows_sum(bf) - y;
     const double pv = row_sum(p * vr), sig = row_sum(pivot ? 0.0 : x * x);
     const double w = p - (0.5 * tau * pv) * vr;
     if (g == 0) L.wsc[i] = w;
@@ -806,8 +866,10 @@ __device__ __forceinline__ void chase_step(double (&D)[4], double (&B)[4], int k
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
         const double t = B[c] - u * z[c];
-        B[c] = 4 * g + c == f ? xf : t;
+        B[c] = !BRANCH && 4 * g + c == f ? xf : t;
     }
+    if constexpr (BRANCH)
+        if (g == gf) set_slot(B, cf, xf);
     // D <- H D H
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
@@ -834,27 +896,26 @@ __device__ __forceinline__ void chase_step(double (&D)[4], double (&B)[4], int k
         }
 }
 
-// Bulge chasing of one submatrix by a workgroup of NW wavefronts.  Step (s, k)
+// Bulge chasing of one submatrix by nw wavefronts (this one its `wave`-th).  Step (s, k)
 // needs (s, k - 1) and (s - 1, k + 1), so at time t = 2 s + k all windows of one
 // parity step at once; a barrier ends each time step.  Wavefront w owns the
-// windows 2 w and 2 w + 1 (mod 2 NW), so the work stays even as the band
+// windows 2 w and 2 w + 1 (mod 2 nw), so the work stays even as the band
 // shortens, and ends when they have left it.  P windows per wavefront live in
-// registers (16 VGPRs each), up to 16 NW P rows; MEM: those above that in device
+// registers (16 VGPRs each), up to 16 nw P rows; MEM: those above that in device
 // memory (state), which they need for the first sweeps only.
 // Bound by instruction issue of the CU (about 390 vector instructions a step; with
 // IEEE square root and divisions, and one row sum per column of B, it was 430).
 // One window of each parity per wavefront where 16 hold them: a step's chain is the
 // time step.  512-water box 21.6 -> 17.3 ms, 256 molecules 46.4 -> 32.0, one
 // 1472-row matrix (every window in memory before) 14.0 -> 11.7.
-template <int NW, int P, bool MEM>
-__device__ __forceinline__ void chase(const BandSub &b, double *sm, const double *__restrict__ ABa,
+template <int P, bool MEM>
+__device__ __forceinline__ void chase(const BandSub &b, double *sm, int nw, int wave, const double *__restrict__ ABa,
                                       double *__restrict__ raw_all, double *__restrict__ rtau_all,
                                       double *__restrict__ d_all, double *__restrict__ e_all,
                                       double *__restrict__ state) {
     const int m = b.m;
     const int K = max((m - 1 + kBW - 1) / kBW, 1);  // windows
-    const int lane = threadIdx.x % PTB_WAVE;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PTB_WAVE);
+    const int lane = threadIdx.x % PTB_WAVE, tid = PTB_WAVE * wave + lane, NW = nw;
     ChaseLds L;
     L.vm = sm;
     L.cm = L.vm + 16 * (K + 2);
@@ -863,12 +924,12 @@ __device__ __forceinline__ void chase(const BandSub &b, double *sm, const double
     L.tm = L.rm + 16 * (K + 2) + 16 * NW;
     L.bm = L.tm + (K + 2);
     const double *ab = ABa + b.ab;
-    for (int l = threadIdx.x; l < 16 * (K + 2); l += NW * 64) {
+    for (int l = tid; l < 16 * (K + 2); l += NW * 64) {
         L.vm[l] = 0.0;
         L.rm[l] = 0.0;
         L.cm[l] = l < 16 && l < m ? ab[l] : 0.0;
     }
-    for (int l = threadIdx.x; l < K + 2; l += NW * 64) {
+    for (int l = tid; l < K + 2; l += NW * 64) {
         L.tm[l] = 0.0;
         L.bm[l] = l == 0 && m > kBW ? ab[kBW] : 0.0;
     }
@@ -910,7 +971,7 @@ __device__ __forceinline__ void chase(const BandSub &b, double *sm, const double
 #pragma unroll
             for (int q = par; q < P; q += 2) {
                 const int k = 2 * wave + 2 * NW * (q / 2) + par, s = t - wave - NW * (q / 2);
-                if (active(k, s)) chase_step(D[q], B[q], k, s, m, b.ng, L, raw, rtau, dv, ev, lane);
+                if (active(k, s)) chase_step<P == 4 || MEM>(D[q], B[q], k, s, m, b.ng, L, raw, rtau, dv, ev, lane);
             }
             if constexpr (MEM)
                 for (int j = P / 2; 2 * wave + par + 2 * NW * j < K; ++j) {
@@ -918,7 +979,7 @@ __device__ __forceinline__ void chase(const BandSub &b, double *sm, const double
                     if (!active(k, s)) break;  // (nor are the windows above)
                     const d4_t p0 = stored(k)[0], p1 = stored(k)[1];
                     double Dk[4] = {p0[0], p0[1], p0[2], p0[3]}, Bk[4] = {p1[0], p1[1], p1[2], p1[3]};
-                    chase_step(Dk, Bk, k, s, m, b.ng, L, raw, rtau, dv, ev, lane);
+                    chase_step<true>(Dk, Bk, k, s, m, b.ng, L, raw, rtau, dv, ev, lane);
                     stored(k)[0] = d4_t{Dk[0], Dk[1], Dk[2], Dk[3]};
                     stored(k)[1] = d4_t{Bk[0], Bk[1], Bk[2], Bk[3]};
                 }
@@ -927,32 +988,69 @@ __device__ __forceinline__ void chase(const BandSub &b, double *sm, const double
     }
 }
 
-template <int NW, int P, bool MEM>
-__global__ __launch_bounds__(NW * 64) void k_chase(const BandSub *__restrict__ subs, int first,
-                                                   const double *__restrict__ ABa,
-                                                   double *__restrict__ raw_all,
-                                                   double *__restrict__ rtau_all,
-                                                   double *__restrict__ d_all,
-                                                   double *__restrict__ e_all,
-                                                   double *__restrict__ state) {
-    extern __shared__ double sm[];
-    const BandSub b = subs[first + blockIdx.x];
-    chase<NW, P, MEM>(b, sm, ABa, raw_all, rtau_all, d_all, e_all, state);
+// One workgroup of the chase: the submatrices [first, first + n), 16 / n wavefronts
+// each (P = 2 windows per wavefront, 4 for the ones that need them).
+struct ChaseJob {
+    int first, n, p;
+};
+// doubles of LDS of a submatrix of m rows and nw wavefronts
+__host__ __device__ inline int chase_lds(int m, int nw) {
+    const int K = m > kBW ? (m - 1 + kBW - 1) / kBW : 1;
+    return 50 * (K + 2) + 16 * nw;
 }
 
-// All submatrices of a small batch (a CU each) in one launch, 16 wavefronts each:
-// the size classes overlap (192 submatrices of 64 waters: 5.3 ms one class after
-// the other, 3.4 so); a larger batch fills the chip with each class.
-__global__ __launch_bounds__(1024) void k_chase_few(const BandSub *__restrict__ subs,
+// A small batch (submatrices of up to 1025 rows) in one launch of 16-wavefront
+// workgroups, a CU each, the largest first: 1025 to 514 rows take 16 wavefronts with
+// two windows of each parity, 513 to 258 16 with one, and below that 2, 4 or 8
+// submatrices share a workgroup and its barriers where there are more of them than
+// CUs.  The small ones run beside the large: 64 waters (192 submatrices) 5.3 ms one
+// class after the other, 3.4 so; 621 single columns of 27 waters 2.3 and 1.4.
+__global__ __launch_bounds__(1024) void k_chase(const BandSub *__restrict__ subs,
+                                                const ChaseJob *__restrict__ jobs,
+                                                const double *__restrict__ ABa,
+                                                double *__restrict__ raw_all,
+                                                double *__restrict__ rtau_all,
+                                                double *__restrict__ d_all,
+                                                double *__restrict__ e_all) {
+    extern __shared__ double sm[];
+    const ChaseJob jb = jobs[blockIdx.x];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PTB_WAVE);
+    const int nw = jb.n == 1 ? 16 : jb.n == 2 ? 8 : jb.n <= 4 ? 4 : 2;
+    const int x = wave / nw;
+    if (x >= jb.n) return;
+    const BandSub b = subs[jb.first + x];
+    double *lds = sm + x * chase_lds(subs[jb.first].m, nw);
+    if (jb.p == 4) chase<4, false>(b, lds, 16, wave, ABa, raw_all, rtau_all, d_all, e_all, nullptr);
+    else chase<2, false>(b, lds, nw, wave % nw, ABa, raw_all, rtau_all, d_all, e_all, nullptr);
+}
+
+// One size class of a large batch, a workgroup of NW wavefronts per submatrix: the
+// smaller workgroups start as wavefronts before them end, which a chip full of each
+// class gains more from than from the overlap of classes (256 molecules 32 ms, 40 in
+// k_chase; C400H802 2.5 and 2.8).
+template <int NW, int P>
+__global__ __launch_bounds__(NW * 64) void k_chase_class(const BandSub *__restrict__ subs,
+                                                         const double *__restrict__ ABa,
+                                                         double *__restrict__ raw_all,
+                                                         double *__restrict__ rtau_all,
+                                                         double *__restrict__ d_all,
+                                                         double *__restrict__ e_all) {
+    extern __shared__ double sm[];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PTB_WAVE);
+    chase<P, false>(subs[blockIdx.x], sm, NW, wave, ABa, raw_all, rtau_all, d_all, e_all, nullptr);
+}
+
+// Submatrices of 1026 to 2048 rows, a workgroup of 16 wavefronts each.
+__global__ __launch_bounds__(1024) void k_chase_mem(const BandSub *__restrict__ subs,
                                                     const double *__restrict__ ABa,
                                                     double *__restrict__ raw_all,
                                                     double *__restrict__ rtau_all,
                                                     double *__restrict__ d_all,
-                                                    double *__restrict__ e_all) {
+                                                    double *__restrict__ e_all,
+                                                    double *__restrict__ state) {
     extern __shared__ double sm[];
-    const BandSub b = subs[blockIdx.x];
-    if (b.m > 513) chase<16, 4, false>(b, sm, ABa, raw_all, rtau_all, d_all, e_all, nullptr);
-    else chase<16, 2, false>(b, sm, ABa, raw_all, rtau_all, d_all, e_all, nullptr);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PTB_WAVE);
+    chase<2, true>(subs[blockIdx.x], sm, 16, wave, ABa, raw_all, rtau_all, d_all, e_all, state);
 }
 
 // ---- application of Q2 ---------------------------------------------------------
@@ -1360,37 +1458,48 @@ int sytrd_band(ptbgpu_ctx *ctx, const std::vector<SubDesc> &desc, double *A, dou
     }
     {
         ProfScope prof_(ctx, "band_chase");
-        // size classes by the rows a workgroup's registers hold
-        int done = 0;
-        auto lds = [&](int m, int nw) {
-            const int K = std::max((m - 1 + kBW - 1) / kBW, 1);
-            return sizeof(double) * (size_t)(50 * (K + 2) + 16 * nw);
-        };
-#define PTB_CHASE(NW, P, MEM, LOW)                                                                    \
-    do {                                                                                              \
-        const int to = count(LOW);                                                                    \
-        if (to > done) {                                                                              \
-            hipLaunchKernelGGL((k_chase<NW, P, MEM>), dim3(to - done), dim3(NW * 64),                 \
-                               lds(subs[done].m, NW), st, ds, done, AB, raw, rtau, d, e, PW);         \
-            PTB_CHECK_LAUNCH(ctx);                                                                    \
-            done = to;                                                                                \
-        }                                                                                             \
-    } while (0)
-        PTB_CHASE(16, 2, true, 1026);
-        if (nb - done <= ctx->num_cus) {
-            if (nb > done) {
-                hipLaunchKernelGGL(k_chase_few, dim3(nb - done), dim3(1024), lds(subs[done].m, 16), st,
-                                   ds + done, AB, raw, rtau, d, e);
+        const int big = count(1026);
+        if (big > 0) {
+            hipLaunchKernelGGL(k_chase_mem, dim3(big), dim3(1024), sizeof(double) * (size_t)chase_lds(max_m, 16),
+                               st, ds, AB, raw, rtau, d, e, PW);
+            PTB_CHECK_LAUNCH(ctx);
+        }
+        std::vector<ChaseJob> jobs;
+        int words = 0;
+        for (int i = big; i < nb;) {
+            const int m = subs[i].m;
+            const int most = nb - big <= ctx->num_cus || m > 257 ? 1 : m > 129 ? 2 : m > 65 ? 4 : 8;
+            const int n = std::min(most, nb - i), nw = n == 1 ? 16 : n == 2 ? 8 : n <= 4 ? 4 : 2;
+            jobs.push_back({i, n, m > 513 ? 4 : 2});
+            words = std::max(words, n * chase_lds(m, nw));
+            i += n;
+        }
+        if (jobs.size() <= 2 * (size_t)ctx->num_cus) {
+            if (!jobs.empty()) {
+                auto *dj = static_cast<ChaseJob *>(
+                    upload_table(ctx, "band_chase", jobs.data(), sizeof(ChaseJob) * jobs.size()));
+                if (!dj) return PTBGPU_E_NOMEM;
+                hipLaunchKernelGGL(k_chase, dim3((unsigned)jobs.size()), dim3(1024), sizeof(double) * (size_t)words,
+                                   st, ds, dj, AB, raw, rtau, d, e);
                 PTB_CHECK_LAUNCH(ctx);
             }
         } else {
-            PTB_CHASE(16, 4, false, 514);
-            PTB_CHASE(16, 2, false, 258);
-            PTB_CHASE(8, 2, false, 130);
-            PTB_CHASE(4, 2, false, 66);
-            PTB_CHASE(2, 2, false, 0);
+            int done = big;
+            auto run = [&](int nw, int low, auto kern) {
+                const int to = count(low);
+                if (to > done)
+                    hipLaunchKernelGGL(kern, dim3(to - done), dim3(nw * 64),
+                                       sizeof(double) * (size_t)chase_lds(subs[done].m, nw), st, ds + done, AB, raw,
+                                       rtau, d, e);
+                done = std::max(done, to);
+            };
+            run(16, 514, k_chase_class<16, 4>);
+            run(16, 258, k_chase_class<16, 2>);
+            run(8, 130, k_chase_class<8, 2>);
+            run(4, 66, k_chase_class<4, 2>);
+            run(2, 0, k_chase_class<2, 2>);
+            PTB_CHECK_LAUNCH(ctx);
         }
-#undef PTB_CHASE
     }
     if (blk > 0) {
         ProfScope prof_(ctx, "q2_prep");

@@ -101,3 +101,30 @@ def test_sweep_groups_of_every_remainder(engine, m):
     tol = 100 * max(m, 8) * np.finfo(float).eps
     assert np.abs(U.T @ S @ U - np.eye(m)).max() < tol
     assert np.abs(A @ U - (S @ U) * e).max() < tol * np.abs(e).max()
+
+
+def test_chase_routes_agree(engine):
+    """The same submatrices in a batch of up to one per CU, of a few times as many
+    (shared workgroups) and of more (a launch per size class): each batch's
+    densities are those of the molecules built alone."""
+    import torch
+    from conftest import small_system
+    mols = [small_system("water", (2, 2, 2), s) for s in range(3)] + [small_system("alkane", 6), small_system("alkane", 20)]
+
+    def item(mol, H, S):
+        dH, dS = torch.from_numpy(H).cuda(), torch.from_numpy(S).cuda()
+        return (mol.ndim, mol.nel, dH, dS, torch.zeros_like(dH), mol.n, mol.xyz, mol.aoat)
+
+    alone = []
+    for m in mols:
+        it = item(*m)
+        engine.sm_stupid_simple_dev(*it, 2, 2)
+        torch.cuda.synchronize()
+        alone.append(it[4])
+    for copies in (3, 10):
+        items = [item(*m) for _ in range(copies) for m in mols]
+        torch.cuda.synchronize()
+        engine.sm_stupid_simple_batch(items, 2, 2, device=True)
+        torch.cuda.synchronize()
+        for k, it in enumerate(items):
+            assert torch.equal(it[4], alone[k % len(mols)])
