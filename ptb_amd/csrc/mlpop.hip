@@ -17,6 +17,8 @@
 //   * q and qsh summed on the host in the reference's AO order.
 // The arithmetic after the float rounding of the inputs is FP64, so the result
 // differs from the reference's by the reference's own float rounding.
+#include <algorithm>
+
 #include "sm_internal.hpp"
 
 namespace {
@@ -43,11 +45,14 @@ __global__ __launch_bounds__(kT) void k_f32_to_f64(const float *__restrict__ a, 
         b[k] = (double)a[k];
 }
 
-// d_i = sum_k s2(i,k) cc(k,i): block b owns rows i0..i0+63; k runs in chunks
-// of 64 staged through LDS (s2 tile read along i, cc tile along k)
+// d_i = sum_k s2(i,k) cc(k,i): a workgroup owns rows i0..i0+63 and chunks of 64 k,
+// which it stages through LDS (s2 tile read along i, cc tile along k).  grid: (row
+// block, slice of the chunks): with one slice, 23 workgroups at 1472 rows, each
+// waiting for its chunks in turn, took 285 us; a chunk each takes 27.  Slice y's
+// sums go to d(:, y).
 __global__ __launch_bounds__(kT) void k_row_col_dot(const float *__restrict__ s2,
                                                     const double *__restrict__ cc, int64_t nao,
-                                                    double *__restrict__ d) {
+                                                    int chunks, double *__restrict__ d) {
     __shared__ double ts[64][65];
     __shared__ double tc[64][65];
     __shared__ double part[4][64];
@@ -55,7 +60,8 @@ __global__ __launch_bounds__(kT) void k_row_col_dot(const float *__restrict__ s2
     const int t = threadIdx.x;
     const int li = t & 63, lq = t >> 6;
     double acc = 0.0;
-    for (int64_t k0 = 0; k0 < nao; k0 += 64) {
+    const int64_t kb = (int64_t)blockIdx.y * chunks * 64, ke = min(nao, kb + (int64_t)chunks * 64);
+    for (int64_t k0 = kb; k0 < ke; k0 += 64) {
         __syncthreads();
         for (int e = t; e < 64 * 64; e += kT) {
             const int r = e & 63, c = e >> 6;
@@ -74,8 +80,18 @@ __global__ __launch_bounds__(kT) void k_row_col_dot(const float *__restrict__ s2
     __syncthreads();
     if (t < 64 && i0 + t < nao) {
         // fixed order over the four partial sums
-        d[i0 + t] = ((part[0][t] + part[1][t]) + part[2][t]) + part[3][t];
+        d[blockIdx.y * nao + i0 + t] = ((part[0][t] + part[1][t]) + part[2][t]) + part[3][t];
     }
+}
+
+// d(:, 0) = the slices' sums in order
+__global__ __launch_bounds__(kT) void k_slice_sum(int64_t nao, int slices, double *__restrict__ d) {
+    const int64_t i = (int64_t)blockIdx.x * kT + threadIdx.x;
+    if (i >= nao) return;
+    double s = d[i];
+#pragma unroll 8
+    for (int y = 1; y < slices; ++y) s += d[y * nao + i];
+    d[i] = s;
 }
 
 int mlpop2_device(ptbgpu_ctx *ctx, int64_t n, int64_t nao, const double *dP, const float *ds1,
@@ -86,7 +102,10 @@ int mlpop2_device(ptbgpu_ctx *ctx, int64_t n, int64_t nao, const double *dP, con
     auto *x = static_cast<double *>(ptb::ws(ctx, "mlpop_x", sizeof(double) * nn));
     auto *s1d = static_cast<double *>(ptb::ws(ctx, "mlpop_s1", sizeof(double) * nn));
     auto *cc = static_cast<double *>(ptb::ws(ctx, "mlpop_cc", sizeof(double) * nn));
-    auto *d = static_cast<double *>(ptb::ws(ctx, "mlpop_d", sizeof(double) * (size_t)nao));
+    // slices of k that give every CU two workgroups
+    const int64_t nb = (nao + 63) / 64, want = std::max<int64_t>(1, 2 * ctx->num_cus / nb);
+    const int chunks = (int)((nb + want - 1) / want), slices = (int)((nb + chunks - 1) / chunks);
+    auto *d = static_cast<double *>(ptb::ws(ctx, "mlpop_d", sizeof(double) * (size_t)nao * slices));
     if (!x || !s1d || !cc || !d) return PTBGPU_E_NOMEM;
     const unsigned nt = (unsigned)((nao + 31) / 32);
     hipLaunchKernelGGL(k_blow84, dim3(nt, nt), dim3(kT), 0, ctx->stream, dP, nao, x);
@@ -101,9 +120,13 @@ int mlpop2_device(ptbgpu_ctx *ctx, int64_t n, int64_t nao, const double *dP, con
     tl.add(&g, 1, true);
     PTB_TRY(tl.upload(ctx, "mlpop_w"));
     PTB_TRY(tl.launch(ctx, 0, false, false, dg, "mlpop"));
-    hipLaunchKernelGGL(k_row_col_dot, dim3((unsigned)((nao + 63) / 64)), dim3(kT), 0, ctx->stream,
-                       ds2, cc, nao, d);
+    hipLaunchKernelGGL(k_row_col_dot, dim3((unsigned)nb, slices), dim3(kT), 0, ctx->stream, ds2, cc, nao,
+                       chunks, d);
     PTB_CHECK_LAUNCH(ctx);
+    if (slices > 1) {
+        hipLaunchKernelGGL(k_slice_sum, dim3((unsigned)((nao + kT - 1) / kT)), dim3(kT), 0, ctx->stream, nao, slices, d);
+        PTB_CHECK_LAUNCH(ctx);
+    }
     std::vector<double> hd((size_t)nao);
     PTB_HIP(ctx, hipMemcpyAsync(hd.data(), d, sizeof(double) * nao, hipMemcpyDeviceToHost, ctx->stream));
     PTB_HIP(ctx, hipStreamSynchronize(ctx->stream));

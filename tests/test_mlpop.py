@@ -67,3 +67,34 @@ def test_gpu_mlpop2_matches_reference(engine, tag):
     d2 = torch.from_numpy(np.ascontiguousarray(c["s14"].T)).cuda()
     qd, qshd = engine.mlpop2(n, nao, dP, d1, d2, c["aoat"], c["shell2ao"])
     assert np.array_equal(qd, q) and np.array_equal(qshd, qsh)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nao", [1, 63, 64, 65, 200, 1500])
+def test_row_slices_match_float64(engine, nao):
+    """Row blocks and k slices with every remainder: populations of random
+    matrices against the same float inputs multiplied in float64."""
+    import torch
+    rng = np.random.default_rng(nao)
+    n = max(1, nao // 3)
+    aoat = np.sort(rng.integers(1, n + 1, size=nao))
+    shell = rng.integers(1, 11, size=nao)
+    iu = np.tril_indices(nao)
+    P = rng.normal(size=nao * (nao + 1) // 2)
+    s34, s14 = (rng.normal(size=(nao, nao)).astype(np.float32) for _ in range(2))
+    s34, s14 = s34 + s34.T, s14 + s14.T
+    q, qsh = engine.mlpop2(n, nao, torch.from_numpy(P).cuda(), torch.from_numpy(s34).cuda(),
+                           torch.from_numpy(s14).cuda(), aoat, shell)
+    p = np.zeros((nao, nao))
+    p[iu] = P.astype(np.float32)
+    p = p + np.tril(p, -1).T
+    a, b = s14.astype(float), p @ s34.astype(float)
+    d = (a * b.T).sum(1)
+    ref = np.zeros((10, n))
+    np.add.at(ref, (shell - 1, aoat - 1), d)
+    scale = (np.abs(a) * (np.abs(p) @ np.abs(s34.astype(float))).T).sum(1)
+    bound = np.zeros((10, n))
+    np.add.at(bound, (shell - 1, aoat - 1), scale)
+    tol = 4 * (nao + 8) * np.finfo(float).eps * np.maximum(bound, 1e-300)
+    assert (np.abs(qsh - ref) <= tol).all()
+    assert (np.abs(q - ref.sum(0)) <= tol.sum(0)).all()
