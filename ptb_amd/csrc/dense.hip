@@ -159,39 +159,84 @@ void k_gemm(const GemmDesc *__restrict__ descs, int count, int tiles,
         const int e = threadIdx.x + q * kT;
         if (!TB) { kk = e & (KS - 1); nn = e / KS; } else { nn = e & (TE - 1); kk = e / TE; }
     };
-    // element offsets are 32-bit (every operand block of the batch is below
-    // 2^32 elements from its descriptor pointer), which keeps the 16 addresses
-    // of a slice in half the registers of 64-bit pointers
-    // Every load is issued, from an address clamped into the operand block;
-    // elements outside it are zeroed when the slice is stored to LDS.  The
-    // empty asm statement there consumes the raw values unconditionally, so
-    // that no load can be moved under the range test: a guarded load waits
-    // for memory inside its branch, one element at a time.  Callers ensure
-    // kend > kbeg >= 0.
+    // Rows of A and columns of B beyond the product are read from its last one: they
+    // only reach results that are not written.  Byte offsets into a slice (32 bits hold
+    // them up to kLdMax) are formed once, from a base that advances along k, so a whole
+    // slice costs an addition per load and no clamps or masks: 58.9 -> 66.7 TFLOP/s on
+    // one 8192^3 product (128 x 128 tiles), A B products of the 512-water box 34.9 ->
+    // 33.1 ms.
+    constexpr int kLdMax = 1 << 22;
+    const bool fits = max(g.lda, g.ldb) < kLdMax;
     const unsigned ulda = (unsigned)g.lda, uldb = (unsigned)g.ldb;
-    auto load = [&](int k0) {
+    const gmem<T> *pA = gA + (TA ? (int64_t)m0 * g.lda + kbeg : m0 + (int64_t)kbeg * g.lda);
+    const gmem<T> *pB = gB + (TB ? n0 + (int64_t)kbeg * g.ldb : (int64_t)n0 * g.ldb + kbeg);
+    const int64_t stepA = TA ? KS : (int64_t)KS * g.lda, stepB = TB ? (int64_t)KS * g.ldb : KS;
+    auto a_off = [&](int q, int kmax) {
+        int mm, kk;
+        a_index(q, mm, kk);
+        const unsigned cm = (unsigned)min(mm, g.M - 1 - m0), ck = (unsigned)min(kk, kmax);
+        return TA ? cm * ulda + ck : ck * ulda + cm;
+    };
+    auto b_off = [&](int q, int kmax) {
+        int kb, nn;
+        b_index(q, kb, nn);
+        const unsigned cn = (unsigned)min(nn, g.N - 1 - n0), ck = (unsigned)min(kb, kmax);
+        return TB ? ck * uldb + cn : cn * uldb + ck;
+    };
+    unsigned oa[NL], ob[NL];  // bytes
 #pragma unroll
-        for (int q = 0; q < NL; ++q) {
-            int mm, kk;
-            a_index(q, mm, kk);
-            const unsigned cm = (unsigned)min(m0 + mm, g.M - 1), ck = (unsigned)min(k0 + kk, kend - 1);
-            xa[q] = gA[TA ? cm * ulda + ck : ck * ulda + cm];
-            int kb, nn;
-            b_index(q, kb, nn);
-            const unsigned cn = (unsigned)min(n0 + nn, g.N - 1), ckb = (unsigned)min(k0 + kb, kend - 1);
-            xb[q] = gB[TB ? ckb * uldb + cn : cn * uldb + ckb];
+    for (int q = 0; q < NL; ++q) {
+        oa[q] = (unsigned)sizeof(T) * a_off(q, KS - 1);
+        ob[q] = (unsigned)sizeof(T) * b_off(q, KS - 1);
+    }
+    auto at = [](const gmem<T> *p, unsigned bytes) {
+        return *(const gmem<T> *)((const gmem<char> *)p + bytes);
+    };
+    // The slice at k0 (pA and pB stand there).  In the last, partial one (or any of such
+    // long columns) every load is issued from an address clamped into the operand
+    // block, and elements outside it are zeroed when the slice is stored to LDS.  The
+    // empty asm statement there consumes the raw values unconditionally, so that no
+    // load can be moved under the range test: a guarded load waits for memory inside
+    // its branch, one element at a time.  Callers ensure kend > kbeg >= 0.
+    auto load = [&](int k0) {
+        if (fits && k0 + KS <= kend) {
+#pragma unroll
+            for (int q = 0; q < NL; ++q) {
+                xa[q] = at(pA, oa[q]);
+                xb[q] = at(pB, ob[q]);
+            }
+        } else {
+            asm volatile("");  // (else the two branches' loads are merged, and their addresses formed per slice)
+#pragma unroll
+            for (int q = 0; q < NL; ++q) {
+                xa[q] = pA[a_off(q, kend - 1 - k0)];
+                xb[q] = pB[b_off(q, kend - 1 - k0)];
+            }
         }
+        pA += stepA;
+        pB += stepB;
     };
     auto store = [&](int k0) {
+        const bool whole = k0 + KS <= kend;
+        if (!whole) {
 #pragma unroll
-        for (int q = 0; q < NL; ++q) asm volatile("" : "+v"(xa[q]), "+v"(xb[q]));
+            for (int q = 0; q < NL; ++q) asm volatile("" : "+v"(xa[q]), "+v"(xb[q]));
+#pragma unroll
+            for (int q = 0; q < NL; ++q) {
+                int mm, kk, kb, nn;
+                a_index(q, mm, kk);
+                b_index(q, kb, nn);
+                xa[q] = k0 + kk < kend ? xa[q] : T(0);
+                xb[q] = k0 + kb < kend ? xb[q] : T(0);
+            }
+        }
 #pragma unroll
         for (int q = 0; q < NL; ++q) {
             int mm, kk, kb, nn;
             a_index(q, mm, kk);
             b_index(q, kb, nn);
-            As[kk][mm] = (m0 + mm < g.M && k0 + kk < kend) ? (double)xa[q] : 0.0;
-            Bs[kb][nn] = (n0 + nn < g.N && k0 + kb < kend) ? (double)xb[q] : 0.0;
+            As[kk][mm] = (double)xa[q];
+            Bs[kb][nn] = (double)xb[q];
         }
     };
     if (kbeg < kend) {
