@@ -145,6 +145,16 @@ void *hws(ptbgpu_ctx *ctx, const char *name, size_t bytes) {
     return b.ptr;
 }
 
+void *hws_mapped(ptbgpu_ctx *ctx, const char *name, size_t bytes, void **dev) {
+    void *h = hws(ctx, name, bytes);
+    if (h && hipHostGetDevicePointer(dev, h, 0) != hipSuccess) {
+        (void)hipGetLastError();
+        fail(ctx, PTBGPU_E_HIP, "no device address of the pinned buffer '%s'", name);
+        return nullptr;
+    }
+    return h;
+}
+
 namespace {
 
 constexpr size_t kStageDirect = (size_t)8 << 20;  // smaller copies: one runtime copy

@@ -111,6 +111,9 @@ void *upload_table(ptbgpu_ctx *ctx, const char *name, const void *src, size_t by
 int upload_async(ptbgpu_ctx *ctx, void *dst, const void *src, size_t bytes);
 // Named pinned host buffer of at least `bytes`.
 void *hws(ptbgpu_ctx *ctx, const char *name, size_t bytes);
+// The same with its device address (small results that a kernel writes straight to
+// the host: no copy between the kernel and the host's wait).
+void *hws_mapped(ptbgpu_ctx *ctx, const char *name, size_t bytes, void **dev);
 // Copies between pageable host memory and the device, on the context's
 // stream.  Large copies go in chunks through two pinned staging buffers: the
 // host side of each chunk is copied by several threads while the previous

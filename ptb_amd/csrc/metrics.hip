@@ -155,16 +155,18 @@ int weighted_dot(ptbgpu_ctx *ctx, const double *dA, const double *dB, int64_t nd
     const int64_t len = ndim * (ndim + 1) / 2;
     const int blocks = (int)std::max<int64_t>(1, std::min<int64_t>((len + kThreads - 1) / kThreads,
                                                                    (int64_t)ctx->num_cus * 8));
-    auto *part = static_cast<double *>(ws(ctx, "metric_part", sizeof(double) * (blocks + 1)));
-    if (!part) return PTBGPU_E_NOMEM;
+    auto *part = static_cast<double *>(ws(ctx, "metric_part", sizeof(double) * blocks));
+    void *sum = nullptr;  // the result, written to the host by the kernel
+    auto *hsum = static_cast<double *>(hws_mapped(ctx, "metric_sum", sizeof(double), &sum));
+    if (!part || !hsum) return PTBGPU_E_NOMEM;
     hipLaunchKernelGGL(k_weighted_dot, dim3(blocks), dim3(kThreads), 0, ctx->stream, dA, dB, len,
                        part);
     PTB_CHECK_LAUNCH(ctx);
-    hipLaunchKernelGGL(k_ordered_sum, dim3(1), dim3(kThreads), 0, ctx->stream, part, blocks, part + blocks);
+    hipLaunchKernelGGL(k_ordered_sum, dim3(1), dim3(kThreads), 0, ctx->stream, part, blocks,
+                       static_cast<double *>(sum));
     PTB_CHECK_LAUNCH(ctx);
-    PTB_HIP(ctx, hipMemcpyAsync(result, part + blocks, sizeof(double), hipMemcpyDeviceToHost,
-                                ctx->stream));
     PTB_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    *result = *hsum;
     return PTBGPU_OK;
 }
 

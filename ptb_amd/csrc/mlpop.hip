@@ -84,14 +84,15 @@ __global__ __launch_bounds__(kT) void k_row_col_dot(const float *__restrict__ s2
     }
 }
 
-// d(:, 0) = the slices' sums in order
-__global__ __launch_bounds__(kT) void k_slice_sum(int64_t nao, int slices, double *__restrict__ d) {
+// out = the slices' sums in order
+__global__ __launch_bounds__(kT) void k_slice_sum(int64_t nao, int slices, const double *__restrict__ d,
+                                                  double *__restrict__ out) {
     const int64_t i = (int64_t)blockIdx.x * kT + threadIdx.x;
     if (i >= nao) return;
     double s = d[i];
 #pragma unroll 8
     for (int y = 1; y < slices; ++y) s += d[y * nao + i];
-    d[i] = s;
+    out[i] = s;
 }
 
 int mlpop2_device(ptbgpu_ctx *ctx, int64_t n, int64_t nao, const double *dP, const float *ds1,
@@ -123,12 +124,12 @@ int mlpop2_device(ptbgpu_ctx *ctx, int64_t n, int64_t nao, const double *dP, con
     hipLaunchKernelGGL(k_row_col_dot, dim3((unsigned)nb, slices), dim3(kT), 0, ctx->stream, ds2, cc, nao,
                        chunks, d);
     PTB_CHECK_LAUNCH(ctx);
-    if (slices > 1) {
-        hipLaunchKernelGGL(k_slice_sum, dim3((unsigned)((nao + kT - 1) / kT)), dim3(kT), 0, ctx->stream, nao, slices, d);
-        PTB_CHECK_LAUNCH(ctx);
-    }
-    std::vector<double> hd((size_t)nao);
-    PTB_HIP(ctx, hipMemcpyAsync(hd.data(), d, sizeof(double) * nao, hipMemcpyDeviceToHost, ctx->stream));
+    void *out = nullptr;  // the sums, written to the host by the kernel
+    auto *hd = static_cast<double *>(ptb::hws_mapped(ctx, "mlpop_h", sizeof(double) * (size_t)nao, &out));
+    if (!hd) return PTBGPU_E_NOMEM;
+    hipLaunchKernelGGL(k_slice_sum, dim3((unsigned)((nao + kT - 1) / kT)), dim3(kT), 0, ctx->stream, nao, slices, d,
+                       static_cast<double *>(out));
+    PTB_CHECK_LAUNCH(ctx);
     PTB_HIP(ctx, hipStreamSynchronize(ctx->stream));
     for (int64_t a = 0; a < n; ++a) q[a] = 0.0;
     for (int64_t a = 0; a < 10 * n; ++a) qsh[a] = 0.0;

@@ -92,6 +92,34 @@ __global__ void k_reduce(const double *__restrict__ A, const double *__restrict_
     }
 }
 
+// C = a A + b B (C may alias A or B) and k_reduce's partials of C without a second
+// operand, summed over the same elements in the same order
+__global__ void k_axpby_reduce(double a, const double *A, double b, const double *B, int64_t n,
+                               double *C, double *__restrict__ part) {
+    __shared__ double red[16];
+    double s2 = 0.0, si = 0.0, nan = 0.0;
+    const int64_t tot = n * n;
+    for (int64_t k = (int64_t)blockIdx.x * kT + threadIdx.x; k < tot;
+         k += (int64_t)gridDim.x * kT) {
+        double v = a * A[k];
+        v += b * B[k];
+        C[k] = v;
+        s2 += v * v;
+        const double d = ((k / n == k % n) ? 1.0 : 0.0) - v;
+        si += d * d;
+        if (v != v) nan += 1.0;
+    }
+    const double t0 = block_sum(s2, red);
+    const double t1 = block_sum(si, red);
+    const double t3 = block_sum(nan, red);
+    if (threadIdx.x == 0) {
+        part[4 * blockIdx.x + 0] = t0;
+        part[4 * blockIdx.x + 1] = t1;
+        part[4 * blockIdx.x + 2] = 0.0;
+        part[4 * blockIdx.x + 3] = t3;
+    }
+}
+
 // per column j: [j] = sum_i |A(i,j)| (gershgorin, source/norms.f90:5-18),
 // [n + j] = sum_i |A(j,i)| (infinity, :32-49), [2n + j] = sum_i A(i,j)^2
 __global__ void k_col_sums(const double *__restrict__ A, int64_t n, double *__restrict__ out) {
@@ -135,7 +163,8 @@ struct Dense {
     ptbgpu_ctx *ctx;
     int64_t n;
     int blocks;
-    double *part;     // 4 * blocks reduction partials
+    double *part;     // 4 * blocks reduction partials (pinned host memory), device address
+    double *hpart;    // the same, host address
     double *sums;     // 3n column sums
     double *wvec;     // n diagonal weights
     GemmDesc *dg;     // kMaxGemm descriptors
@@ -171,14 +200,19 @@ struct Dense {
     int reduce(const double *A, const double *B, double r[4]) {
         hipLaunchKernelGGL(k_reduce, dim3(blocks), dim3(kT), 0, ctx->stream, A, B, n, part);
         PTB_CHECK_LAUNCH(ctx);
-        auto *h = static_cast<double *>(ptb::hws(ctx, "pur_part_h", sizeof(double) * 4 * blocks));
-        if (!h) return PTBGPU_E_NOMEM;
-        PTB_HIP(ctx, hipMemcpyAsync(h, part, sizeof(double) * 4 * blocks, hipMemcpyDeviceToHost,
-                                    ctx->stream));
+        return collect(r);
+    }
+    // C = a A + b B, and reduce(C) in the same pass
+    int axpby_reduce(double a, const double *A, double b, const double *B, double *C, double r[4]) {
+        hipLaunchKernelGGL(k_axpby_reduce, dim3(blocks), dim3(kT), 0, ctx->stream, a, A, b, B, n, C, part);
+        PTB_CHECK_LAUNCH(ctx);
+        return collect(r);
+    }
+    int collect(double r[4]) {
         PTB_HIP(ctx, hipStreamSynchronize(ctx->stream));
         for (int q = 0; q < 4; ++q) r[q] = 0.0;
         for (int b = 0; b < blocks; ++b)
-            for (int q = 0; q < 4; ++q) r[q] += h[4 * b + q];
+            for (int q = 0; q < 4; ++q) r[q] += hpart[4 * b + q];
         return PTBGPU_OK;
     }
     // column sums of A into the host vector h (3n: abs col, abs row, squares)
@@ -263,13 +297,15 @@ int ptbgpu_purify_dev(ptbgpu_ctx *ctx, const ptbgpu_pur_settings *ps, int64_t n,
     }
     double *H = m[0], *S = m[1], *X = m[2], *G = m[3], *P = m[4], *T1 = m[5], *T2 = m[6],
            *T3 = m[7];
-    Dense D{ctx, n, 0, nullptr, nullptr, nullptr, nullptr, {}};
+    Dense D{ctx, n, 0, nullptr, nullptr, nullptr, nullptr, nullptr, {}};
     D.blocks = (int)std::max<int64_t>(1, std::min<int64_t>((n * n + kT - 1) / kT, 1024));
-    D.part = static_cast<double *>(ptb::ws(ctx, "pur_part", sizeof(double) * 4 * D.blocks));
+    void *part = nullptr;
+    D.hpart = static_cast<double *>(ptb::hws_mapped(ctx, "pur_part", sizeof(double) * 4 * D.blocks, &part));
+    D.part = static_cast<double *>(part);
     D.sums = static_cast<double *>(ptb::ws(ctx, "pur_sums", sizeof(double) * 3 * n));
     D.wvec = static_cast<double *>(ptb::ws(ctx, "pur_w", sizeof(double) * n));
     D.dg = static_cast<GemmDesc *>(ptb::ws(ctx, "pur_gemm", sizeof(GemmDesc) * kMaxGemm));
-    if (!D.part || !D.sums || !D.wvec || !D.dg) return PTBGPU_E_NOMEM;
+    if (!D.hpart || !D.sums || !D.wvec || !D.dg) return PTBGPU_E_NOMEM;
     D.table.reserve(kMaxGemm);
     const int ub = (int)std::min<int64_t>(n, 2048);
     hipLaunchKernelGGL(k_unpack, dim3(ub), dim3(kT), 0, ctx->stream, dHp, n, H);
@@ -368,7 +404,7 @@ int ptbgpu_purify_dev(ptbgpu_ctx *ctx, const ptbgpu_pur_settings *ps, int64_t n,
             }
             PTB_TRY(D.axpby(2.0, P, 0.0, nullptr, 0.0, P));
         } else {
-            double *sign_ = T3;
+            double *sign_ = T3, *work = T2;
             if (ps->type == PADE || ps->type == NEWTON) {
                 // sign_iterative (:512-601)
                 PTB_TRY(D.copy(G, sign_));
@@ -377,15 +413,16 @@ int ptbgpu_purify_dev(ptbgpu_ctx *ctx, const ptbgpu_pur_settings *ps, int64_t n,
                     const double norm = std::sqrt(r[0]);
                     PTB_TRY(D.gemm(sign_, false, sign_, false, T1));     // X^2
                     if (ps->type == PADE) {
-                        PTB_TRY(D.gemm(T1, false, T1, false, T2));       // X^4
-                        PTB_TRY(D.axpby(-10.0, T1, 3.0, T2, 15.0, T1));  // 15I - 10X^2 + 3X^4
-                        PTB_TRY(D.gemm(sign_, false, T1, false, T2, 0.125));
+                        PTB_TRY(D.gemm(T1, false, T1, false, work));     // X^4
+                        PTB_TRY(D.axpby(-10.0, T1, 3.0, work, 15.0, T1));  // 15I - 10X^2 + 3X^4
+                        PTB_TRY(D.gemm(sign_, false, T1, false, work, 0.125));
+                        std::swap(sign_, work);
+                        PTB_TRY(D.reduce(sign_, nullptr, r));
                     } else {
-                        PTB_TRY(D.gemm(sign_, false, T1, false, T2));    // X^3
-                        PTB_TRY(D.axpby(1.5, sign_, -0.5, T2, 0.0, T2)); // (3X - X^3) / 2
+                        PTB_TRY(D.gemm(sign_, false, T1, false, work));  // X^3
+                        // (3X - X^3) / 2
+                        PTB_TRY(D.axpby_reduce(1.5, sign_, -0.5, work, sign_, r));
                     }
-                    PTB_TRY(D.copy(T2, sign_));
-                    PTB_TRY(D.reduce(sign_, nullptr, r));
                     if (r[3] > 0.0) return ptb::fail(ctx, PTBGPU_E_NAN, kNaNPur);
                     if (std::fabs(std::sqrt(r[0]) - norm) < tnorm) break;
                 }
