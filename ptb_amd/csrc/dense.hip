@@ -444,11 +444,13 @@ __global__ __launch_bounds__(kT, sizeof(T) == 4 ? 6 : 4) void k_gemm_nt1(
 //
 // A panel is a serial chain (32 square roots and divisions), so one wavefront
 // keeps the block in registers (lane = row; a column reaches the other lanes
-// through scalar registers, no barrier) while the others load their rows below;
-// these are then solved by substitution, a thread per row, the factor read from
-// LDS (one address per wavefront).  With four wavefronts and three barriers per
-// column, the block's inverse and X = P L_kk^-T by it, a panel of one 1472-row
-// matrix (modes 1 and 2) took 76 us, now 28; one of the 512-water box 120, now 71.
+// through scalar registers, no barrier) and inverts it there (lane = column) while
+// the others load their rows below; these are then multiplied by the inverse, a
+// thread per row, read from LDS at one address per wavefront.  With four wavefronts
+// and three barriers per column a panel of one 1472-row matrix (modes 1 and 2) took
+// 76 us, now 31; one of the 512-water box 120, now 77.  (Substitution instead of the
+// inverse is faster still, 28 and 71 us, but rounds the rows differently, and the
+// float copy of K that a mixed build reduces takes such a change on to its density.)
 //
 // mode 0: the whole panel (grid (submatrix, 1)).  For few submatrices the
 // panel is split: mode 1 forms the rows below the diagonal block, sliced over
@@ -465,7 +467,7 @@ __global__ __launch_bounds__(kT) void k_potrf_panel(const SubDesc *__restrict__ 
     if (k0 >= m) return;
     double *a = Aa + d.off + (int64_t)k0 * ld;  // the panel's columns
     const int kb = min(32, m - k0);
-    __shared__ double Lc[32][32], rinv[32];  // Lc[c][r] = L(r, c)
+    __shared__ double Li[32][32];  // L_kk^-1
     double p[32];
     // a row of the panel below (there are none unless kb = 32)
     auto load = [&](int i) {
@@ -482,7 +484,6 @@ __global__ __launch_bounds__(kT) void k_potrf_panel(const SubDesc *__restrict__ 
 #pragma unroll
         for (int c = 0; c < 32; ++c) x[c] = r < kb && c < kb ? (r >= c ? x[c] : 0.0) : r == c ? 1.0 : 0.0;
         bool bad = false;
-        double diag = 1.0;
 #pragma unroll
         for (int j = 0; j < 32; ++j) {
             double q = lane_value(x[j], j);
@@ -492,7 +493,6 @@ __global__ __launch_bounds__(kT) void k_potrf_panel(const SubDesc *__restrict__ 
             }
             const double sq = sqrt(q), l = r == j ? sq : x[j] / sq;
             x[j] = l;
-            diag = r == j ? sq : diag;
 #pragma unroll
             for (int c = j + 1; c < 32; ++c) x[c] -= l * lane_value(l, c);
         }
@@ -504,26 +504,37 @@ __global__ __launch_bounds__(kT) void k_potrf_panel(const SubDesc *__restrict__ 
             if (threadIdx.x == 0 && bad) flags[blockIdx.x] |= 1;
         }
         if (mode == 2) return;
-        if (threadIdx.x < 32) {
+        // the inverse by forward substitution, lane r its column r (zero above r)
+        double y[32];
 #pragma unroll
-            for (int c = 0; c < 32; ++c) Lc[c][r] = x[c];
-            rinv[r] = 1.0 / diag;
+        for (int c = 0; c < 32; ++c) {
+            double t = r == c ? 1.0 : 0.0;
+#pragma unroll
+            for (int q = 0; q < c; ++q) t -= lane_value(x[q], c) * y[q];
+            y[c] = t / lane_value(x[c], c);
+            if (threadIdx.x < 32) Li[c][r] = y[c];
         }
         if (i < m) load(i);
     } else if (i < m) {
         load(i);
     }
     __syncthreads();
-    // p <- p L^-T, column by column
+    // X(i, c) = sum_{t <= c} P(i, t) Li(c, t), the last columns first (in place), four
+    // chains at a time
     int zero = 0;
     while (i < m) {
-        asm volatile("" : "+v"(zero));  // (keeps the factor in LDS)
+        asm volatile("" : "+v"(zero));  // (keeps the inverse in LDS)
 #pragma unroll
-        for (int c = 0; c < 32; ++c) {
-            p[c] *= rinv[c + zero];
+        for (int c = 28; c >= 0; c -= 4) {
+            double v[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-            for (int t = c + 1; t < 32; ++t) p[t] -= p[c] * Lc[c][t + zero];
-            if (c & 1) __builtin_amdgcn_sched_barrier(0);  // (nor read all of it ahead)
+            for (int t = 0; t < c + 4; ++t)
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    if (t <= c + u) v[u] += p[t] * Li[c + u][t + zero];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) p[c + u] = v[u];
+            __builtin_amdgcn_sched_barrier(0);  // (nor read all of it ahead)
         }
 #pragma unroll
         for (int c = 0; c < 32; ++c) a[(unsigned)c * ld + (unsigned)i] = p[c];
