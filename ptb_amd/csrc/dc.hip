@@ -712,7 +712,7 @@ __global__ __launch_bounds__(NT) void k_dc_merge(const SubDesc *__restrict__ des
         gg.C32 = nullptr;
     }
     // a node from device scratch leaves the O(K^2) phases to three kernels
-    // over the whole chip (k_dc_roots_big, k_dc_loewner_big, k_dc_vectors_big)
+    // over the whole chip (k_dc_roots_columns, k_dc_loewner_deflated, k_dc_vectors_big)
     if constexpr (kGlobal)
         if (threadIdx.x == 0) gK[4 * blockIdx.x] = K;
     if constexpr (MODE != kDcLds) return;
