@@ -136,11 +136,11 @@ int ptbgpu_stream(ptbgpu_ctx *ctx, void **stream);
  * refinement; 0 puts every submatrix on float storage (default 288).
  * "gemm_tile": output tile edge of the FP64 products, 64 or 128 (identical
  * results either way); 0 (default) chooses per launch: 128 only for launches
- * of fewer than 8 large products.  "dc_global_min": merge size classes of at
+ * of fewer than 8 large products, 32 for launches of few tiles.  "dc_global_min": merge size classes of at
  * least this many rows run their secular roots and vectors over the whole
  * chip from device scratch even when they fit in LDS (identical results;
  * slower on MI355X, so 0, the default, keeps that path for the classes that
- * do not fit).  "lowp_merge_max_m": a mixed build's float-reduced
+ * do not fit; levels of few nodes then go over the chip from LDS).  "lowp_merge_max_m": a mixed build's float-reduced
  * submatrices of up to this many rows take their merge products in the
  * low-precision arithmetic (then two Loewdin steps in the refinement instead
  * of one); 0 (default) keeps FP64 merge products, as fast on MI355X.

@@ -54,10 +54,12 @@ struct ptbgpu_ctx {
     int64_t lowp_merge_max_m = 0;
     // merge size classes (power-of-two node sizes) at or above this run their
     // secular roots, Loewner vectors and eigenvectors over the whole chip from
-    // device scratch even when they fit in LDS (0: only those that do not)
+    // device scratch even when they fit in LDS (0: only those that do not, and
+    // levels of no more nodes than CUs, from LDS)
     int64_t dc_global_min = 0;
     // tile edge of the FP64 GEMM launches: 0 chooses per launch (128 x 128
-    // tiles for launches with many large products), 64 or 128 forces it
+    // tiles for a few large products, 32 x 32 for launches of few tiles), 64 or
+    // 128 forces it
     int64_t gemm_tile = 0;
     // "graph": the eigen phase of repeated one-chunk builds replays a captured
     // hipGraph; the cache of instantiated graphs (keyed by shapes and
