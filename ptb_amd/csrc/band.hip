@@ -31,6 +31,7 @@
 #include <type_traits>
 #include <utility>
 
+#include "reflector.hpp"
 #include "sm_internal.hpp"
 
 namespace {
@@ -133,21 +134,13 @@ __device__ __forceinline__ double sum16(const double (&p)[16], int lane) {
     return dpp_add<0x4E>(dpp_add<0xB1>(v));
 }
 
-// The reflector of x (alpha at the pivot, sigma the squares of the rest):
-// H = I - tau u u^T, u = 1 at the pivot and x * scale elsewhere, H x = beta.
-struct Reflector {
-    double beta, tau, scale;
-};
-__device__ __forceinline__ Reflector reflector(double alpha, double sigma) {
-    if (sigma == 0.0) return {alpha, 0.0, 0.0};
-    const double beta = -copysign(sqrt(alpha * alpha + sigma), alpha);
-    return {beta, (beta - alpha) / beta, 1.0 / (alpha - beta)};
-}
-// The same for the chase, where it is on the serial chain of every step: the norm
+// reflector() for the chase, where it is on the serial chain of every step: the norm
 // and its reciprocal from one hardware estimate of 1 / sqrt (coupled Newton
-// steps), the scale from one of 1 / x, each refined to rounding level.
+// steps), the scale from one of 1 / x, each refined to rounding level.  The chase
+// works on a matrix whose largest element is near 1, so elements that the test drops
+// (3e-145 of it) count for nothing, and the squares of the others are normal.
 __device__ __forceinline__ Reflector reflector_fast(double alpha, double sigma) {
-    if (sigma == 0.0) return {alpha, 0.0, 0.0};
+    if (sigma < kSquareMin) return {alpha, 0.0, 0.0};
     const double n2 = alpha * alpha + sigma, y = __builtin_amdgcn_rsq(n2);
     double g = n2 * y, h = 0.5 * y;
     double e = fma(-h, g, 0.5);
@@ -162,7 +155,6 @@ __device__ __forceinline__ Reflector reflector_fast(double alpha, double sigma) 
     r = fma(r, fma(-q, r, 1.0), r);
     return {-copysign(g, alpha), fma(2.0 * h, fabs(alpha), 1.0), copysign(r, alpha)};
 }
-
 // ---- stage 1 ------------------------------------------------------------------
 
 // QR of one 16-column panel, rows r0 .. m - 1 in registers (thread t holds rows
@@ -202,28 +194,39 @@ __global__ __launch_bounds__(NT, R == 4 ? 2 : 4) void k_band_qr(const BandSub *_
         constexpr int j = decltype(J)::value;
         if (j >= nref) return;
         const int bf = j & 1;
-        double p[kBW];
-#pragma unroll
-        for (int l = 0; l < kBW; ++l) p[l] = 0.0;
-#pragma unroll
-        for (int q = 0; q < R; ++q) {
-            const double xi = (int)threadIdx.x + NT * q > j ? x[q][j] : 0.0;
-#pragma unroll
-            for (int l = 0; l < kBW; ++l) p[l] += xi * x[q][l];
-        }
-        const double s = sum16(p, lane);
-        if ((lane & 3) == 0) red[bf][wave][lane >> 2] = s;
-        if ((int)threadIdx.x == j)
-#pragma unroll
-            for (int l = 0; l < kBW; ++l) prow[bf][l] = x[0][l];
-        __syncthreads();
-        // every wavefront forms the scalars, lane l (mod 16) those of column l
         const int l = lane & 15;
-        double dot = 0.0;
+        double pl, dot, alpha, sigma, down = 1.0;
+        for (;;) {
+            double p[kBW];
 #pragma unroll
-        for (int w = 0; w < NW; ++w) dot += red[bf][w][l];
-        const double pl = prow[bf][l];
-        const Reflector h = reflector(read_lane(pl, j), read_lane(dot, j));
+            for (int l = 0; l < kBW; ++l) p[l] = 0.0;
+#pragma unroll
+            for (int q = 0; q < R; ++q) {
+                const double xi = (int)threadIdx.x + NT * q > j ? x[q][j] : 0.0;
+#pragma unroll
+                for (int l = 0; l < kBW; ++l) p[l] += xi * x[q][l];
+            }
+            const double s = sum16(p, lane);
+            if ((lane & 3) == 0) red[bf][wave][lane >> 2] = s;
+            if ((int)threadIdx.x == j)
+#pragma unroll
+                for (int l = 0; l < kBW; ++l) prow[bf][l] = x[0][l];
+            __syncthreads();
+            // every wavefront forms the scalars, lane l (mod 16) those of column l
+            dot = 0.0;
+#pragma unroll
+            for (int w = 0; w < NW; ++w) dot += red[bf][w][l];
+            pl = prow[bf][l];
+            alpha = read_lane(pl, j), sigma = read_lane(dot, j);
+            if (!(alpha * alpha + sigma < kSquareMin) || down != 1.0) break;
+            down = 1.0 / kRescale;
+#pragma unroll
+            for (int q = 0; q < R; ++q)
+                x[q][j] *= (int)threadIdx.x + NT * q >= j ? kRescale : 1.0;
+            __syncthreads();  // (the sums are written again)
+        }
+        Reflector h = reflector(alpha, sigma);
+        h.beta *= down;
         const double zl = pl + h.scale * dot;  // A(:, l)^T v
         const double wl = l > j ? h.tau * zl : 0.0;
         if (threadIdx.x < kBW) zt[j][l] = zl;
@@ -718,7 +721,8 @@ __global__ __launch_bounds__(256) void k_band_extract(const BandSub *__restrict_
 
 // Message area of a chase, per window k: the reflector that acts on it (vm, by
 // slot; tm), its diagonal block's first column and the element below it (cm,
-// bm), and its off-diagonal block's first row (rm).
+// bm), and its off-diagonal block's first row (rm).  Before vm: what takes the
+// scaled matrix back (vm[-2]).
 struct ChaseLds {
     double *vm, *tm, *cm, *bm, *rm, *wsc;
 };
@@ -819,8 +823,8 @@ __device__ __forceinline__ void chase_step(double (&D)[4], double (&B)[4], int k
         }
         if (lane == 0) {
             L.tm[0] = h.tau;
-            dv[s] = dia;
-            ev[s] = s < m - 1 ? h.beta : 0.0;
+            dv[s] = dia * L.vm[-2];
+            ev[s] = s < m - 1 ? h.beta * L.vm[-2] : 0.0;
             if (!last) rtau[blk * 16 + (s & 15)] = h.tau;
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -917,21 +921,34 @@ __device__ __forceinline__ void chase(const BandSub &b, double *sm, int nw, int 
     const int K = max((m - 1 + kBW - 1) / kBW, 1);  // windows
     const int lane = threadIdx.x % PTB_WAVE, tid = PTB_WAVE * wave + lane, NW = nw;
     ChaseLds L;
-    L.vm = sm;
+    L.vm = sm + 2;
     L.cm = L.vm + 16 * (K + 2);
     L.rm = L.cm + 16 * (K + 2);
     L.wsc = L.rm + 16 * (K + 2) + 16 * wave;
     L.tm = L.rm + 16 * (K + 2) + 16 * NW;
     L.bm = L.tm + (K + 2);
     const double *ab = ABa + b.ab;
+    // the power of two that brings the largest element near 1 (see reflector_fast)
+    double up = 1.0;
+    {
+        double big = 0.0;
+        for (int l = tid; l < kABL * m; l += NW * 64)
+            big = fmax(big, l / kABL + l % kABL < m ? fabs(ab[l]) : 0.0);
+        big = wave_max(big);
+        if (lane == 0) L.wsc[0] = big;
+        __syncthreads();
+        for (int w = 0; w < NW; ++w) big = fmax(big, L.wsc[16 * (w - wave)]);
+        if (big > 0.0 && big < HUGE_VAL) up = ldexp(1.0, -min(max(ilogb(big), -1000), 1000));
+        if (tid == 0) L.vm[-2] = 1.0 / up;
+    }
     for (int l = tid; l < 16 * (K + 2); l += NW * 64) {
         L.vm[l] = 0.0;
         L.rm[l] = 0.0;
-        L.cm[l] = l < 16 && l < m ? ab[l] : 0.0;
+        L.cm[l] = l < 16 && l < m ? up * ab[l] : 0.0;
     }
     for (int l = tid; l < K + 2; l += NW * 64) {
         L.tm[l] = 0.0;
-        L.bm[l] = l == 0 && m > kBW ? ab[kBW] : 0.0;
+        L.bm[l] = l == 0 && m > kBW ? up * ab[kBW] : 0.0;
     }
     double *raw = raw_all + b.blk * 256, *rtau = rtau_all + b.blk * 16;
     double *dv = d_all + b.mapoff, *ev = e_all + b.mapoff;
@@ -942,8 +959,8 @@ __device__ __forceinline__ void chase(const BandSub &b, double *sm, int nw, int 
         for (int c = 0; c < 4; ++c) {
             const int cl = 1 + 16 * k + ((4 * g + c - 1) & 15);
             const int lo = min(r, cl), hi = max(r, cl);
-            D[c] = hi < m ? ab[(int64_t)lo * kABL + hi - lo] : 0.0;
-            B[c] = r + 16 < m && r <= cl ? ab[(int64_t)cl * kABL + r + 16 - cl] : 0.0;
+            D[c] = hi < m ? up * ab[(int64_t)lo * kABL + hi - lo] : 0.0;
+            B[c] = r + 16 < m && r <= cl ? up * ab[(int64_t)cl * kABL + r + 16 - cl] : 0.0;
         }
     };
     auto active = [&](int k, int s) { return s >= 0 && s < m && (k == 0 || s + 1 + 16 * k < m); };
@@ -996,7 +1013,7 @@ struct ChaseJob {
 // doubles of LDS of a submatrix of m rows and nw wavefronts
 __host__ __device__ inline int chase_lds(int m, int nw) {
     const int K = m > kBW ? (m - 1 + kBW - 1) / kBW : 1;
-    return 50 * (K + 2) + 16 * nw;
+    return 50 * (K + 2) + 16 * nw + 2;
 }
 
 // A small batch (submatrices of up to 1025 rows) in one launch of 16-wavefront

@@ -22,6 +22,7 @@
 // stored values are rounded to T.
 #include <algorithm>
 
+#include "reflector.hpp"
 #include "sm_internal.hpp"
 
 namespace {
@@ -169,19 +170,24 @@ __global__ __launch_bounds__(kT, sizeof(T) == 4 ? 3 : 2) void k_sytrd_panel(cons
                 for (int t = 0; t < jj; ++t) dkk -= 2.0 * c2[t] * c1[t];
                 dd[k] = dkk;
             }
-            const double sigma = block_reduce(part_s, red);  // includes a barrier
+            double sigma = block_reduce(part_s, red);  // includes a barrier
             // (c) reflector
-            const double alpha = vs[k + 1];
-            double beta, tk, scale;
-            if (sigma == 0.0) {
-                beta = alpha;
-                tk = 0.0;
-                scale = 0.0;
-            } else {
-                beta = -copysign(sqrt(alpha * alpha + sigma), alpha);
-                tk = (beta - alpha) / beta;
-                scale = 1.0 / (alpha - beta);
+            double alpha = vs[k + 1], down = 1.0;
+            // (float storage: no square of its columns is that small)
+            if (sizeof(T) == 8 && alpha * alpha + sigma < kSquareMin) {  // the same in every thread
+                __syncthreads();
+                part_s = 0.0;
+                for (int i = k + 1 + threadIdx.x; i < m; i += kT) {
+                    const double x = vs[i] * kRescale;
+                    vs[i] = x;
+                    if (i > k + 1) part_s += x * x;
+                }
+                sigma = block_reduce(part_s, red);
+                alpha = vs[k + 1];
+                down = 1.0 / kRescale;
             }
+            const Reflector h = reflector(alpha, sigma);
+            const double beta = h.beta * down, tk = h.tau, scale = h.scale;
             __syncthreads();
             for (int i = k + 1 + threadIdx.x; i < m; i += kT) {
                 const double v = (i == k + 1) ? 1.0 : vs[i] * scale;
@@ -420,7 +426,8 @@ __global__ void k_sytrd_finish(const SubDesc *__restrict__ desc, const T *__rest
 // submatrix and holds its vectors in LDS, which bounds m and, for a single
 // large matrix, leaves all but one CU idle).  Per column k of a panel:
 //   k_big_col      x = column k with the pending terms applied (rows > k),
-//                  d_k, and per-workgroup parts of sigma = |x(k+2:)|^2;
+//                  d_k, and per-workgroup parts of sigma = |x(k+2:)|^2
+//                  (and of its rescaled form, see reflector.hpp);
 //   k_big_reflect  the reflector from the summed parts (every workgroup
 //                  forms the same scalars), v stored in A and the panel
 //                  buffer, and per-workgroup parts of W^T v and V^T v;
@@ -464,17 +471,20 @@ __global__ __launch_bounds__(kBR) void k_big_col(const T *__restrict__ a, int m,
     }
     __syncthreads();
     const int i = k + 1 + blockIdx.x * kBR + threadIdx.x;
-    double part = 0.0;
+    double part = 0.0, up = 0.0;  // up: of the rescaled column
     if (i < m) {
         double x = a[(int64_t)k * ld + i];
         for (int t = 0; t < jj; ++t)
             x -= a[(int64_t)(k0 + t) * ld + i] * c1[t] + W[(int64_t)t * ld + i] * c2[t];
         vs[i] = x;
-        if (i > k + 1) part = x * x;
+        if (i > k + 1) part = x * x, up = (x * kRescale) * (x * kRescale);
         else scal[0] = x;  // alpha, read by every workgroup of the next kernel
     }
-    const double tot = block_reduce(part, red);
-    if (threadIdx.x == 0) psig[blockIdx.x] = tot;
+    const double tot = block_reduce(part, red), tot_up = sizeof(T) == 8 ? block_reduce(up, red) : 0.0;
+    if (threadIdx.x == 0) {
+        psig[blockIdx.x] = tot;
+        psig[gridDim.x + blockIdx.x] = tot_up;
+    }
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         double dkk = a[(int64_t)k * ld + k];
         for (int t = 0; t < jj; ++t) dkk -= 2.0 * c2[t] * c1[t];
@@ -491,30 +501,29 @@ __global__ __launch_bounds__(kBR) void k_big_reflect(T *__restrict__ a, int m, i
                                                      double *__restrict__ ee,
                                                      double *__restrict__ tt,
                                                      double *__restrict__ pq) {
-    __shared__ double sig, wred[kWaves][2 * kNB];
+    __shared__ double sig, upsh, wred[kWaves][2 * kNB];
     const int k = k0 + jj;
     const int lane = threadIdx.x % PTB_WAVE, wid = threadIdx.x / PTB_WAVE;
     if (threadIdx.x == 0) {
         double s = 0.0;
         for (int b = 0; b < nblk; ++b) s += psig[b];
+        upsh = 1.0;
+        // (float storage: no square of its columns is that small)
+        if (sizeof(T) == 8 && scal[0] * scal[0] + s < kSquareMin) {
+            s = 0.0;
+            for (int b = 0; b < nblk; ++b) s += psig[nblk + b];
+            upsh = kRescale;
+        }
         sig = s;
     }
     __syncthreads();
-    const double sigma = sig, alpha = scal[0];
-    double beta, tk, scale;
-    if (sigma == 0.0) {
-        beta = alpha;
-        tk = 0.0;
-        scale = 0.0;
-    } else {
-        beta = -copysign(sqrt(alpha * alpha + sigma), alpha);
-        tk = (beta - alpha) / beta;
-        scale = 1.0 / (alpha - beta);
-    }
+    const double up = upsh;
+    const Reflector h = reflector(scal[0] * up, sig);
+    const double beta = h.beta / up, tk = h.tau, scale = h.scale;
     const int i = k + 1 + blockIdx.x * kBR + threadIdx.x;
     double v = 0.0;
     if (i < m) {
-        v = (i == k + 1) ? 1.0 : vs[i] * scale;
+        v = (i == k + 1) ? 1.0 : vs[i] * up * scale;
         vs[i] = v;
         a[(int64_t)k * ld + i] = (T)v;
         W[(int64_t)(kNB + jj) * ld + i] = (T)v;
@@ -682,12 +691,12 @@ int sytrd_big(ptbgpu_ctx *ctx, const SubDesc &x, const SubDesc *dx, T *A, double
     double *dd = d + x.mapoff, *ee = e + x.mapoff, *tt = tau + x.mapoff;
     const int nbt = (m + kBT - 1) / kBT;         // 64-row blocks
     const int gmax = (m + kBR - 1) / kBR;        // row workgroups at most
-    const size_t nsc = (size_t)m + 2 * (size_t)nbt * m + (size_t)gmax * (2 + 2 * kNB) + 4;
+    const size_t nsc = (size_t)m + 2 * (size_t)nbt * m + (size_t)gmax * (3 + 2 * kNB) + 4;
     auto *sc = static_cast<double *>(ws(ctx, "sybig_scr", sizeof(double) * nsc));
     auto *W = static_cast<T *>(ws(ctx, f32 ? "sybig_pw32" : "sybig_pw", sizeof(T) * (size_t)ld * 3 * kNB));
     if (!sc || !W) return PTBGPU_E_NOMEM;
     double *vs = sc, *PR = vs + m, *PQ = PR + (size_t)nbt * m, *psig = PQ + (size_t)nbt * m;
-    double *ppv = psig + gmax, *pq = ppv + gmax, *scal = pq + (size_t)gmax * 2 * kNB;
+    double *ppv = psig + 2 * gmax, *pq = ppv + gmax, *scal = pq + (size_t)gmax * 2 * kNB;
     const int npanel = m > 2 ? (m - 2 + kNB - 1) / kNB : 0;
     std::vector<GemmDesc> g;
     for (int p = 0; p < npanel; ++p) {
