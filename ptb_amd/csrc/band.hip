@@ -155,6 +155,7 @@ __device__ __forceinline__ Reflector reflector_fast(double alpha, double sigma) 
     r = fma(r, fma(-q, r, 1.0), r);
     return {-copysign(g, alpha), fma(2.0 * h, fabs(alpha), 1.0), copysign(r, alpha)};
 }
+
 // ---- stage 1 ------------------------------------------------------------------
 
 // QR of one 16-column panel, rows r0 .. m - 1 in registers (thread t holds rows
@@ -1450,12 +1451,18 @@ int sytrd_band(ptbgpu_ctx *ctx, const std::vector<SubDesc> &desc, double *A, dou
             {
                 ProfScope kprof_(ctx, "band_step");
                 const int nunit = band_units(ns);
-                const dim3 grid((unsigned)((na + 7) / 8 * 8 * nunit));
-                if (p == 0)
-                    hipLaunchKernelGGL(k_band_step<false>, grid, dim3(256), 0, st, ds, na, A, PW, PX, p, nunit);
-                else
-                    hipLaunchKernelGGL(k_band_step<true>, grid, dim3(256), 0, st, ds, na, A, PW, PX, p, nunit);
-                PTB_CHECK_LAUNCH(ctx);
+                // (a grid holds fewer than 2^32 threads: 116 504 submatrices, if one of
+                // them has 2048 rows)
+                const int most = (int)(((int64_t)1 << 32) / 256 - 1) / nunit / 8 * 8;
+                for (int f = 0; f < na; f += most) {
+                    const int nf = std::min(na - f, most);
+                    const dim3 grid((unsigned)((nf + 7) / 8 * 8 * nunit));
+                    if (p == 0)
+                        hipLaunchKernelGGL(k_band_step<false>, grid, dim3(256), 0, st, ds + f, nf, A, PW, PX, p, nunit);
+                    else
+                        hipLaunchKernelGGL(k_band_step<true>, grid, dim3(256), 0, st, ds + f, nf, A, PW, PX, p, nunit);
+                    PTB_CHECK_LAUNCH(ctx);
+                }
             }
             {
                 ProfScope kprof_(ctx, "band_x");
