@@ -56,15 +56,16 @@ void ws_trim(ptbgpu_ctx *ctx, const char *name, size_t bytes) {
 
 // Tables go into one half of the ring after the other; a half is used again when
 // the copies out of it are done.  It starts small and grows (to kRingHalfMax) while
-// tables do not fit or the host would wait for it; larger tables are copied as
-// they are.
+// tables do not fit or the host would wait for it; larger tables, and all while
+// there is no pinned memory for a ring, are copied as they are.
 int upload_async(ptbgpu_ctx *ctx, void *dst, const void *src, size_t bytes) {
     constexpr size_t kRingHalfMin = (size_t)1 << 20, kRingHalfMax = (size_t)32 << 20;
     const size_t need = (bytes + 255) & ~(size_t)255;
-    if (need > kRingHalfMax) {
+    auto as_it_is = [&]() -> int {
         PTB_HIP(ctx, hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, ctx->stream));
         return PTBGPU_OK;
-    }
+    };
+    if (need > kRingHalfMax) return as_it_is();
     for (auto &e : ctx->ring_ev)
         if (!e) PTB_HIP(ctx, hipEventCreateWithFlags(&e, hipEventDisableTiming));
     size_t half = std::max(ctx->ring_half, kRingHalfMin);
@@ -87,7 +88,10 @@ int upload_async(ptbgpu_ctx *ctx, void *dst, const void *src, size_t bytes) {
     if (half != ctx->ring_half) {
         ctx->ring_half = 0;
         // (hws waits for the stream before it gives the old ring back)
-        if (!hws(ctx, "table_ring", 2 * half)) return PTBGPU_E_NOMEM;
+        if (!hws(ctx, "table_ring", 2 * half)) {
+            ctx->last_error.clear();
+            return as_it_is();
+        }
         ctx->ring_half = half;
         ctx->ring_pos = 0;
         ctx->ring_cur = 0;
