@@ -1415,6 +1415,11 @@ int sytrd_band(ptbgpu_ctx *ctx, const std::vector<SubDesc> &desc, double *A, dou
     auto *rtau = static_cast<double *>(ws(ctx, "band_q2tau", sizeof(double) * 16 * std::max<int64_t>(blk, 1)));
     auto *fac = static_cast<double *>(ws(ctx, "band_q2fac", sizeof(double) * 1024 * std::max<int64_t>(blk, 1)));
     if (!PW || !PX || !AB || !raw || !rtau || !fac) return PTBGPU_E_NOMEM;
+    if (ctx->poison_arenas && !ctx->capturing) {  // all bytes 0xff: NaN
+        const std::pair<void *, int64_t> bufs[] = {{PW, pw}, {PX, px}, {AB, ab}, {raw, 256 * blk}, {rtau, 16 * blk},
+                                                   {fac, 1024 * blk}};
+        for (const auto &[p, n] : bufs) PTB_HIP(ctx, hipMemsetAsync(p, 0xff, sizeof(double) * n, ctx->stream));
+    }
     auto *ds = static_cast<BandSub *>(upload_table(ctx, "band_subs", subs.data(), sizeof(BandSub) * nb));
     if (!ds) return PTBGPU_E_NOMEM;
     qf.q2fac = fac;

@@ -86,3 +86,31 @@ def test_poisoned_batch_and_chip_wide_merges(engine, poisoned):
         for a, b in zip(results[0], r):
             assert np.isfinite(b).all()
             assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("kind,size,seed,cols", CASES + [("water", (3, 3, 3), 2, 1), ("alkane", 9, 0, 1)])
+def test_poisoned_band_buffers_change_nothing(engine, poisoned, precision, kind, size, seed, cols):
+    """The two-stage reduction's buffers (panels, parts of X, band, chase reflectors and
+    their factors) hold NaN too.  A mixed build at the default threshold reduces its
+    small submatrices through them."""
+    mol, H, S = small_system(kind, size, seed, filt=1e-4 if kind == "water" else 1e-5)
+    out = []
+    for eng in (engine, poisoned):
+        P = np.zeros_like(H)
+        rep = eng.sm_stupid_simple(mol.ndim, mol.nel, H, S, P, mol.n, mol.xyz, mol.aoat, cols, 2, precision=precision)
+        out.append((P, rep["mu"]))
+    assert np.isfinite(out[1][0]).all()
+    assert out[0][1] == out[1][1]
+    assert np.array_equal(out[0][0], out[1][0])
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 16, 17, 18, 19, 33, 34, 83, 131, 273, 530, 1025, 1041, 1100])
+def test_poisoned_dense_solve(engine, poisoned, n):
+    """One matrix of every size class, edges not multiples of 16 or 64."""
+    rng = np.random.default_rng(n)
+    B = rng.normal(size=(n, n))
+    A = B @ B.T / n + np.eye(n)
+    R = poisoned.matrix_root(A)
+    assert np.isfinite(R).all()
+    assert np.array_equal(R, engine.matrix_root(A))
