@@ -174,9 +174,12 @@ __global__ void k_bisect_step(BisState *__restrict__ st, const double *__restric
 }
 
 // The whole bisection of molecules of at most kBisRows states, a workgroup each:
-// the states stay in its registers, and a pass costs a reduction instead of two
-// launches (8 waters: 48 launches of 2.5 us and the host's wait for them).  The
-// sums are those of k_nel_partial with one chunk.
+// the states stay in its registers (16 per thread), and a pass costs a reduction
+// instead of two launches of 2.5 us.  Builds with it and without: 4 waters (1082
+// states) 1.40 -> 1.21 ms, 7 waters (3222) 2.14 -> 1.91, one 1472-row block 24.90 ->
+// 24.71.  8 waters have about 4200 states, so they and any batch with a molecule of
+// more than kBisRows take the general kernels.  The sums are those of k_nel_partial
+// with one chunk.
 constexpr int kBisRows = 4096;
 __global__ __launch_bounds__(kT) void k_bisect_whole(const double *__restrict__ e,
                                                      const double *__restrict__ fe,
