@@ -487,8 +487,9 @@ __global__ __launch_bounds__(NT) void k_dc_merge(const SubDesc *__restrict__ des
     bitonic_sort<NT>(Dk, ix, npow);
     for (int j = threadIdx.x; j < n; j += NT) z[j] = zraw[ix[j]];
     __syncthreads();
+    // (the node's scale: D + rho z z^T, z of unit norm)
     double mx = 0.0;
-    for (int j = threadIdx.x; j < n; j += NT) mx = fmax(mx, fmax(fabs(Dk[j]), fabs(z[j])));
+    for (int j = threadIdx.x; j < n; j += NT) mx = fmax(mx, fmax(fabs(Dk[j]), rho * fabs(z[j])));
     const double tol = 8.0 * kEps * block_max<NT>(mx, red);
 
     // Deflation.  Type 1: rho |z_j| <= tol.  Type 2: neighbouring surviving

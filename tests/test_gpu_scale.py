@@ -51,3 +51,17 @@ def test_weakly_coupled_blocks_of_every_route(engine, n):
     and the one-stage reduction above 2048 rows."""
     for x in (156, 159, 161):
         _check(engine, _two_blocks(n, 10.0 ** -x, "diagonal"))
+
+
+@pytest.mark.parametrize("shift", [-400, -100, -40, -12, 12, 400])
+@pytest.mark.parametrize("n", [2, 12, 17, 60, 300, 1100, 2100])
+def test_scaled_matrices(engine, n, shift):
+    """A power of two in front of a matrix comes out as its root, exactly but for the
+    rounding of a reduction: no test in the solver compares with 1."""
+    rng = np.random.default_rng(3 * n)
+    B = rng.normal(size=(n, n))
+    A = B @ B.T / n + np.eye(n)
+    w = np.linalg.eigvalsh(A)
+    tol = 10 * max(n, 8) * np.finfo(float).eps * w[-1] / w[0]
+    R = np.ldexp(engine.matrix_root(np.ldexp(A, shift)), shift // 2)
+    assert np.abs(R @ A @ R - np.eye(n)).max() < tol
