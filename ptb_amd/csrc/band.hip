@@ -63,10 +63,7 @@ __device__ inline int64_t q2_block(int ng, int G, int k) {
 // ---- cross-lane sums --------------------------------------------------------
 template <int CTRL>
 __device__ __forceinline__ double dpp_add(double v) {
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, true);
-    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
-    return v + __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+    return v + dpp_mov<CTRL>(v);
 }
 // sum over the 16 lanes of a row, in every lane: quad_perm 1032, 2301, then
 // the mirrors within 8 and within 16
@@ -75,13 +72,6 @@ __device__ __forceinline__ double row_sum(double v) {
     v = dpp_add<0x4E>(v);
     v = dpp_add<0x141>(v);
     return dpp_add<0x140>(v);
-}
-template <int CTRL>
-__device__ __forceinline__ double dpp_mov(double v) {
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, true);
-    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
-    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
 // sums over the 16 lanes of a row of four values, times a, in every lane: two
 // halving exchanges (quad_perm 1032, 2301) leave one value per lane, summed over
@@ -112,12 +102,6 @@ __device__ __forceinline__ double rows_sum(double v) {
     const auto h = __builtin_amdgcn_permlane32_swap((unsigned)(b >> 32), (unsigned)(b >> 32), false, false);
     return __longlong_as_double(((long long)h[0] << 32) | l[0]) +
            __longlong_as_double(((long long)h[1] << 32) | l[1]);
-}
-__device__ __forceinline__ double read_lane(double v, int lane) {
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_readlane((int)b, lane);
-    const int hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
-    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
 // Sum over the wavefront of 16 values per lane; value q ends in the lanes with
 // (lane >> 2) & 15 == q.

@@ -180,6 +180,24 @@ __device__ __forceinline__ T wave_max(T v) {
     return v;
 }
 
+// ---- wavefront exchanges of doubles ----------------------------------------
+// v of the lane that the DPP control CTRL names
+template <int CTRL>
+__device__ __forceinline__ double dpp_mov(double v) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
+// a wavefront lane's v, in scalar registers
+__device__ __forceinline__ double read_lane(double v, int lane) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_readlane((int)b, lane);
+    const int hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
 // Block-wide sum; every thread gets the result. `scratch` holds >= 16 T.
 template <typename T>
 __device__ __forceinline__ T block_sum(T v, T *scratch) {

@@ -182,13 +182,6 @@ __device__ __forceinline__ double rcp64(double x) {
 // merges of the 512-water box took 1-4 % less with eight than with one (in
 // workgroups too few to be latency-bound), the roots of 8 waters 0.38 -> 0.10 ms.
 constexpr int kRootLanes = 8;
-template <int CTRL>
-__device__ __forceinline__ double dpp_mov(double v) {
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, true);
-    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
-    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
-}
 // op over the eight lanes of a group, the same value in each (quad_perm 1032 and
 // 2301, then the mirror within 8)
 template <typename F>
@@ -819,8 +812,8 @@ __global__ __launch_bounds__(kMT) void k_dc_roots_columns(const SubDesc *__restr
                 Za + ds.off + (int64_t)(nd.lo + c) * ld + nd.lo, half ? cb : 0, half ? ce : n, lane, cb, ce);
 }
 
-// Loewner entries (the first nroot blocks) and, after kDcSpread, 64 rows a block: the deflation rotations in order, then the deflated columns to their
-// final place.
+// Loewner entries (the first nroot blocks) and, after kDcSpread, 64 rows a block: the
+// deflation rotations in order, then the deflated columns to their final place.
 __global__ __launch_bounds__(kMT) void k_dc_loewner_deflated(const SubDesc *__restrict__ desc,
                                                              const DcNode *__restrict__ nodes, int npow,
                                                              const double *__restrict__ e_all,

@@ -51,14 +51,6 @@ using gmem = __attribute__((address_space(1))) T;
 // per SIMD cost 20 % more.
 constexpr int kKS = 32;  // k depth up to which a product counts as one slice (k_gemm_nt1)
 
-// a wavefront lane's value, in scalar registers
-__device__ __forceinline__ double lane_value(double v, int lane) {
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_readlane((int)b, lane);
-    const int hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
-    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
-}
-
 template <int TE>
 struct GemmTileShape {
     static constexpr int KS = TE == 32 ? 64 : 16;  // k slice
@@ -486,7 +478,7 @@ __global__ __launch_bounds__(kT) void k_potrf_panel(const SubDesc *__restrict__ 
         bool bad = false;
 #pragma unroll
         for (int j = 0; j < 32; ++j) {
-            double q = lane_value(x[j], j);
+            double q = read_lane(x[j], j);
             if (!(q > 0.0)) {
                 bad = true;
                 q = 1.0;
@@ -494,7 +486,7 @@ __global__ __launch_bounds__(kT) void k_potrf_panel(const SubDesc *__restrict__ 
             const double sq = sqrt(q), l = r == j ? sq : x[j] / sq;
             x[j] = l;
 #pragma unroll
-            for (int c = j + 1; c < 32; ++c) x[c] -= l * lane_value(l, c);
+            for (int c = j + 1; c < 32; ++c) x[c] -= l * read_lane(l, c);
         }
         if (mode != 1) {
             if (threadIdx.x < 32)
@@ -510,8 +502,8 @@ __global__ __launch_bounds__(kT) void k_potrf_panel(const SubDesc *__restrict__ 
         for (int c = 0; c < 32; ++c) {
             double t = r == c ? 1.0 : 0.0;
 #pragma unroll
-            for (int q = 0; q < c; ++q) t -= lane_value(x[q], c) * y[q];
-            y[c] = t / lane_value(x[c], c);
+            for (int q = 0; q < c; ++q) t -= read_lane(x[q], c) * y[q];
+            y[c] = t / read_lane(x[c], c);
             if (threadIdx.x < 32) Li[c][r] = y[c];
         }
         if (i < m) load(i);
@@ -1078,8 +1070,9 @@ static int launch_gemm(ptbgpu_ctx *ctx, bool ta, bool tb, bool f32, dim3 grid, c
 }
 
 constexpr int64_t kSmallTiles = 2;
-// Tile edge of an FP64 launch of `count` products from its tile counts and the multiply-adds its tiles issue at both edges (padded output
-// times the k range of each tile): the gemm_tile knob forces 64 or 128; else
+// Tile edge of an FP64 launch of `count` products from its tile counts and the
+// multiply-adds its tiles issue at both edges (padded output times the k range of
+// each tile): the gemm_tile knob forces 64 or 128; else
 // 128 x 128 tiles only for launches of fewer products than XCDs (single large
 // products, spread over the chip) with at least 4 such tiles per CU and at
 // most 3 % more work than 64 x 64 tiles.  On MI355X they reach 58 TFLOP/s on
