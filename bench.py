@@ -24,6 +24,8 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0
+BAND_WIDTH = 16      # subdiagonals of the two-stage FP64 reduction
+BAND_MAX_M = 2048    # the largest matrix it takes
 FP64_PEAK_TFS = 78.6
 METRIC = "density builds/s: mixed-prec batched vs FP64 GPU, |ΔE_band|≤1e-6 Eh, 512 H2O"
 WORKLOADS = {
@@ -38,9 +40,10 @@ WORKLOADS = {
 PHASES = ["potrf", "trsm", "trsm_h", "trsm_k", "trsm_e", "trsm_u", "sytrd", "apply_q",
           "apply_q_x", "apply_q_o", "apply_q_r1", "apply_q_r2", "gemm_sytrd", "gemm_potrf",
           "gemm_trsm", "gemm_dc", "gemm_q", "gemm_fe", "gemm_refine", "gemm_other", "refine_all",
-          "inv_lower", "gemm_linv", "gemm_kform", "gemm_u"]
+          "inv_lower", "gemm_linv", "gemm_kform", "gemm_u", "band_reduce"]
 KERNELS = ["pattern", "group_union", "group_map", "gather", "potrf_panel", "diag_inv",
-           "transpose", "sytrd_panel", "sytrd_panel_f32", "zero_upper", "dc_leaf", "dc_merge", "gemm", "larft",
+           "transpose", "sytrd_panel", "sytrd_panel_f32", "zero_upper", "band_qr", "band_step", "band_x", "band_w",
+           "band_chase", "q2_prep", "apply_q2", "dc_leaf", "dc_merge", "gemm", "larft",
            "fe_rows", "fe_finish", "bisect", "occ_compact", "dmat_scatter", "to_f32", "promote",
            "refine"]
 
@@ -61,19 +64,37 @@ def sytrd_bytes(ms, elem=8):
     return tot
 
 
+def band_bytes(ms):
+    """Algorithmic HBM bytes of k_band_step in one build (all panels): the trailing
+    triangle below each 16-column panel read once, and written once with the panel
+    before's update (none before the first)."""
+    tot = 0.0
+    for m in ms:
+        n = np.arange(m - BAND_WIDTH, 1, -BAND_WIDTH, dtype=np.float64)
+        tri = 8.0 * n * (n + 1) / 2.0
+        tot += float(2.0 * np.sum(tri) - (tri[0] if len(tri) else 0.0))
+    return tot
+
+
 def roofline_model(name, ms, ndim, mixed=False, thr=0):
     """(bound, algorithmic units of one build summed over the kernel's launches,
     unit); divided by the kernel's bracketed time of one build this is the
-    per-launch figure averaged over its launches.  A mixed build reduces the
-    submatrices below `thr` (mixed_min_m) with the FP64 panel kernel
-    (`sytrd_panel`) and the others with the float one (`sytrd_panel_f32`)."""
+    per-launch figure averaged over its launches.  FP64 submatrices of up to
+    BAND_MAX_M rows are reduced through a band (`band_step`), larger ones of a
+    batch by the FP64 panel kernel (`sytrd_panel`); a mixed build reduces the
+    submatrices below `thr` (mixed_min_m) in FP64 and the others with the float
+    panel kernel (`sytrd_panel_f32`)."""
     m = np.asarray(ms, dtype=np.float64)
     npk = ndim * (ndim + 1) / 2.0
     if name == "sytrd_panel_f32":
         return "hbm", sytrd_bytes([x for x in ms if x >= thr], 4), "GB/s"
+    fp64 = [x for x in ms if not mixed or x < thr]
     if name == "sytrd_panel":
-        sel = [x for x in ms if not mixed or x < thr]
+        sel = [x for x in fp64 if x > BAND_MAX_M]
         return ("hbm", sytrd_bytes(sel, 8), "GB/s") if sel else None
+    if name == "band_step":
+        sel = [x for x in fp64 if x <= BAND_MAX_M]
+        return ("hbm", band_bytes(sel), "GB/s") if sel else None
     if name == "gather":   # dense Hsm and Ssm written + packed reads counted once
         return "hbm", float(np.sum(16.0 * m * m)) + 16.0 * npk, "GB/s"
     if name == "pattern":
@@ -149,8 +170,9 @@ def gemm_site_flops(site, ms, cs, nos, mixed, thr=0, lowp_max=0):
         return float(np.sum(m ** 3) / 3.0), 0.0
     if site == "gemm_kform":
         return float(np.sum(m ** 3)), 0.0
-    if site == "gemm_sytrd":
-        return float(np.sum(2.0 * m ** 3 / 3.0)), 0.0
+    if site == "gemm_sytrd":  # the one-stage reduction's updates (the band route has none)
+        one_stage = (m > BAND_MAX_M) | ((m >= thr) if mixed else False)
+        return float(np.sum(2.0 * m[one_stage] ** 3 / 3.0)), 0.0
     if site == "gemm_dc":
         f = 2.0 * m ** 3 / 3.0
         return float(np.sum(f[~lowp])), float(np.sum(f[lowp]))
@@ -468,7 +490,7 @@ def main():
         for site, (ms, cnt) in sorted(r["kernels"].items(), key=lambda kv: -kv[1][0]):
             fl = gemm_site_flops(site, r["m"], cs, nos, main_prec == "mixed", thr,
                                  eng.get_tuning("lowp_merge_max_m"))
-            if fl is None or ms <= 0:
+            if fl is None or ms <= 0 or sum(fl) == 0:
                 continue
             fp, bf = fl
             tf = (fp + bf) / (ms * 1e-3) / 1e12
@@ -485,7 +507,7 @@ def main():
                           "algorithmic_tflop": round((fp + bf) / 1e12, 4), "ms": round(ms, 3),
                           "achieved": round(tf, 2), "peak": round(peak, 1),
                           "unit": "TFLOP/s", "frac": round(tf / peak, 4)})
-        for name in ("sytrd_panel_f32", "sytrd_panel", "gather", "pattern"):
+        for name in ("sytrd_panel_f32", "sytrd_panel", "band_step", "gather", "pattern"):
             if name in r["kernels"]:
                 ms, cnt = r["kernels"][name]
                 model = roofline_model(name, r["m"], n, mixed=main_prec == "mixed", thr=thr)

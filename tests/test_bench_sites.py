@@ -64,3 +64,29 @@ def test_q_application_adds_the_refinement_passes():
     extra = float(np.sum(8.0 * M[ref].astype(float) ** 2 * NO[ref]))
     fp, bf = bench.gemm_site_flops("gemm_q", M, C, NO, True, THR, 0)
     assert fp == pytest.approx(base + extra) and bf == 0.0
+
+
+def test_band_step_bytes():
+    """k_band_step per 16-column panel: the trailing lower triangle read, and written
+    with the panel before's update."""
+    for m in (1, 17, 18, 34, 100, 999):
+        want, p = 0, 0
+        while m - 16 * (p + 1) >= 2:
+            n = m - 16 * (p + 1)
+            want += 8 * n * (n + 1) // 2 * (1 if p == 0 else 2)
+            p += 1
+        assert bench.band_bytes([m]) == want
+    assert bench.band_bytes([100, 999]) == bench.band_bytes([100]) + bench.band_bytes([999])
+
+
+def test_fp64_reductions_by_size():
+    # an FP64 build: the band route up to 2048 rows, the panel kernel above
+    assert bench.roofline_model("sytrd_panel", [500, 2048], 5000) is None
+    assert bench.roofline_model("sytrd_panel", [500, 2100, 2200], 5000)[1] == bench.sytrd_bytes([2100, 2200])
+    assert bench.roofline_model("band_step", [500, 2048, 2100], 5000)[1] == bench.band_bytes([500, 2048])
+    # a mixed build: only the submatrices below the threshold
+    assert bench.roofline_model("band_step", [200, 500], 5000, mixed=True, thr=288)[1] == bench.band_bytes([200])
+    assert bench.roofline_model("sytrd_panel_f32", [200, 500], 5000, mixed=True, thr=288)[1] == bench.sytrd_bytes([500], 4)
+    # and the one-stage updates' products likewise
+    assert bench.gemm_site_flops("gemm_sytrd", [500, 2100], C[:2], NO[:2], False, 288) == (2.0 * 2100 ** 3 / 3.0, 0.0)
+    assert bench.gemm_site_flops("gemm_sytrd", [200, 600], C[:2], NO[:2], True, 288) == (2.0 * 600 ** 3 / 3.0, 0.0)
