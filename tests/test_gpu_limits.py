@@ -1,4 +1,4 @@
-"""Batches at the limits of a launch."""
+"""Limits of a launch's threads and of a product's offsets."""
 import numpy as np
 import pytest
 
@@ -52,3 +52,36 @@ def test_more_submatrices_than_one_launch_of_the_largest(engine):
     for it in items[:-1]:
         assert torch.equal(it[4], alone[0][4])
     assert torch.equal(items[-1][4], alone[1][4])
+
+
+@pytest.mark.parametrize("edge", [0, 64, 128])
+@pytest.mark.parametrize("ld", [(1 << 22) - 1, 1 << 22, (1 << 22) + 5])
+@pytest.mark.parametrize("order", ["nn", "tn", "nt", "tt"])
+def test_products_with_long_strides(engine, order, ld, edge):
+    """Leading dimensions on both sides of 2^22, up to which a product forms its byte
+    offsets once.  Error per element at most k eps |A| |B|."""
+    import torch
+    m, n, k = 130, 131, 70
+    ta, tb = order[0] == "t", order[1] == "t"
+    g = torch.Generator(device="cuda").manual_seed(ld)
+
+    def stored(rows, cols):  # column-major, columns `ld` apart
+        x = torch.empty((cols - 1) * ld + rows, device="cuda", dtype=torch.float64).as_strided((cols, rows), (ld, 1))
+        return x.copy_(torch.randn((cols, rows), generator=g, device="cuda", dtype=torch.float64))
+
+    A, B = stored(k, m) if ta else stored(m, k), stored(n, k) if tb else stored(k, n)
+    C = torch.empty((n, m), device="cuda", dtype=torch.float64)
+    torch.cuda.synchronize()
+    one = [np.array([v], dtype=np.int64) for v in (m, n, k, ld, ld, m)]
+    ptr = [np.array([t.data_ptr()], dtype=np.uint64) for t in (A, B, C)]
+    at = lambda x: x.ctypes.data
+    saved = engine.get_tuning("gemm_tile")
+    engine.set_tuning("gemm_tile", edge)
+    try:
+        engine._check(engine.lib.ptbgpu_gemm_batch_dev(
+            engine.ctx, 0, int(ta), int(tb), 1, at(one[0]), at(one[1]), at(one[2]), at(ptr[0]), at(one[3]),
+            at(ptr[1]), at(one[4]), at(ptr[2]), at(one[5]), 1.0, 0.0))
+    finally:
+        engine.set_tuning("gemm_tile", saved)
+    a, b = (A if ta else A.t()).contiguous(), (B if tb else B.t()).contiguous()
+    assert ((C.t() - a @ b).abs() <= k * np.finfo(float).eps * (a.abs() @ b.abs())).all()
